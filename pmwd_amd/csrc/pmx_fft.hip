@@ -13,24 +13,22 @@
 // inverse ends with y (strided) and z c2r (rows).
 #include "pmx_internal.h"
 
-#define FFT_TPB 512                  // threads per FFT workgroup
-#define FFT_CAP 8192                 // complex values per workgroup
-#define FFT_MAXV (FFT_CAP / FFT_TPB) // values per thread
-#define RFFT_CAP 4096                // row passes: fewer values per thread
-#define RFFT_MAXV (RFFT_CAP / FFT_TPB)
-// Poisson x pass: 8 columns of 512 per 512-thread workgroup, three such
-// workgroups (40 KB of LDS each) per CU; 16 columns per 1024 or per 512
-// threads and 8 per 256 measured slower, two waves per SIMD no faster
-#ifndef PFFT_TPB
-#define PFFT_TPB 512
-#endif
-#ifndef PFFT_CAP
-#define PFFT_CAP 4096
-#endif
-#ifndef PFFT_WPE                     // waves per SIMD the register budget allows
-#define PFFT_WPE 1
-#endif
-#define PFFT_MAXV (PFFT_CAP / PFFT_TPB)
+#define FFT_CAP 8192                 // complex values per strided workgroup, fixed lengths
+#define PFFT_CAP 4096                // Poisson x pass (8 columns of 512, three 40 KB workgroups
+                                     // per CU; 16 columns measured slower)
+#define RFFT_CAP 4096                // row passes
+// Kernels for lengths known only at run time: up to 512 threads of eight
+// values (gen_tpb); their TPB argument is 0, the launch's own block size.
+// With 16 values a thread the stages' addresses and twiddles spilled.
+#define GEN_CAP 4096
+#define GEN_MAXV 8
+#define GEN_TPB 0
+#define GEN_MAXTPB (GEN_CAP / GEN_MAXV)
+
+template <int TPB>
+__device__ __forceinline__ int tpb() {
+  return TPB ? TPB : (int)blockDim.x;
+}
 
 // Complex products inside the transforms may fuse into FMAs (the file is
 // otherwise built with separate roundings).
@@ -103,12 +101,126 @@ __device__ __forceinline__ void dft8(float2* v) {
   v[7] = csub(e[3], o3);
 }
 
+// Odd radices: with a_q = v_q + v_{R-q}, b_q = v_q - v_{R-q} for q = 1..(R-1)/2,
+// X_r and X_{R-r} = v_0 + sum_q cos(2 pi q r / R) a_q -+ i sum_q sin(2 pi q r / R) b_q
+// (exp(-2 pi i q r / R) forward).
+template <int R>
+struct OddTab;
+template <>
+struct OddTab<3> {
+  static constexpr float c[1] = {-0.4999999999999998f};
+  static constexpr float s[1] = {0.8660254037844387f};
+};
+template <>
+struct OddTab<5> {
+  static constexpr float c[2] = {0.30901699437494745f, -0.8090169943749473f};
+  static constexpr float s[2] = {0.9510565162951535f, 0.5877852522924732f};
+};
+template <>
+struct OddTab<7> {
+  static constexpr float c[3] = {0.6234898018587336f, -0.22252093395631434f, -0.900968867902419f};
+  static constexpr float s[3] = {0.7818314824680298f, 0.9749279121818236f, 0.43388373911755823f};
+};
+
+template <int R, int DIR>
+__device__ __forceinline__ void dft_odd(float2* v) {
+#pragma clang fp contract(fast)
+  constexpr int K = (R - 1) / 2;
+  float2 a[K], b[K];
+  const float2 x0 = v[0];
+  float2 sum = x0;
+#pragma unroll
+  for (int q = 1; q <= K; ++q) {
+    a[q - 1] = cadd(v[q], v[R - q]);
+    b[q - 1] = csub(v[q], v[R - q]);
+    sum = cadd(sum, a[q - 1]);
+  }
+  v[0] = sum;
+#pragma unroll
+  for (int r = 1; r <= K; ++r) {
+    float2 m = x0, d = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int q = 1; q <= K; ++q) {
+      const int t = (q * r) % R;
+      const float c = t <= K ? OddTab<R>::c[t - 1] : OddTab<R>::c[R - t - 1];
+      const float e = t <= K ? OddTab<R>::s[t - 1] : -OddTab<R>::s[R - t - 1];
+      m.x += c * a[q - 1].x;
+      m.y += c * a[q - 1].y;
+      d.x += e * b[q - 1].x;
+      d.y += e * b[q - 1].y;
+    }
+    d = mul_mi<DIR>(d);
+    v[r] = cadd(m, d);
+    v[R - r] = csub(m, d);
+  }
+}
+
+// Radix 2 N with N odd (Good-Thomas): input N n1 + 2 n2 mod 2N, output
+// N k1 + (N + 1) k2 mod 2N, no twiddles.
+template <int N, int DIR>
+__device__ __forceinline__ void dft_2odd(float2* v) {
+  float2 e[N], o[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    e[i] = cadd(v[(2 * i) % (2 * N)], v[(N + 2 * i) % (2 * N)]);
+    o[i] = csub(v[(2 * i) % (2 * N)], v[(N + 2 * i) % (2 * N)]);
+  }
+  dft_odd<N, DIR>(e);
+  dft_odd<N, DIR>(o);
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    v[((N + 1) * k) % (2 * N)] = e[k];
+    v[(N + (N + 1) * k) % (2 * N)] = o[k];
+  }
+}
+
+// Radix 9 as 3 x 3.
+template <int DIR>
+__device__ __forceinline__ void dft9(float2* v) {
+  // exp(-2 pi i m / 9), m = 1, 2, 4
+  const float2 w1 = make_float2(0.76604444311897803520f, -0.64278760968653932632f);
+  const float2 w2 = make_float2(0.17364817766693034885f, -0.98480775301220805937f);
+  const float2 w4 = make_float2(-0.93969262078590838405f, -0.34202014332566873304f);
+  float2 u[3][3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) u[i][j] = v[i + 3 * j];
+    dft_odd<3, DIR>(u[i]);
+  }
+  u[1][1] = cmul_dir<DIR>(u[1][1], w1);
+  u[1][2] = cmul_dir<DIR>(u[1][2], w2);
+  u[2][1] = cmul_dir<DIR>(u[2][1], w2);
+  u[2][2] = cmul_dir<DIR>(u[2][2], w4);
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    float2 t[3] = {u[0][j], u[1][j], u[2][j]};
+    dft_odd<3, DIR>(t);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[j + 3 * k] = t[k];
+  }
+}
+
 template <int R, int DIR>
 __device__ __forceinline__ void dftR(float2* v) {
-  if (R == 2) dft2<DIR>(v);
-  else if (R == 4) dft4<DIR>(v);
-  else dft8<DIR>(v);
+  if constexpr (R == 2) dft2<DIR>(v);
+  else if constexpr (R == 4) dft4<DIR>(v);
+  else if constexpr (R == 8) dft8<DIR>(v);
+  else if constexpr (R == 9) dft9<DIR>(v);
+  else if constexpr (R % 2 == 0) dft_2odd<R / 2, DIR>(v);
+  else dft_odd<R, DIR>(v);
 }
+
+// i / d by a multiply, exact while i * d < 2^32 (the callers' i and d are
+// below 2^16)
+struct FastDiv {
+  unsigned d, m;
+  __device__ __forceinline__ explicit FastDiv(int d_)
+      : d((unsigned)d_), m(d_ > 1 ? 0xffffffffu / (unsigned)d_ + 1u : 0u) {}
+  __device__ __forceinline__ int operator()(int i) const {
+    return d > 1 ? (int)__umulhi((unsigned)i, m) : i;
+  }
+};
 
 // LDS layouts of P pencils of length n:
 //   ROWS (pencil-major):  element (p, j) at p*(n + n/8) + j + j/8; the gap
@@ -130,19 +242,25 @@ __host__ __device__ constexpr int lds_elems(int lay, int n, int P) {
 
 __host__ __device__ constexpr int ilog2c(int n) { return n <= 1 ? 0 : 1 + ilog2c(n >> 1); }
 
-// pencils per workgroup for length n: a power of two with P*n <= cap
-__host__ __device__ constexpr int fft_pencils(int n, int cap = FFT_CAP) {
-  int P = 1;
-  while (P * 2 * n <= cap && P * 2 <= 256) P *= 2;
-  return P;
+// Columns per workgroup of a strided pass of fixed length 2^ln: 16 (128-byte
+// segments of a row), fewer when they exceed cap values; and its threads, of
+// v values each.  A 64^3 or 128^3 mesh has 33 or 65 columns, which blocks
+// filled to cap (128 and 64 columns) left half empty and too few.
+__host__ __device__ constexpr int ct_cols(int ln, int cap) {
+  return (cap >> ln) >= 16 ? 16 : (cap >> ln);
 }
+__host__ __device__ constexpr int ct_tpb(int ln, int cols, int v) { return (cols << ln) / v; }
+#define FFT_V 16   // y and plain x passes
+#define PFFT_V 8   // Poisson x pass
 
-// rows per workgroup for the row passes: P*n <= RFFT_CAP and the swizzled
-// ROWS block within FFT_CAP elements (64 KB)
-__host__ __device__ constexpr int row_pencils(int n) {
-  int P = 1;
-  while (P * 2 * n <= RFFT_CAP && lds_elems(ROWS, n, P * 2) <= FFT_CAP && P * 2 <= 256) P *= 2;
-  return P;
+// Rows per workgroup of a row pass of fixed length 2^lh: RFFT_CAP values, or
+// a quarter of that for meshes whose row blocks would leave CUs idle.  The
+// workgroup has eight values per thread.
+__host__ __device__ constexpr int ct_rows(int lh, bool small) {
+  return (small ? RFFT_CAP / 4 : RFFT_CAP) >> lh ? ((small ? RFFT_CAP / 4 : RFFT_CAP) >> lh) : 1;
+}
+__host__ __device__ constexpr int ct_row_tpb(int lh, bool small) {
+  return (ct_rows(lh, small) << lh) / 8;
 }
 
 // One Stockham stage of radix R (n a power of two, Ns the size of the
@@ -163,7 +281,7 @@ __device__ __forceinline__ void fft_stage(float2* s, int n, int P, int Ns, int l
   int mm[NG];
 #pragma unroll
   for (int it = 0; it < NG; ++it) {
-    int idx = threadIdx.x + it * TPB;
+    int idx = threadIdx.x + it * tpb<TPB>();
     mm[it] = 0;
     if (idx < total) {
       int p = LAY == ROWS ? (idx >> lnb) : (idx & (P - 1));
@@ -179,7 +297,7 @@ __device__ __forceinline__ void fft_stage(float2* s, int n, int P, int Ns, int l
   }
 #pragma unroll
   for (int it = 0; it < NG; ++it) {
-    int idx = threadIdx.x + it * TPB;
+    int idx = threadIdx.x + it * tpb<TPB>();
     if (idx < total) {
       if (mm[it] != 0) {
         float2* u = &v[it * R];
@@ -202,7 +320,7 @@ __device__ __forceinline__ void fft_stage(float2* s, int n, int P, int Ns, int l
   __syncthreads();
 #pragma unroll
   for (int it = 0; it < NG; ++it) {
-    int idx = threadIdx.x + it * TPB;
+    int idx = threadIdx.x + it * tpb<TPB>();
     if (idx < total) {
       int p = LAY == ROWS ? (idx >> lnb) : (idx & (P - 1));
       int j = LAY == ROWS ? (idx & (nb - 1)) : (idx >> lP);
@@ -215,57 +333,164 @@ __device__ __forceinline__ void fft_stage(float2* s, int n, int P, int Ns, int l
   __syncthreads();
 }
 
-// Direct DFT of P pencils of any length n (P*n <= FFT_CAP).
-template <int DIR, int LAY, int MAXV, int TPB>
-__device__ __forceinline__ void fft_direct(float2* s, int n, int P, const float2* __restrict__ tw,
-                                           int tws) {
-  float2 v[MAXV];
-  const int total = P * n;
+// One Stockham stage of radix R for a length n that is no power of two: as
+// fft_stage, with divisions by the run-time sub-transform sizes and every
+// twiddle power read from the table.
+template <int R, int DIR, int LAY, int MAXV, int TPB>
+__device__ __forceinline__ void fft_mix_stage(float2* s, int n, int P, int Ns, int lP,
+                                              const float2* __restrict__ tw, int tws) {
+  constexpr int NG = (MAXV + R - 1) / R;
+  const int nb = n / R;
+  const int total = P * nb;
+  const int step = nb / Ns * tws;
+  const FastDiv dnb(nb), dNs(Ns);
+  float2 v[NG * R];
+  int ob[NG], pp[NG];
 #pragma unroll
-  for (int it = 0; it < MAXV; ++it) {
-    int idx = threadIdx.x + it * TPB;
+  for (int it = 0; it < NG; ++it) {
+    const int idx = threadIdx.x + it * tpb<TPB>();
     if (idx < total) {
-      int p = LAY == ROWS ? idx / n : idx % P;
-      int k = LAY == ROWS ? idx % n : idx / P;
-      float2 acc = make_float2(0.f, 0.f);
-      int m = 0;
-      for (int j = 0; j < n; ++j) {
-        float2 w = twiddle<DIR>(tw, m * tws);
-        float2 x = s[lidx<LAY>(p, j, n, P)];
-        acc.x += x.x * w.x - x.y * w.y;
-        acc.y += x.x * w.y + x.y * w.x;
-        m += k;
-        if (m >= n) m -= n;
+      const int p = LAY == ROWS ? dnb(idx) : (idx & (P - 1));
+      const int j = LAY == ROWS ? idx - p * nb : (idx >> lP);
+      const int k = j - dNs(j) * Ns;
+      pp[it] = p;
+      ob[it] = (j - k) * R + k;
+      const int m = k * step;
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[it * R + r] = s[lidx<LAY>(p, j + r * nb, n, P)];
+      if (Ns > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[it * R + r] = cmul_dir<DIR>(v[it * R + r], tw[r * m]);
       }
-      v[it] = acc;
+      dftR<R, DIR>(&v[it * R]);
     }
   }
   __syncthreads();
 #pragma unroll
-  for (int it = 0; it < MAXV; ++it) {
-    int idx = threadIdx.x + it * TPB;
-    if (idx < total) {
-      int p = LAY == ROWS ? idx / n : idx % P;
-      int k = LAY == ROWS ? idx % n : idx / P;
-      s[lidx<LAY>(p, k, n, P)] = v[it];
+  for (int it = 0; it < NG; ++it) {
+    if ((int)threadIdx.x + it * tpb<TPB>() < total) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[lidx<LAY>(pp[it], ob[it] + r * Ns, n, P)] = v[it * R + r];
     }
   }
   __syncthreads();
 }
 
+// The stage of a prime radix R >= 11: the twiddles in place, then outputs r
+// and R - r of a butterfly together (dft_odd's sums), (R + 1) / 2 work items
+// each of (R - 1) / 2 terms.
+template <int DIR, int LAY, int MAXV, int TPB>
+__device__ __forceinline__ void fft_prime_stage(float2* s, int n, int P, int Ns, int R, int lP,
+                                                const float2* __restrict__ tw, int tws) {
+#pragma clang fp contract(fast)
+  constexpr int NG = (MAXV * 6 + 10) / 11;  // (R + 1) / (2 R) <= 6 / 11 items per value
+  const int nb = n / R, K = (R - 1) / 2;
+  const FastDiv dnb(nb), dn(n), dNs(Ns);
+  if (Ns > 1) {
+    const int step = nb / Ns * tws;
+    for (int idx = threadIdx.x; idx < P * n; idx += tpb<TPB>()) {
+      const int p = LAY == ROWS ? dn(idx) : (idx & (P - 1));
+      const int e = LAY == ROWS ? idx - p * n : (idx >> lP);
+      const int q = dnb(e), j = e - q * nb;
+      const int k = j - dNs(j) * Ns;
+      float2* x = s + lidx<LAY>(p, e, n, P);
+      *x = cmul_dir<DIR>(*x, tw[q * k * step]);
+    }
+    __syncthreads();
+  }
+  const int per = nb * (K + 1), total = P * per;
+  const FastDiv dper(per);
+  float2 u[NG], v[NG];
+#pragma unroll
+  for (int it = 0; it < NG; ++it) {
+    const int idx = threadIdx.x + it * tpb<TPB>();
+    if (idx < total) {
+      const int p = LAY == ROWS ? dper(idx) : (idx & (P - 1));
+      const int e = LAY == ROWS ? idx - p * per : (idx >> lP);
+      const int r = dnb(e), j = e - r * nb;
+      float2 m = s[lidx<LAY>(p, j, n, P)], d = make_float2(0.f, 0.f);
+      int t = 0;
+#pragma unroll 2
+      for (int q = 1; q <= K; ++q) {
+        t += r;
+        if (t >= R) t -= R;
+        const float2 w = tw[t * nb * tws];  // (cos, -sin)
+        const float2 a = s[lidx<LAY>(p, j + q * nb, n, P)];
+        const float2 b = s[lidx<LAY>(p, j + (R - q) * nb, n, P)];
+        m.x += w.x * (a.x + b.x);
+        m.y += w.x * (a.y + b.y);
+        d.x -= w.y * (a.x - b.x);
+        d.y -= w.y * (a.y - b.y);
+      }
+      d = mul_mi<DIR>(d);
+      u[it] = cadd(m, d);
+      v[it] = csub(m, d);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < NG; ++it) {
+    const int idx = threadIdx.x + it * tpb<TPB>();
+    if (idx < total) {
+      const int p = LAY == ROWS ? dper(idx) : (idx & (P - 1));
+      const int e = LAY == ROWS ? idx - p * per : (idx >> lP);
+      const int r = dnb(e), j = e - r * nb;
+      const int k = j - dNs(j) * Ns, o = (j - k) * R + k;
+      s[lidx<LAY>(p, o + r * Ns, n, P)] = u[it];
+      if (r) s[lidx<LAY>(p, o + (R - r) * Ns, n, P)] = v[it];
+    }
+  }
+  __syncthreads();
+}
+
+// Smallest prime factor of m that is at least 11 (m has no smaller one).
+__device__ __forceinline__ int prime_factor(int m) {
+  for (int q = 11; q * q <= m; q += 2)
+    if (m % q == 0) return q;
+  return m;
+}
+
+// Mixed-radix FFT of P pencils of any length: radices 8, 4, then 6 and 10
+// (which take a remaining factor 2 along), 2, 9, 3, 5 and 7, then the primes
+// from 11 up.
+template <int DIR, int LAY, int MAXV, int TPB>
+__device__ __forceinline__ void fft_mixed(float2* s, int n, int P, int lP,
+                                          const float2* __restrict__ tw, int tws) {
+#define PMX_STAGE(R) fft_mix_stage<R, DIR, LAY, MAXV, TPB>(s, n, P, Ns, lP, tw, tws), Ns *= R, rem /= R
+  int Ns = 1, rem = n;
+  while (rem > 1) {
+    if (rem % 8 == 0) PMX_STAGE(8);
+    else if (rem % 4 == 0) PMX_STAGE(4);
+    else if (rem % 6 == 0) PMX_STAGE(6);
+    else if (rem % 10 == 0) PMX_STAGE(10);
+    else if (rem % 2 == 0) PMX_STAGE(2);
+    else if (rem % 9 == 0) PMX_STAGE(9);
+    else if (rem % 3 == 0) PMX_STAGE(3);
+    else if (rem % 5 == 0) PMX_STAGE(5);
+    else if (rem % 7 == 0) PMX_STAGE(7);
+    else {
+      const int R = prime_factor(rem);
+      fft_prime_stage<DIR, LAY, MAXV, TPB>(s, n, P, Ns, R, lP, tw, tws);
+      Ns *= R;
+      rem /= R;
+    }
+  }
+#undef PMX_STAGE
+}
+
 // Unnormalised in-LDS FFT of P pencils (exp(DIR 2 pi i jk/n)).  POW2
-// selects the Stockham path (n and P powers of two) or the direct DFT.  tw
+// selects the power-of-two stages or the mixed-radix ones.  tw
 // is a table of exp(-2 pi i m/(n tws)); tws > 1 reuses a longer table.
 // Callers synchronise before it; it ends with a barrier.
-template <int DIR, int LAY, bool POW2, int MAXV = FFT_MAXV, int TPB = FFT_TPB>
+template <int DIR, int LAY, bool POW2, int MAXV, int TPB>
 __device__ __forceinline__ void lds_fft(float2* s, int n, int P, const float2* __restrict__ tw,
                                         int tws = 1) {
   if (n == 1) return;
+  const int lP = __ffs(P) - 1;
   if (!POW2) {
-    fft_direct<DIR, LAY, MAXV, TPB>(s, n, P, tw, tws);
+    fft_mixed<DIR, LAY, MAXV, TPB>(s, n, P, lP, tw, tws);
     return;
   }
-  const int lP = __ffs(P) - 1;
   int Ns = 1;
   while (Ns < n) {
     int rem = n / Ns;
@@ -309,7 +534,7 @@ __device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ t
   int ob[NG];
 #pragma unroll
   for (int it = 0; it < NG; ++it) {
-    const int idx = threadIdx.x + it * TPB;
+    const int idx = threadIdx.x + it * tpb<TPB>();
     if (FULL || idx < TOTAL) {
       const int p = LAY == ROWS ? idx >> LNB : idx & (P - 1);
       const int j = LAY == ROWS ? idx & (NB - 1) : idx >> LP;
@@ -334,7 +559,7 @@ __device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ t
   }
 #pragma unroll
   for (int it = 0; it < NG; ++it) {
-    const int idx = threadIdx.x + it * TPB;
+    const int idx = threadIdx.x + it * tpb<TPB>();
     if (FULL || idx < TOTAL) {
       float2* u = &v[it * R];
       if (NS > 1) {
@@ -355,7 +580,7 @@ __device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ t
   __syncthreads();
 #pragma unroll
   for (int it = 0; it < NG; ++it) {
-    const int idx = threadIdx.x + it * TPB;
+    const int idx = threadIdx.x + it * tpb<TPB>();
     if (FULL || idx < TOTAL) {
       if (SEP_OUT) {
 #pragma unroll
@@ -402,12 +627,12 @@ __device__ __forceinline__ void batch_copy(int total, LD ld, ST st) {
   float2 r[MAXV];
 #pragma unroll
   for (int it = 0; it < MAXV; ++it) {
-    int idx = threadIdx.x + it * TPB;
+    int idx = threadIdx.x + it * tpb<TPB>();
     if (idx < total) r[it] = ld(idx);
   }
 #pragma unroll
   for (int it = 0; it < MAXV; ++it) {
-    int idx = threadIdx.x + it * TPB;
+    int idx = threadIdx.x + it * tpb<TPB>();
     if (idx < total) st(idx, r[it]);
   }
 }
@@ -415,7 +640,7 @@ __device__ __forceinline__ void batch_copy(int total, LD ld, ST st) {
 // Copies the twiddle table tw[0, n) to LDS (no barrier).
 template <int TPB>
 __device__ __forceinline__ void stage_twiddles(float2* stw, const float2* __restrict__ tw, int n) {
-  for (int base = 0; base < n; base += 4 * TPB)
+  for (int base = 0; base < n; base += 4 * tpb<TPB>())
     batch_copy<4, TPB>(n - base, [&](int i) { return tw[base + i]; },
                        [&](int i, float2 v) { stw[base + i] = v; });
 }
@@ -430,104 +655,136 @@ __device__ __forceinline__ unsigned pass_block(unsigned lin, unsigned nb, int re
 }
 
 // ------------------------------------------------------------ z passes --
-// In-place r2c of padded rows as a length-n2 complex FFT of the real row
-// (any n2); PRE applies (x - 1) * coef on load (gravity.py:52-54).
-// LDS: the row block, then the n2-entry twiddle table.
+// Up to three meshes of one row pass: block b works on field b / nblk, in the
+// block order of pass_block (rev per field).  fold: the halo shells of field
+// i lie i * hstride floats into the halo.
+struct RowFields {
+  float* f[3];
+  int rev[3];
+  unsigned nblk;
+  long long hstride;
+};
+__device__ __forceinline__ int row_field(unsigned nblk, int rev0, int rev1, int rev2, unsigned& blk) {
+  const unsigned i = blockIdx.x / nblk;
+  blk = pass_block(blockIdx.x - i * nblk, nblk, i == 0 ? rev0 : (i == 1 ? rev1 : rev2));
+  return (int)i;
+}
+#define PMX_ROW_FIELD(rf, blk) row_field((rf).nblk, (rf).rev[0], (rf).rev[1], (rf).rev[2], blk)
+#define PMX_ROW_DATA(rf, i) ((i) == 0 ? (rf).f[0] : ((i) == 1 ? (rf).f[1] : (rf).f[2]))
+
+// In-place r2c of padded rows by a length-n2 complex FFT (odd n2; even ones
+// take z_r2c_half_k): two rows a and b are transformed as z = a + i b, and
+//   A[k] = (Z[k] + conj Z[n2-k]) / 2,  B[k] = -i (Z[k] - conj Z[n2-k]) / 2.
+// PRE applies (x - 1) * coef on load (gravity.py:52-54).  A block takes P
+// pairs of rows.  LDS: the P pencils, then the n2-entry twiddle table.
 template <int PRE, bool POW2>
-__global__ void __launch_bounds__(FFT_TPB, 4) z_r2c_k(float* __restrict__ data, long long nrows, int n2,
-                                                      int rs, int P, float coef,
+__global__ void __launch_bounds__(GEN_MAXTPB, 4) z_r2c_k(RowFields rf, long long nrows, int n2, int rs,
+                                                      int P, float coef,
                                                       const float2* __restrict__ tw,
                                                       const float* __restrict__ fcoef) {
   extern __shared__ float2 s[];
   if (PRE && fcoef) coef = fcoef[0];
   float2* stw = s + lds_elems(ROWS, n2, P);
-  long long row0 = (long long)blockIdx.x * P;
-  int np = (int)((nrows - row0) < P ? (nrows - row0) : P);
-  stage_twiddles<FFT_TPB>(stw, tw, n2);
-  batch_copy<RFFT_MAXV, FFT_TPB>(
+  unsigned blk;
+  const int field = PMX_ROW_FIELD(rf, blk);
+  float* data = PMX_ROW_DATA(rf, field);
+  const long long row0 = (long long)blk * 2 * P;
+  const int nr = (int)((nrows - row0) < 2 * P ? (nrows - row0) : 2 * P);
+  const int np = (nr + 1) / 2;
+  const FastDiv dn(n2);
+  stage_twiddles<GEN_TPB>(stw, tw, n2);
+  batch_copy<GEN_MAXV, GEN_TPB>(
       np * n2,
       [&](int idx) {
-        int p = idx / n2, j = idx - (idx / n2) * n2;
-        float x = data[(row0 + p) * rs + j];
+        const int p = dn(idx), j = idx - p * n2;
+        const float* r = data + (row0 + 2 * p) * rs + j;
+        float2 v = make_float2(r[0], 2 * p + 1 < nr ? r[rs] : 0.f);
         if (PRE) {
-          x = x - 1.f;
-          x = x * coef;
+          v.x = v.x - 1.f;
+          v.x = v.x * coef;
+          v.y = v.y - 1.f;
+          v.y = v.y * coef;
         }
-        return make_float2(x, 0.f);
-      },
-      [&](int idx, float2 v) {
-        int p = idx / n2, j = idx - (idx / n2) * n2;
-        s[lidx<ROWS>(p, j, n2, P)] = v;
-      });
-  __syncthreads();
-  lds_fft<-1, ROWS, POW2, RFFT_MAXV>(s, n2, np, stw);
-  const int n2h = n2 / 2 + 1;
-  float2* out = reinterpret_cast<float2*>(data);
-  const int rsc = rs / 2;
-  batch_copy<RFFT_MAXV, FFT_TPB>(
-      np * n2h,
-      [&](int idx) {
-        int p = idx / n2h, k = idx - (idx / n2h) * n2h;
-        return s[lidx<ROWS>(p, k, n2, P)];
-      },
-      [&](int idx, float2 v) {
-        int p = idx / n2h, k = idx - (idx / n2h) * n2h;
-        out[(row0 + p) * rsc + k] = v;
-      });
-}
-
-// In-place c2r of padded rows with a final scale (any n2).  The full
-// spectrum is rebuilt from the half (X[n-k] = conj X[k]) and the real part
-// of the inverse is kept, which discards Im X[0] and Im X[n/2] as irfft does.
-template <bool POW2>
-__global__ void __launch_bounds__(FFT_TPB, 4) z_c2r_k(float* __restrict__ data, long long nrows, int n2,
-                                                      int rs, int P, float scale,
-                                                      const float2* __restrict__ tw) {
-  extern __shared__ float2 s[];
-  float2* stw = s + lds_elems(ROWS, n2, P);
-  long long row0 = (long long)blockIdx.x * P;
-  int np = (int)((nrows - row0) < P ? (nrows - row0) : P);
-  const float2* in = reinterpret_cast<const float2*>(data);
-  const int rsc = rs / 2;
-  const int half = n2 / 2;
-  stage_twiddles<FFT_TPB>(stw, tw, n2);
-  batch_copy<RFFT_MAXV, FFT_TPB>(
-      np * n2,
-      [&](int idx) {
-        int p = idx / n2, k = idx - (idx / n2) * n2;
-        int kk = k <= half ? k : n2 - k;
-        float2 v = in[(row0 + p) * rsc + kk];
-        if (k > half) v.y = -v.y;
         return v;
       },
       [&](int idx, float2 v) {
-        int p = idx / n2, k = idx - (idx / n2) * n2;
-        s[lidx<ROWS>(p, k, n2, P)] = v;
+        const int p = dn(idx);
+        s[lidx<ROWS>(p, idx - p * n2, n2, P)] = v;
       });
   __syncthreads();
-  lds_fft<1, ROWS, POW2, RFFT_MAXV>(s, n2, np, stw);
-  batch_copy<RFFT_MAXV, FFT_TPB>(
-      np * n2,
-      [&](int idx) {
-        int p = idx / n2, j = idx - (idx / n2) * n2;
-        return s[lidx<ROWS>(p, j, n2, P)];
-      },
-      [&](int idx, float2 v) {
-        int p = idx / n2, j = idx - (idx / n2) * n2;
-        data[(row0 + p) * rs + j] = v.x * scale;
-      });
+  lds_fft<-1, ROWS, POW2, GEN_MAXV, GEN_TPB>(s, n2, np, stw);
+  const int n2h = n2 / 2 + 1;
+  float2* out = reinterpret_cast<float2*>(data);
+  const int rsc = rs / 2;
+  const FastDiv dh(n2h);
+  for (int idx = threadIdx.x; idx < np * n2h; idx += tpb<GEN_TPB>()) {
+    const int p = dh(idx), k = idx - p * n2h;
+    const float2 z = s[lidx<ROWS>(p, k, n2, P)];
+    float2 m = s[lidx<ROWS>(p, k ? n2 - k : 0, n2, P)];
+    m.y = -m.y;
+    float2* o = out + (row0 + 2 * p) * rsc + k;
+    o[0] = make_float2(0.5f * (z.x + m.x), 0.5f * (z.y + m.y));
+    if (2 * p + 1 < nr) o[rsc] = make_float2(0.5f * (z.y - m.y), -0.5f * (z.x - m.x));
+  }
 }
 
-// Half-length r2c for even n2 with H = n2/2 a power of two: the row is read
-// as H complex values z[m] = x[2m] + i x[2m+1], Z = FFT_H(z), and for
-// k = 0..H:  X[k] = E + w^k O,  E = (Z[k] + conj Z[H-k])/2,
+// In-place c2r of padded rows with a final scale (odd n2), two rows a time:
+// Z = A + i B over the full spectra rebuilt from the halves (X[n-k] = conj
+// X[k]), Im X[0] and (even n2) Im X[n2/2] dropped as irfft does; the inverse
+// is a + i b.
+template <bool POW2>
+__global__ void __launch_bounds__(GEN_MAXTPB, 4) z_c2r_k(RowFields rf, long long nrows, int n2, int rs,
+                                                      int P, float scale,
+                                                      const float2* __restrict__ tw) {
+  extern __shared__ float2 s[];
+  float2* stw = s + lds_elems(ROWS, n2, P);
+  unsigned blk;
+  const int field = PMX_ROW_FIELD(rf, blk);
+  float* data = PMX_ROW_DATA(rf, field);
+  const long long row0 = (long long)blk * 2 * P;
+  const int nr = (int)((nrows - row0) < 2 * P ? (nrows - row0) : 2 * P);
+  const int np = (nr + 1) / 2;
+  const float2* in = reinterpret_cast<const float2*>(data);
+  const int rsc = rs / 2;
+  const int half = n2 / 2;
+  const FastDiv dn(n2);
+  stage_twiddles<GEN_TPB>(stw, tw, n2);
+  batch_copy<GEN_MAXV, GEN_TPB>(
+      np * n2,
+      [&](int idx) {
+        const int p = dn(idx), k = idx - p * n2;
+        const int kk = k <= half ? k : n2 - k;
+        const float2* r = in + (row0 + 2 * p) * rsc + kk;
+        float2 a = r[0], b = make_float2(0.f, 0.f);
+        if (2 * p + 1 < nr) b = r[rsc];
+        if (kk == 0 || 2 * kk == n2) a.y = b.y = 0.f;
+        return k <= half ? make_float2(a.x - b.y, a.y + b.x) : make_float2(a.x + b.y, b.x - a.y);
+      },
+      [&](int idx, float2 v) {
+        const int p = dn(idx);
+        s[lidx<ROWS>(p, idx - p * n2, n2, P)] = v;
+      });
+  __syncthreads();
+  lds_fft<1, ROWS, POW2, GEN_MAXV, GEN_TPB>(s, n2, np, stw);
+  for (int idx = threadIdx.x; idx < np * n2; idx += tpb<GEN_TPB>()) {
+    const int p = dn(idx), j = idx - p * n2;
+    const float2 v = s[lidx<ROWS>(p, j, n2, P)];
+    float* r = data + (row0 + 2 * p) * rs + j;
+    r[0] = v.x * scale;
+    if (2 * p + 1 < nr) r[rs] = v.y * scale;
+  }
+}
+
+// Half-length r2c for even n2, H = n2/2: the row is read as H complex values z[m] = x[2m] + i x[2m+1],
+// Z = FFT_H(z), and for k = 0..H:  X[k] = E + w^k O,  E = (Z[k] + conj Z[H-k])/2,
 // O = -i (Z[k] - conj Z[H-k])/2,  w = exp(-2 pi i/n2)  (Z[H] = Z[0]).
 // PRE applies (x - 1) * coef on load.  LH > 0 fixes H = 2^LH and
-// P = row_pencils(H) at compile time (the launch then holds whole blocks).
+// P = ct_rows(LH, SM) at compile time (the launch then holds whole blocks);
+// LH = 0 takes any H, POW2 telling whether it is a power of two.
 __device__ __forceinline__ float2 r2c_half_x(const float2* s, const float2* stw, int p, int k, int H,
                                              int P) {
-  float2 zk = s[lidx<ROWS>(p, k & (H - 1), H, P)];
-  float2 zm = s[lidx<ROWS>(p, (H - k) & (H - 1), H, P)];
+  float2 zk = s[lidx<ROWS>(p, k == H ? 0 : k, H, P)];
+  float2 zm = s[lidx<ROWS>(p, k == 0 ? 0 : H - k, H, P)];
   zm.y = -zm.y;
   float2 e = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y + zm.y));
   float2 dd = csub(zk, zm);
@@ -615,7 +872,7 @@ __device__ __forceinline__ void fold_rows(float2 (&r)[NV], const FoldIn& fi, int
   const int lx = x & 15;
 #pragma unroll
   for (int it = 0; it < NV; ++it) {
-    const int idx = threadIdx.x + it * TPB;
+    const int idx = threadIdx.x + it * tpb<TPB>();
     if (idx >= total) continue;
     const int p = idx >> lH, y = y0 + p, m = idx & (H - 1);
     const int ly = y & 15, z = 2 * m, lz = z & 15, k = (m >> 3) * P + p;
@@ -641,28 +898,43 @@ __device__ __forceinline__ void fold_rows(float2 (&r)[NV], const FoldIn& fi, int
   }
 }
 
+// Splits a block's value index into row and position (shifts when H = 2^LH).
+template <int LH>
+struct RowSplit {
+  int H;
+  FastDiv d;
+  __device__ __forceinline__ explicit RowSplit(int H_) : H(H_), d(LH ? 1 : H_) {}
+  __device__ __forceinline__ int row(int idx) const { return LH ? idx >> LH : d(idx); }
+  __device__ __forceinline__ int col(int idx, int p) const {
+    return LH ? idx & ((1 << LH) - 1) : idx - p * H;
+  }
+};
+
 // FOLD (with LH > 0, 16^3 tiles, P | n1): the density is the deposit's tile
 // interiors plus the fold of fi.halo, added here on load.
-template <int PRE, int LH, bool FOLD = false>
-__global__ void __launch_bounds__(FFT_TPB, 4) z_r2c_half_k(float* __restrict__ data, long long nrows,
-                                                           int n2, int rs, int P_, float coef,
-                                                           const float2* __restrict__ tw,
-                                                           FoldIn fi, const float* __restrict__ fcoef,
-                                                           int rev) {
+template <int PRE, int LH, bool SM, bool FOLD, bool POW2>
+__global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
+    z_r2c_half_k(RowFields rf, long long nrows, int n2, int rs, int P_, float coef,
+                 const float2* __restrict__ tw, FoldIn fi, const float* __restrict__ fcoef) {
   extern __shared__ float2 s[];
   // 1.5 Omega_m from the device factor table when the call has one
   if (PRE && fcoef) coef = fcoef[0];
-  constexpr int PC = LH ? row_pencils(1 << LH) : 1;
+  constexpr int PC = LH ? ct_rows(LH, SM) : 1;
+  constexpr int TPB = LH ? ct_row_tpb(LH, SM) : GEN_TPB;
+  constexpr int MAXV = LH ? (PC << LH) / TPB : GEN_MAXV;
   const int H = LH ? 1 << LH : n2 >> 1;
-  const int lH = LH ? LH : __ffs(H) - 1;
   const int P = LH ? PC : P_;
+  const RowSplit<LH> rsp(H);
   float2* stw = s + lds_elems(ROWS, H, P);
-  const long long row0 = (long long)pass_block(blockIdx.x, gridDim.x, rev) * P;
+  unsigned bk;
+  const int field = PMX_ROW_FIELD(rf, bk);
+  const long long row0 = (long long)bk * P;
   const int np = LH ? PC : (int)((nrows - row0) < P ? (nrows - row0) : P);
   const int rsc = rs / 2;
-  float2* blk = reinterpret_cast<float2*>(data) + row0 * rsc;
+  float2* blk = reinterpret_cast<float2*>(PMX_ROW_DATA(rf, field)) + row0 * rsc;
   const int total = np * H;
-  stage_twiddles<FFT_TPB>(stw, tw, 2 * H);
+  if (FOLD) fi.halo += field * rf.hstride;
+  stage_twiddles<TPB>(stw, tw, 2 * H);
   // the block's rows lie in one x plane when folding
   const int fx = FOLD ? (int)row0 / fi.n1 : 0;
   const int fy0 = FOLD ? (int)row0 - fx * fi.n1 : 0;
@@ -674,12 +946,13 @@ __global__ void __launch_bounds__(FFT_TPB, 4) z_r2c_half_k(float* __restrict__ d
     float* Z0 = T + PC * 2 * H;
     float* Z1 = Z0 + PC * (H >> 3);
     float z0 = 0.f, z1 = 0.f;
-    if (FOLD) fold_tables<PC, FFT_TPB>(fi, fx, fy0, lH, H, T, z0, z1);
-    float2 r[RFFT_MAXV];
+    if (FOLD) fold_tables<PC, TPB>(fi, fx, fy0, LH, H, T, z0, z1);
+    float2 r[MAXV];
 #pragma unroll
-    for (int it = 0; it < RFFT_MAXV; ++it) {
-      const int idx = threadIdx.x + it * FFT_TPB;
-      if (idx < total) r[it] = blk[__umul24(idx >> lH, rsc) + (idx & (H - 1))];
+    for (int it = 0; it < MAXV; ++it) {
+      const int idx = threadIdx.x + it * tpb<TPB>();
+      const int p = rsp.row(idx);
+      if (idx < total) r[it] = blk[__umul24(p, rsc) + rsp.col(idx, p)];
     }
     if (FOLD) {
       if ((int)threadIdx.x < PC * (H >> 3)) {
@@ -688,12 +961,12 @@ __global__ void __launch_bounds__(FFT_TPB, 4) z_r2c_half_k(float* __restrict__ d
       }
       __builtin_amdgcn_s_waitcnt(0);  // T's loads into LDS have landed
       __syncthreads();
-      fold_rows<RFFT_MAXV, FFT_TPB, PC>(r, fi, fx, fy0, lH, H, total, T, Z0, Z1);
+      fold_rows<MAXV, TPB, PC>(r, fi, fx, fy0, LH, H, total, T, Z0, Z1);
       __syncthreads();  // T is read before the rows take its place
     }
     if (PRE) {
 #pragma unroll
-      for (int it = 0; it < RFFT_MAXV; ++it) {
+      for (int it = 0; it < MAXV; ++it) {
         r[it].x = r[it].x - 1.f;
         r[it].x = r[it].x * coef;
         r[it].y = r[it].y - 1.f;
@@ -701,69 +974,77 @@ __global__ void __launch_bounds__(FFT_TPB, 4) z_r2c_half_k(float* __restrict__ d
       }
     }
 #pragma unroll
-    for (int it = 0; it < RFFT_MAXV; ++it) {
-      const int idx = threadIdx.x + it * FFT_TPB;
-      if (idx < total) s[lidx<ROWS>(idx >> lH, idx & (H - 1), H, P)] = r[it];
+    for (int it = 0; it < MAXV; ++it) {
+      const int idx = threadIdx.x + it * tpb<TPB>();
+      const int p = rsp.row(idx);
+      if (idx < total) s[lidx<ROWS>(p, rsp.col(idx, p), H, P)] = r[it];
     }
   }
   __syncthreads();
-  fft_run<-1, ROWS, true, LH, ilog2c(PC), RFFT_MAXV, FFT_TPB, 2>(s, H, np, stw);
+  fft_run<-1, ROWS, POW2, LH, ilog2c(PC), MAXV, TPB, 2>(s, H, np, stw);
   {
-    float2 r[RFFT_MAXV];
+    float2 r[MAXV];
 #pragma unroll
-    for (int it = 0; it < RFFT_MAXV; ++it) {
-      const int idx = threadIdx.x + it * FFT_TPB;
-      if (idx < total) r[it] = r2c_half_x(s, stw, idx >> lH, idx & (H - 1), H, P);
+    for (int it = 0; it < MAXV; ++it) {
+      const int idx = threadIdx.x + it * tpb<TPB>();
+      const int p = rsp.row(idx);
+      if (idx < total) r[it] = r2c_half_x(s, stw, p, rsp.col(idx, p), H, P);
     }
 #pragma unroll
-    for (int it = 0; it < RFFT_MAXV; ++it) {
-      const int idx = threadIdx.x + it * FFT_TPB;
-      if (idx < total) blk[__umul24(idx >> lH, rsc) + (idx & (H - 1))] = r[it];
+    for (int it = 0; it < MAXV; ++it) {
+      const int idx = threadIdx.x + it * tpb<TPB>();
+      const int p = rsp.row(idx);
+      if (idx < total) blk[__umul24(p, rsc) + rsp.col(idx, p)] = r[it];
     }
     // X[H] of each row
-    if ((int)threadIdx.x < np)
-      blk[__umul24(threadIdx.x, rsc) + H] = r2c_half_x(s, stw, threadIdx.x, H, H, P);
+    for (int p = threadIdx.x; p < np; p += tpb<TPB>()) blk[__umul24(p, rsc) + H] = r2c_half_x(s, stw, p, H, H, P);
   }
 }
 
 // Half-length c2r (inverse of the above) with a final scale:
 // Z[k] = (X[k] + conj X[H-k]) + i w^-k (X[k] - conj X[H-k]) for k < H with
 // Im X[0] = Im X[H] = 0 (as irfft), z = IFFT_H(Z), x[2m] + i x[2m+1] = z[m].
-// LH as in z_r2c_half_k.
-template <int LH>
-__global__ void __launch_bounds__(FFT_TPB, 4) z_c2r_half_k(float* __restrict__ data, long long nrows,
-                                                           int n2, int rs, int P_, float scale,
-                                                           const float2* __restrict__ tw, int rev) {
+// LH, SM and POW2 as in z_r2c_half_k.
+template <int LH, bool SM, bool POW2>
+__global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
+    z_c2r_half_k(RowFields rf, long long nrows, int n2, int rs, int P_, float scale,
+                 const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
-  constexpr int PC = LH ? row_pencils(1 << LH) : 1;
+  constexpr int PC = LH ? ct_rows(LH, SM) : 1;
+  constexpr int TPB = LH ? ct_row_tpb(LH, SM) : GEN_TPB;
+  constexpr int MAXV = LH ? (PC << LH) / TPB : GEN_MAXV;
   const int H = LH ? 1 << LH : n2 >> 1;
-  const int lH = LH ? LH : __ffs(H) - 1;
   const int P = LH ? PC : P_;
+  const RowSplit<LH> rsp(H);
   float2* stw = s + lds_elems(ROWS, H, P);
-  const long long row0 = (long long)pass_block(blockIdx.x, gridDim.x, rev) * P;
+  unsigned bk;
+  const int field = PMX_ROW_FIELD(rf, bk);
+  float* data = PMX_ROW_DATA(rf, field);
+  const long long row0 = (long long)bk * P;
   const int np = LH ? PC : (int)((nrows - row0) < P ? (nrows - row0) : P);
   const int rsc = rs / 2;
   float2* blk = reinterpret_cast<float2*>(data) + row0 * rsc;
   const int total = np * H;
-  stage_twiddles<FFT_TPB>(stw, tw, 2 * H);
+  stage_twiddles<TPB>(stw, tw, 2 * H);
   // X[k] and X[H-k] per thread: both loads of the batch are issued first
-  float2 xa[RFFT_MAXV], xb[RFFT_MAXV];
+  float2 xa[MAXV], xb[MAXV];
 #pragma unroll
-  for (int it = 0; it < RFFT_MAXV; ++it) {
-    const int idx = threadIdx.x + it * FFT_TPB;
+  for (int it = 0; it < MAXV; ++it) {
+    const int idx = threadIdx.x + it * tpb<TPB>();
+    const int p = rsp.row(idx);
     if (idx < total) {
-      const float2* row = blk + __umul24(idx >> lH, rsc);
-      const int k = idx & (H - 1);
+      const float2* row = blk + __umul24(p, rsc);
+      const int k = rsp.col(idx, p);
       xa[it] = row[k];
       xb[it] = row[H - k];
     }
   }
   __syncthreads();  // the twiddle table is read below
 #pragma unroll
-  for (int it = 0; it < RFFT_MAXV; ++it) {
-    const int idx = threadIdx.x + it * FFT_TPB;
+  for (int it = 0; it < MAXV; ++it) {
+    const int idx = threadIdx.x + it * tpb<TPB>();
     if (idx < total) {
-      const int p = idx >> lH, k = idx & (H - 1);
+      const int p = rsp.row(idx), k = rsp.col(idx, p);
       float2 a = xa[it], b = xb[it];
       if (k == 0) {
         a.y = 0.f;
@@ -777,18 +1058,20 @@ __global__ void __launch_bounds__(FFT_TPB, 4) z_c2r_half_k(float* __restrict__ d
     }
   }
   __syncthreads();
-  fft_run<1, ROWS, true, LH, ilog2c(PC), RFFT_MAXV, FFT_TPB, 2>(s, H, np, stw);
-  float2 r[RFFT_MAXV];
+  fft_run<1, ROWS, POW2, LH, ilog2c(PC), MAXV, TPB, 2>(s, H, np, stw);
+  float2 r[MAXV];
 #pragma unroll
-  for (int it = 0; it < RFFT_MAXV; ++it) {
-    const int idx = threadIdx.x + it * FFT_TPB;
-    if (idx < total) r[it] = s[lidx<ROWS>(idx >> lH, idx & (H - 1), H, P)];
+  for (int it = 0; it < MAXV; ++it) {
+    const int idx = threadIdx.x + it * tpb<TPB>();
+    const int p = rsp.row(idx);
+    if (idx < total) r[it] = s[lidx<ROWS>(p, rsp.col(idx, p), H, P)];
   }
 #pragma unroll
-  for (int it = 0; it < RFFT_MAXV; ++it) {
-    const int idx = threadIdx.x + it * FFT_TPB;
+  for (int it = 0; it < MAXV; ++it) {
+    const int idx = threadIdx.x + it * tpb<TPB>();
+    const int p = rsp.row(idx);
     if (idx < total)
-      blk[__umul24(idx >> lH, rsc) + (idx & (H - 1))] = make_float2(r[it].x * scale, r[it].y * scale);
+      blk[__umul24(p, rsc) + rsp.col(idx, p)] = make_float2(r[it].x * scale, r[it].y * scale);
   }
 }
 
@@ -823,7 +1106,7 @@ __device__ __forceinline__ ColMap col_map(int lB) {
   ColMap m;
   m.b = threadIdx.x & ((1 << lB) - 1);
   m.j0 = threadIdx.x >> lB;
-  m.js = TPB >> lB;
+  m.js = tpb<TPB>() >> lB;
   return m;
 }
 
@@ -831,13 +1114,15 @@ __device__ __forceinline__ ColMap col_map(int lB) {
 // element j of pencil (o, c) is at o*ostride + j*es + c.  A workgroup takes
 // B consecutive columns, so each of its loads is B contiguous float2.
 // LDS: the n x B block, then the n-entry twiddle table.  LN > 0 fixes
-// n = 2^LN and B = fft_pencils(n) at compile time.
+// n = 2^LN and B = ct_cols(LN, FFT_CAP) at compile time.
 template <int DIR, bool POW2, int LN>
-__global__ void __launch_bounds__(FFT_TPB, 4) strided_fft_k(Fields3 fl, int n_, long long es,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) : GEN_MAXTPB, 4) strided_fft_k(Fields3 fl, int n_, long long es,
                                                          long long ostride, int ncol, int B_,
                                                          const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
-  constexpr int BC = LN ? fft_pencils(1 << LN) : 1;
+  constexpr int BC = LN ? ct_cols(LN, FFT_CAP) : 1;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, FFT_V) : GEN_TPB;
+  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
   const int n = LN ? 1 << LN : n_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
@@ -846,28 +1131,28 @@ __global__ void __launch_bounds__(FFT_TPB, 4) strided_fft_k(Fields3 fl, int n_, 
   xcd_block3(bx, by, bz, fl.rev);
   const int c0 = bx * B;
   const int nb = ncol - c0 < B ? ncol - c0 : B;
-  const ColMap cm = col_map<FFT_TPB>(lB);
+  const ColMap cm = col_map<TPB>(lB);
   const bool live = cm.b < nb;
   float2* g = (bz == 0 ? fl.f[0] : (bz == 1 ? fl.f[1] : fl.f[2])) + (long long)by * ostride + c0 +
               cm.b + (long long)cm.j0 * es;
   const long long gs = (long long)cm.js * es;
-  stage_twiddles<FFT_TPB>(stw, tw, n);
-  float2 r[FFT_MAXV];
+  stage_twiddles<TPB>(stw, tw, n);
+  float2 r[MAXV];
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     r[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n) r[it] = g[it * gs];
   }
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * FFT_TPB] = r[it];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * tpb<TPB>()] = r[it];
   __syncthreads();
-  fft_run<DIR, COLS, POW2, LN, ilog2c(BC), FFT_MAXV, FFT_TPB>(s, n, B, stw);
+  fft_run<DIR, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * FFT_TPB];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * tpb<TPB>()];
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
+  for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n) g[it * gs] = r[it];
 }
 
@@ -888,10 +1173,12 @@ struct KTab {
 // columns.  LDS: the n0 x B block, the n0-entry twiddle table, then the k_0
 // and km_0 tables.
 template <bool POW2, int LN, bool KIN = false>
-__global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(PFFT_WPE))) poisson_x_k(Fields3 fl, int n0_, int n1, int n2h, int n2p,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V) : GEN_MAXTPB) poisson_x_k(Fields3 fl, int n0_, int n1, int n2h, int n2p,
                                                        int B_, KTab kt, const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
-  constexpr int BC = LN ? fft_pencils(1 << LN, PFFT_CAP) : 1;
+  constexpr int BC = LN ? ct_cols(LN, PFFT_CAP) : 1;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, PFFT_V) : GEN_TPB;
+  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
   const int n0 = LN ? 1 << LN : n0_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
@@ -904,37 +1191,37 @@ __global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(P
   const int c0 = bx * B;
   const int nb = n2h - c0 < B ? n2h - c0 : B;
   const long long off = (long long)y * n2p + c0;
-  stage_twiddles<PFFT_TPB>(stw, tw, n0);
-  for (int i = threadIdx.x; i < n0; i += PFFT_TPB) {
+  stage_twiddles<TPB>(stw, tw, n0);
+  for (int i = threadIdx.x; i < n0; i += tpb<TPB>()) {
     sk[i] = kt.k[0][i];
     skm[i] = kt.km[0][i];
   }
-  const ColMap cm = col_map<PFFT_TPB>(lB);
+  const ColMap cm = col_map<TPB>(lB);
   const bool live = cm.b < nb;
   float2* g0 = fl.f[0] + off + cm.b + (long long)cm.j0 * es;
   float2* g1 = fl.f[1] + off + cm.b + (long long)cm.j0 * es;
   const long long gs = (long long)cm.js * es;
-  float2 r[PFFT_MAXV];
+  float2 r[MAXV];
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     r[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n0) r[it] = g0[it * gs];
   }
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * PFFT_TPB] = r[it];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = r[it];
   __syncthreads();
   // KIN: the input is already transformed along x (a full 3D spectrum)
-  if constexpr (!KIN) fft_run<-1, COLS, POW2, LN, ilog2c(BC), PFFT_MAXV, PFFT_TPB>(s, n0, B, stw);
+  if constexpr (!KIN) fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
   const float ky = kt.k[1][y];
   const float kz = live ? kt.k[2][c0 + cm.b] : 0.f;
-  float2 h[PFFT_MAXV];
+  float2 h[MAXV];
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     const int j = cm.j0 + it * cm.js;
     h[it] = make_float2(0.f, 0.f);
     if (live && j < n0) {
-      float2 v = s[threadIdx.x + it * PFFT_TPB];
+      float2 v = s[threadIdx.x + it * tpb<TPB>()];
       float kx = sk[j];
       float k2 = kx * kx;
       k2 = k2 + ky * ky;
@@ -949,33 +1236,33 @@ __global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(P
   __syncthreads();
   // x component: IFFT_x(km_0 h) to c_0
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     const int j = cm.j0 + it * cm.js;
     if (j < n0) {
       const float kmx = skm[j];
-      s[threadIdx.x + it * PFFT_TPB] = make_float2(kmx * h[it].x, kmx * h[it].y);
+      s[threadIdx.x + it * tpb<TPB>()] = make_float2(kmx * h[it].x, kmx * h[it].y);
     }
   }
   __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), PFFT_MAXV, PFFT_TPB>(s, n0, B, stw);
+  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) r[it] = s[threadIdx.x + it * PFFT_TPB];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n0) r[it] = s[threadIdx.x + it * tpb<TPB>()];
   __syncthreads();
   // h to c_1
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * PFFT_TPB] = h[it];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = h[it];
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
+  for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n0) g0[it * gs] = r[it];
   __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), PFFT_MAXV, PFFT_TPB>(s, n0, B, stw);
+  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) r[it] = s[threadIdx.x + it * PFFT_TPB];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n0) r[it] = s[threadIdx.x + it * tpb<TPB>()];
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
+  for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n0) g1[it * gs] = r[it];
 }
 
@@ -987,10 +1274,12 @@ __global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(P
 // LDS block (the first result kept in registers), then the inverse of the
 // sum.  LDS as poisson_x_k.
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(PFFT_WPE))) poisson_x_adj_k(Fields3 fl, int n0_, int n1, int n2h, int n2p,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V) : GEN_MAXTPB) poisson_x_adj_k(Fields3 fl, int n0_, int n1, int n2h, int n2p,
                                                            int B_, KTab kt, const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
-  constexpr int BC = LN ? fft_pencils(1 << LN, PFFT_CAP) : 1;
+  constexpr int BC = LN ? ct_cols(LN, PFFT_CAP) : 1;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, PFFT_V) : GEN_TPB;
+  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
   const int n0 = LN ? 1 << LN : n0_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
@@ -1003,49 +1292,49 @@ __global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(P
   const int c0 = bx * B;
   const int nb = n2h - c0 < B ? n2h - c0 : B;
   const long long off = (long long)y * n2p + c0;
-  stage_twiddles<PFFT_TPB>(stw, tw, n0);
-  for (int i = threadIdx.x; i < n0; i += PFFT_TPB) {
+  stage_twiddles<TPB>(stw, tw, n0);
+  for (int i = threadIdx.x; i < n0; i += tpb<TPB>()) {
     sk[i] = kt.k[0][i];
     skm[i] = kt.km[0][i];
   }
-  const ColMap cm = col_map<PFFT_TPB>(lB);
+  const ColMap cm = col_map<TPB>(lB);
   const bool live = cm.b < nb;
   float2* g0 = fl.f[0] + off + cm.b + (long long)cm.j0 * es;
   const float2* g1 = fl.f[1] + off + cm.b + (long long)cm.j0 * es;
   const long long gs = (long long)cm.js * es;
-  float2 x0[PFFT_MAXV];
+  float2 x0[MAXV];
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     x0[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n0) x0[it] = g0[it * gs];
   }
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * PFFT_TPB] = x0[it];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = x0[it];
   __syncthreads();
-  fft_run<-1, COLS, POW2, LN, ilog2c(BC), PFFT_MAXV, PFFT_TPB>(s, n0, B, stw);
+  fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
   {
-    float2 yz[PFFT_MAXV];
+    float2 yz[MAXV];
 #pragma unroll
-    for (int it = 0; it < PFFT_MAXV; ++it) {
+    for (int it = 0; it < MAXV; ++it) {
       yz[it] = make_float2(0.f, 0.f);
       if (live && cm.j0 + it * cm.js < n0) yz[it] = g1[it * gs];
     }
 #pragma unroll
-    for (int it = 0; it < PFFT_MAXV; ++it)
-      if (cm.j0 + it * cm.js < n0) x0[it] = s[threadIdx.x + it * PFFT_TPB];
+    for (int it = 0; it < MAXV; ++it)
+      if (cm.j0 + it * cm.js < n0) x0[it] = s[threadIdx.x + it * tpb<TPB>()];
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < PFFT_MAXV; ++it)
-      if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * PFFT_TPB] = yz[it];
+    for (int it = 0; it < MAXV; ++it)
+      if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = yz[it];
   }
   __syncthreads();
-  fft_run<-1, COLS, POW2, LN, ilog2c(BC), PFFT_MAXV, PFFT_TPB>(s, n0, B, stw);
+  fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
   const float ky = kt.k[1][y];
   const float kz = live ? kt.k[2][c0 + cm.b] : 0.f;
-  float2 acc[PFFT_MAXV];
+  float2 acc[MAXV];
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     const int j = cm.j0 + it * cm.js;
     acc[it] = make_float2(0.f, 0.f);
     if (live && j < n0) {
@@ -1055,7 +1344,7 @@ __global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(P
       k2 = k2 + kz * kz;
       if (k2 != 0.f) {
         const float kmx = skm[j];
-        const float2 w = s[threadIdx.x + it * PFFT_TPB];
+        const float2 w = s[threadIdx.x + it * tpb<TPB>()];
         float sx = kmx * x0[it].x + w.x, sy = kmx * x0[it].y + w.y;
         // pot = -sum / k^2, acc = -i pot = (pot.y, -pot.x)
         const float q = 1.f / k2;
@@ -1065,20 +1354,20 @@ __global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(P
   }
   __syncthreads();
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * PFFT_TPB] = acc[it];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = acc[it];
   __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), PFFT_MAXV, PFFT_TPB>(s, n0, B, stw);
+  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) acc[it] = s[threadIdx.x + it * PFFT_TPB];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n0) acc[it] = s[threadIdx.x + it * tpb<TPB>()];
 #pragma unroll
-  for (int it = 0; it < PFFT_MAXV; ++it)
+  for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n0) g0[it * gs] = acc[it];
 }
 
 // y passes of the gradient components, paired (pencils along axis 1 of
-// (n0,n1,n2h); blockIdx.y = x row, blockIdx.x = block of B = fft_pencils(n)
+// (n0,n1,n2h); blockIdx.y = x row, blockIdx.x = block of B
 // kz columns, 128-byte segments at n = 512; LDS: the n x B block, then the
 // twiddle table).  The two transforms run one after the other in the same
 // LDS block.
@@ -1092,11 +1381,13 @@ __global__ void __launch_bounds__(PFFT_TPB) __attribute__((amdgpu_waves_per_eu(P
 // of c_2, then their combination km_1 FFT_y(c_1) + km_2 FFT_y(c_2) to c_1
 // for poisson_x_adj_k.
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(FFT_TPB, 2) y_inv_seq_k(Fields3 fl, int n_, long long es,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) : GEN_MAXTPB, 2) y_inv_seq_k(Fields3 fl, int n_, long long es,
                                                         long long ostride, int ncol, int B_,
                                                         KTab kt, const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
-  constexpr int BC = LN ? fft_pencils(1 << LN) : 1;
+  constexpr int BC = LN ? ct_cols(LN, FFT_CAP) : 1;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, FFT_V) : GEN_TPB;
+  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
   const int n = LN ? 1 << LN : n_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
@@ -1106,56 +1397,58 @@ __global__ void __launch_bounds__(FFT_TPB, 2) y_inv_seq_k(Fields3 fl, int n_, lo
   const int c0 = bx * B;
   const int nb = ncol - c0 < B ? ncol - c0 : B;
   const long long off = (long long)by * ostride + c0;
-  stage_twiddles<FFT_TPB>(stw, tw, n);
-  const ColMap cm = col_map<FFT_TPB>(lB);
+  stage_twiddles<TPB>(stw, tw, n);
+  const ColMap cm = col_map<TPB>(lB);
   const bool live = cm.b < nb;
   const float kmz = live ? kt.km[2][c0 + cm.b] : 0.f;
   float2* g1 = fl.f[1] + off + cm.b + (long long)cm.j0 * es;
   float2* g2 = fl.f[2] + off + cm.b + (long long)cm.j0 * es;
   const long long gs = (long long)cm.js * es;
-  float2 h[FFT_MAXV], r[FFT_MAXV];
+  float2 h[MAXV], r[MAXV];
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     h[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n) h[it] = g1[it * gs];
   }
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     const int j = cm.j0 + it * cm.js;
     if (j < n) {
       const float kmy = kt.km[1][j];
-      s[threadIdx.x + it * FFT_TPB] = make_float2(kmy * h[it].x, kmy * h[it].y);
+      s[threadIdx.x + it * tpb<TPB>()] = make_float2(kmy * h[it].x, kmy * h[it].y);
     }
   }
   __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), FFT_MAXV, FFT_TPB>(s, n, B, stw);
+  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * FFT_TPB];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * tpb<TPB>()];
   __syncthreads();
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
+  for (int it = 0; it < MAXV; ++it)
     if (cm.j0 + it * cm.js < n)
-      s[threadIdx.x + it * FFT_TPB] = make_float2(kmz * h[it].x, kmz * h[it].y);
+      s[threadIdx.x + it * tpb<TPB>()] = make_float2(kmz * h[it].x, kmz * h[it].y);
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
+  for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n) g1[it * gs] = r[it];
   __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), FFT_MAXV, FFT_TPB>(s, n, B, stw);
+  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * FFT_TPB];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * tpb<TPB>()];
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
+  for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n) g2[it * gs] = r[it];
 }
 
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(FFT_TPB, 2) y_fwd_seq_k(Fields3 fl, int n_, long long es,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) : GEN_MAXTPB, 2) y_fwd_seq_k(Fields3 fl, int n_, long long es,
                                                         long long ostride, int ncol, int B_,
                                                         KTab kt, const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
-  constexpr int BC = LN ? fft_pencils(1 << LN) : 1;
+  constexpr int BC = LN ? ct_cols(LN, FFT_CAP) : 1;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, FFT_V) : GEN_TPB;
+  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
   const int n = LN ? 1 << LN : n_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
@@ -1165,52 +1458,52 @@ __global__ void __launch_bounds__(FFT_TPB, 2) y_fwd_seq_k(Fields3 fl, int n_, lo
   const int c0 = bx * B;
   const int nb = ncol - c0 < B ? ncol - c0 : B;
   const long long off = (long long)by * ostride + c0;
-  stage_twiddles<FFT_TPB>(stw, tw, n);
-  const ColMap cm = col_map<FFT_TPB>(lB);
+  stage_twiddles<TPB>(stw, tw, n);
+  const ColMap cm = col_map<TPB>(lB);
   const bool live = cm.b < nb;
   const float kmz = live ? kt.km[2][c0 + cm.b] : 0.f;
   float2* g1 = fl.f[1] + off + cm.b + (long long)cm.j0 * es;
   const float2* g2 = fl.f[2] + off + cm.b + (long long)cm.j0 * es;
   const long long gs = (long long)cm.js * es;
-  float2 a[FFT_MAXV];
+  float2 a[MAXV];
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     a[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n) a[it] = g1[it * gs];
   }
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * FFT_TPB] = a[it];
+  for (int it = 0; it < MAXV; ++it)
+    if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * tpb<TPB>()] = a[it];
   __syncthreads();
-  fft_run<-1, COLS, POW2, LN, ilog2c(BC), FFT_MAXV, FFT_TPB>(s, n, B, stw);
+  fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
   {
-    float2 c[FFT_MAXV];
+    float2 c[MAXV];
 #pragma unroll
-    for (int it = 0; it < FFT_MAXV; ++it) {
+    for (int it = 0; it < MAXV; ++it) {
       c[it] = make_float2(0.f, 0.f);
       if (live && cm.j0 + it * cm.js < n) c[it] = g2[it * gs];
     }
 #pragma unroll
-    for (int it = 0; it < FFT_MAXV; ++it)
-      if (cm.j0 + it * cm.js < n) a[it] = s[threadIdx.x + it * FFT_TPB];
+    for (int it = 0; it < MAXV; ++it)
+      if (cm.j0 + it * cm.js < n) a[it] = s[threadIdx.x + it * tpb<TPB>()];
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < FFT_MAXV; ++it)
-      if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * FFT_TPB] = c[it];
+    for (int it = 0; it < MAXV; ++it)
+      if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * tpb<TPB>()] = c[it];
   }
   __syncthreads();
-  fft_run<-1, COLS, POW2, LN, ilog2c(BC), FFT_MAXV, FFT_TPB>(s, n, B, stw);
+  fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it) {
+  for (int it = 0; it < MAXV; ++it) {
     const int j = cm.j0 + it * cm.js;
     if (j < n) {
-      const float2 c = s[threadIdx.x + it * FFT_TPB];
+      const float2 c = s[threadIdx.x + it * tpb<TPB>()];
       const float kmy = kt.km[1][j];
       a[it] = make_float2(kmy * a[it].x + kmz * c.x, kmy * a[it].y + kmz * c.y);
     }
   }
 #pragma unroll
-  for (int it = 0; it < FFT_MAXV; ++it)
+  for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n) g1[it * gs] = a[it];
 }
 
@@ -1246,30 +1539,67 @@ static size_t lds_bytes(int n, int P, int lay = COLS) {
 static size_t tw_bytes(int n) { return (size_t)n * sizeof(float2); }
 
 
-static bool half_ok(int n2) { return n2 >= 4 && (n2 & 1) == 0 && is_pow2(n2 / 2); }
-
-// rows per workgroup, LDS bytes and pencil length of the z pass of n2
-struct RowPlan {
-  bool half;
-  int P, len;
-  size_t lds;
-};
-
-static RowPlan row_plan(int n2) {
-  RowPlan r;
-  r.half = half_ok(n2);
-  r.len = r.half ? n2 / 2 : n2;
-  r.P = row_pencils(r.len);
-  r.lds = lds_bytes(r.len, r.P, ROWS) + tw_bytes(n2);
-  return r;
-}
-
 // log2 of a length that has compile-time kernel variants (64..1024), else 0
 static int ct_log2(int n) {
   if (!is_pow2(n) || n < 64 || n > 1024) return 0;
   int l = 0;
   while ((1 << l) < n) ++l;
   return l;
+}
+
+// Threads of a run-time-length workgroup of `total` values.
+static int gen_tpb(int total) {
+  const int t = (total + GEN_MAXV - 1) / GEN_MAXV;
+  return t < 64 ? 64 : (t + 63) / 64 * 64;
+}
+
+// Fewest workgroups of a pass before its blocks are made smaller: four per CU.
+#define FFT_MIN_WGS 1024
+
+// The z pass of n2 over nrows rows: even n2 as half-length transforms, of
+// compile-time length 2^lh when that is 64..1024 and the row blocks come out
+// even, else (and for odd n2, two rows a pencil) at run time.  rows: rows per
+// workgroup.  Meshes of few rows take smaller blocks (sm): a 128^3 mesh has
+// 256 row blocks of 4096 values, one per CU, and their load, barrier and
+// store phases then follow each other with nothing to overlap.
+struct RowPlan {
+  bool half, sm;
+  int lh, P, len, rows, tpb;
+  size_t lds;
+};
+
+static RowPlan row_plan(int n2, long long nrows) {
+  RowPlan r;
+  r.half = n2 >= 4 && (n2 & 1) == 0;
+  r.len = r.half ? n2 / 2 : n2;
+  r.lh = r.half ? ct_log2(r.len) : 0;
+  r.sm = false;
+  if (r.lh) {
+    r.sm = nrows / ct_rows(r.lh, false) < FFT_MIN_WGS;
+    r.P = ct_rows(r.lh, r.sm);
+    r.tpb = ct_row_tpb(r.lh, r.sm);
+    if (nrows % r.P) r.lh = 0;
+  }
+  if (!r.lh) {
+    r.P = 1;
+    while (2 * r.P * r.len <= GEN_CAP / 2) r.P *= 2;
+    const int per = r.half ? 1 : 2;
+    while (r.P > 1 && r.P * r.len > GEN_CAP / 8 && nrows / (per * r.P) < FFT_MIN_WGS) r.P /= 2;
+  }
+  if (!r.lh) r.tpb = gen_tpb(r.P * r.len);
+  r.rows = r.half ? r.P : 2 * r.P;
+  r.lds = lds_bytes(r.len, r.P, ROWS) + tw_bytes(n2);
+  return r;
+}
+
+// Columns per workgroup of a strided pass of length n without compile-time
+// variants: 16 (128-byte segments), fewer when they exceed GEN_CAP values or
+// would leave CUs idle.
+static int gen_cols(int n, int ncol, long long nouter) {
+  int B = 16;
+  while (B > 1 && B * n > GEN_CAP) B /= 2;
+  while (B > 4 && B * n > GEN_CAP / 4 && (ncol + B - 1) / B * nouter < FFT_MIN_WGS / 2) B /= 2;
+  return B;
 }
 
 // CALL(L) with L the compile-time constant for ln (0: generic kernels)
@@ -1290,79 +1620,114 @@ int pmx_fold_deferrable(const pmx_ctx* c) {
   const TileGeom& t = c->tg;
   if (t.tx != 16 || t.ty != 16 || t.tz != 16) return 0;
   if (c->n[0] % 16 || c->n[1] % 16 || c->n[2] % 16) return 0;
-  const RowPlan r = row_plan(c->n[2]);
-  return r.half && ct_log2(r.len) > 0 && c->n[1] % r.P == 0;
+  const RowPlan r = row_plan(c->n[2], (long long)c->n[0] * c->n[1]);
+  return r.lh > 0 && c->n[1] % r.P == 0;
 }
 
-// In-place r2c of a padded real mesh; pre applies (x - 1) * coef.  With
-// halo (one channel's shells; pmx_fold_deferrable must hold) the deposit's
-// fold is added on load.
-int pmx_fft_r2c_inplace(pmx_ctx* c, float* buf, int pre, float coef, const float* halo, int rev) {
+static RowFields row_fields(float* const* f, int nf, const int* rev, unsigned nblk, long long hstride) {
+  RowFields rf;
+  for (int i = 0; i < 3; ++i) {
+    rf.f[i] = f[i < nf ? i : 0];
+    rf.rev[i] = rev[i < nf ? i : 0];
+  }
+  rf.nblk = nblk;
+  rf.hstride = hstride;
+  return rf;
+}
+
+// In-place r2c of nf padded real meshes; pre applies (x - 1) * coef.  With
+// halo (pmx_fold_deferrable must hold; one channel's shells per mesh) the
+// deposit's fold is added on load.
+int pmx_fft_r2c_inplace(pmx_ctx* c, float* const* f, int nf, int pre, float coef, const float* halo,
+                        const int* rev) {
   const long long nrows = (long long)c->n[0] * c->n[1];
   const int n2 = c->n[2];
-  const RowPlan r = row_plan(n2);
-  if (int rc = fft_fits("z r2c", n2, r.len * r.P, RFFT_CAP, r.lds)) return rc;
-  const unsigned nblk = (unsigned)((nrows + r.P - 1) / r.P);
-  const int P = r.P;
-  const size_t lds = r.lds;
+  const RowPlan r = row_plan(n2, nrows);
+  if (int rc = fft_fits("z r2c", n2, r.len * r.P, GEN_CAP, r.lds)) return rc;
+  const unsigned nblk = (unsigned)((nrows + r.rows - 1) / r.rows);
   const FoldIn fi = {halo, c->tg.shell, c->tg.ntx, c->tg.nty, c->tg.ntz, c->n[1]};
+  const RowFields rf = row_fields(f, nf, rev, nblk, c->ntiles * c->tg.shell);
   const float* fc = pre ? c->dfac : nullptr;
   PMX_REQUIRE(!halo || pmx_fold_deferrable(c), "z r2c: no fold on load for this mesh");
   pmx_tic(c, PMX_T_ZR2C);
-  if (r.half) {
-    const int lh = nrows % P == 0 ? ct_log2(r.len) : 0;
-#define R2C_HALF(L)                                                                                \
-  if (halo && pre)                                                                                 \
-    z_r2c_half_k<1, L, (L > 0)><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, coef,  \
-                                                                  c->tw[2], fi, fc, rev);              \
-  else if (halo)                                                                                   \
-    z_r2c_half_k<0, L, (L > 0)><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, coef,  \
-                                                                  c->tw[2], fi, fc, rev);              \
-  else if (pre)                                                                                    \
-    z_r2c_half_k<1, L><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, coef, c->tw[2], fi, fc, rev); \
-  else                                                                                             \
-    z_r2c_half_k<0, L><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, coef, c->tw[2], fi, fc, rev)
-    PMX_CT_SWITCH(lh, R2C_HALF);
-#undef R2C_HALF
+  const unsigned grid = nblk * (unsigned)nf;
+#define R2C(PRE, L, SM, FOLD, P2)                                                        \
+  z_r2c_half_k<PRE, L, SM, FOLD, P2><<<grid, r.tpb, r.lds, c->stream>>>(                 \
+      rf, nrows, n2, c->rs, r.P, coef, c->tw[2], fi, fc)
+#define R2C_SM(L, SM)                                   \
+  do {                                                  \
+    if (halo && pre) R2C(1, L, SM, (L > 0), true);      \
+    else if (halo) R2C(0, L, SM, (L > 0), true);        \
+    else if (pre) R2C(1, L, SM, false, true);           \
+    else R2C(0, L, SM, false, true);                    \
+  } while (0)
+#define R2C_HALF(L)                       \
+  if (r.sm && L) R2C_SM(L, (L > 0));      \
+  else R2C_SM(L, false)
+#define R2C_FULL(PRE, P2)                                                              \
+  z_r2c_k<PRE, P2><<<grid, r.tpb, r.lds, c->stream>>>(rf, nrows, n2, c->rs, r.P, coef, c->tw[2], fc)
+  if (r.half && is_pow2(r.len)) {
+    PMX_CT_SWITCH(r.lh, R2C_HALF);
+  } else if (r.half) {
+    if (pre) R2C(1, 0, false, false, false);
+    else R2C(0, 0, false, false, false);
+  } else if (is_pow2(n2)) {
+    if (pre) R2C_FULL(1, true);
+    else R2C_FULL(0, true);
   } else {
-    const bool p2 = is_pow2(n2);
-    if (pre && p2)
-      z_r2c_k<1, true><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, coef, c->tw[2], fc);
-    else if (pre)
-      z_r2c_k<1, false><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, coef, c->tw[2], fc);
-    else if (p2)
-      z_r2c_k<0, true><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, coef, c->tw[2], fc);
-    else
-      z_r2c_k<0, false><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, coef, c->tw[2], fc);
+    if (pre) R2C_FULL(1, false);
+    else R2C_FULL(0, false);
   }
+#undef R2C_FULL
+#undef R2C_HALF
+#undef R2C_SM
+#undef R2C
   pmx_toc(c, PMX_T_ZR2C);
   PMX_LAUNCH_CHECK();
   return PMX_OK;
 }
 
-int pmx_fft_c2r_inplace(pmx_ctx* c, float* buf, float scale, int rev) {
+// In-place c2r of nf padded meshes with a final scale.
+int pmx_fft_c2r_inplace(pmx_ctx* c, float* const* f, int nf, float scale, const int* rev) {
   const long long nrows = (long long)c->n[0] * c->n[1];
   const int n2 = c->n[2];
-  const RowPlan r = row_plan(n2);
-  if (int rc = fft_fits("z c2r", n2, r.len * r.P, RFFT_CAP, r.lds)) return rc;
-  const unsigned nblk = (unsigned)((nrows + r.P - 1) / r.P);
-  const int P = r.P;
-  const size_t lds = r.lds;
+  const RowPlan r = row_plan(n2, nrows);
+  if (int rc = fft_fits("z c2r", n2, r.len * r.P, GEN_CAP, r.lds)) return rc;
+  const unsigned nblk = (unsigned)((nrows + r.rows - 1) / r.rows);
+  const RowFields rf = row_fields(f, nf, rev, nblk, 0);
+  const unsigned grid = nblk * (unsigned)nf;
   pmx_tic(c, PMX_T_ZC2R);
-  if (r.half) {
-    const int lh = nrows % P == 0 ? ct_log2(r.len) : 0;
-#define C2R_HALF(L) \
-  z_c2r_half_k<L><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, scale, c->tw[2], rev)
-    PMX_CT_SWITCH(lh, C2R_HALF);
-#undef C2R_HALF
+#define C2R(L, SM, P2)                                                                         \
+  z_c2r_half_k<L, SM, P2><<<grid, r.tpb, r.lds, c->stream>>>(rf, nrows, n2, c->rs, r.P, scale, \
+                                                             c->tw[2])
+#define C2R_HALF(L)                    \
+  if (r.sm && L) C2R(L, (L > 0), true); \
+  else C2R(L, false, true)
+#define C2R_FULL(P2) \
+  z_c2r_k<P2><<<grid, r.tpb, r.lds, c->stream>>>(rf, nrows, n2, c->rs, r.P, scale, c->tw[2])
+  if (r.half && is_pow2(r.len)) {
+    PMX_CT_SWITCH(r.lh, C2R_HALF);
+  } else if (r.half) {
+    C2R(0, false, false);
   } else if (is_pow2(n2)) {
-    z_c2r_k<true><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, scale, c->tw[2]);
+    C2R_FULL(true);
   } else {
-    z_c2r_k<false><<<nblk, FFT_TPB, lds, c->stream>>>(buf, nrows, n2, c->rs, P, scale, c->tw[2]);
+    C2R_FULL(false);
   }
+#undef C2R_FULL
+#undef C2R_HALF
+#undef C2R
   pmx_toc(c, PMX_T_ZC2R);
   PMX_LAUNCH_CHECK();
   return PMX_OK;
+}
+
+// One mesh.
+int pmx_fft_r2c_inplace(pmx_ctx* c, float* buf, int pre, float coef, const float* halo, int rev) {
+  return pmx_fft_r2c_inplace(c, &buf, 1, pre, coef, halo, &rev);
+}
+int pmx_fft_c2r_inplace(pmx_ctx* c, float* buf, float scale, int rev) {
+  return pmx_fft_c2r_inplace(c, &buf, 1, scale, &rev);
 }
 
 // axis 1 (y) or axis 0 (x) complex FFT of nf fields in place
@@ -1370,9 +1735,8 @@ int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int
   Fields3 fl;
   for (int i = 0; i < 3; ++i) fl.f[i] = f[i < nf ? i : 0];
   fl.rev = rev;
-  int n = c->n[axis];
-  int B = fft_pencils(n);
-  int ncol = c->n2h;
+  const int n = c->n[axis];
+  const int ncol = c->n2h;
   long long es, ostride;
   unsigned nouter;
   if (axis == 1) {
@@ -1384,22 +1748,24 @@ int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int
     ostride = c->n2p;
     nouter = c->n[1];
   }
+  const int ln = ct_log2(n);
+  const int B = ln ? ct_cols(ln, FFT_CAP) : gen_cols(n, ncol, (long long)nouter * nf);
+  const int tpb = ln ? ct_tpb(ln, B, FFT_V) : gen_tpb(n * B);
   dim3 grid((ncol + B - 1) / B, nouter, nf);
   size_t lds = lds_bytes(n, B) + tw_bytes(n);
-  if (int rc = fft_fits("strided FFT", n, n * B, FFT_CAP, lds)) return rc;
+  if (int rc = fft_fits("strided FFT", n, n * B, ln ? FFT_CAP : GEN_CAP, lds)) return rc;
   const bool p2 = is_pow2(n);
-  const int ln = ct_log2(n);
   const int cls = axis == 1 ? (dir < 0 ? PMX_T_YFWD : PMX_T_YINV) : PMX_T_OTHER;
   pmx_tic(c, cls);
 #define STRIDED(L)                                                                                  \
   if (dir < 0 && (L || p2))                                                                         \
-    strided_fft_k<-1, true, L><<<grid, FFT_TPB, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]); \
+    strided_fft_k<-1, true, L><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]); \
   else if (dir < 0)                                                                                 \
-    strided_fft_k<-1, false, 0><<<grid, FFT_TPB, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]); \
+    strided_fft_k<-1, false, 0><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]); \
   else if (L || p2)                                                                                 \
-    strided_fft_k<1, true, L><<<grid, FFT_TPB, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]);  \
+    strided_fft_k<1, true, L><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]);  \
   else                                                                                              \
-    strided_fft_k<1, false, 0><<<grid, FFT_TPB, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis])
+    strided_fft_k<1, false, 0><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis])
   PMX_CT_SWITCH(ln, STRIDED);
 #undef STRIDED
   pmx_toc(c, cls);
@@ -1423,26 +1789,27 @@ static KTab ktab(const pmx_ctx* c) {
 int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev) {
   Fields3 fl = {{f[0], f[1], f[2]}, rev};
   const int n = c->n[1];
-  const int B = fft_pencils(n);
   const int ncol = c->n2h;
+  const int ln = ct_log2(n);
+  const int B = ln ? ct_cols(ln, FFT_CAP) : gen_cols(n, ncol, c->n[0]);
+  const int tpb = ln ? ct_tpb(ln, B, FFT_V) : gen_tpb(n * B);
   const long long es = c->n2p, ostride = (long long)n * c->n2p;
   dim3 grid((ncol + B - 1) / B, c->n[0], 1);
   const size_t lds = lds_bytes(n, B) + tw_bytes(n);
-  if (int rc = fft_fits("paired y FFT", n, n * B, FFT_CAP, lds)) return rc;
+  if (int rc = fft_fits("paired y FFT", n, n * B, ln ? FFT_CAP : GEN_CAP, lds)) return rc;
   const KTab kt = ktab(c);
   const bool p2 = is_pow2(n);
-  const int ln = ct_log2(n);
   const int cls = dir < 0 ? PMX_T_YFWD : PMX_T_YINV;
   pmx_tic(c, cls);
 #define YPAIR(L)                                                                                  \
   if (dir < 0 && (L || p2))                                                                       \
-    y_fwd_seq_k<true, L><<<grid, FFT_TPB, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
+    y_fwd_seq_k<true, L><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
   else if (dir < 0)                                                                               \
-    y_fwd_seq_k<false, 0><<<grid, FFT_TPB, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
+    y_fwd_seq_k<false, 0><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
   else if (L || p2)                                                                               \
-    y_inv_seq_k<true, L><<<grid, FFT_TPB, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
+    y_inv_seq_k<true, L><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
   else                                                                                            \
-    y_inv_seq_k<false, 0><<<grid, FFT_TPB, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1])
+    y_inv_seq_k<false, 0><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1])
   PMX_CT_SWITCH(ln, YPAIR);
 #undef YPAIR
   pmx_toc(c, cls);
@@ -1453,28 +1820,29 @@ int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev) {
 int pmx_poisson_x(pmx_ctx* c, float2* const* f, int adjoint, int kin, int rev) {
   Fields3 fl = {{f[0], f[1], f[2]}, rev};
   const int n0 = c->n[0];
-  const int B = fft_pencils(n0, PFFT_CAP);
+  const int ln = ct_log2(n0);
+  const int B = ln ? ct_cols(ln, PFFT_CAP) : gen_cols(n0, c->n2h, c->n[1]);
+  const int tpb = ln ? ct_tpb(ln, B, PFFT_V) : gen_tpb(n0 * B);
   dim3 grid((c->n2h + B - 1) / B, c->n[1], 1);
   // the data block, the twiddles, then the k_0 and km_0 tables
   size_t lds = lds_bytes(n0, B) + tw_bytes(n0) + 2 * (size_t)n0 * sizeof(float);
   if (int rc = fft_fits("Poisson x pass", n0, n0 * B, PFFT_CAP, lds)) return rc;
   const bool p2 = is_pow2(n0);
-  const int ln = ct_log2(n0);
   const KTab kt = ktab(c);
   pmx_tic(c, PMX_T_POISSON);
 #define PX(L)                                                                                             \
   if (adjoint && (L || p2))                                                                               \
-    poisson_x_adj_k<true, L><<<grid, PFFT_TPB, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
+    poisson_x_adj_k<true, L><<<grid, tpb, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
   else if (adjoint)                                                                                       \
-    poisson_x_adj_k<false, 0><<<grid, PFFT_TPB, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
+    poisson_x_adj_k<false, 0><<<grid, tpb, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
   else if ((L || p2) && kin)                                                                              \
-    poisson_x_k<true, L, true><<<grid, PFFT_TPB, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
+    poisson_x_k<true, L, true><<<grid, tpb, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
   else if (kin)                                                                                           \
-    poisson_x_k<false, 0, true><<<grid, PFFT_TPB, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
+    poisson_x_k<false, 0, true><<<grid, tpb, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
   else if (L || p2)                                                                                       \
-    poisson_x_k<true, L><<<grid, PFFT_TPB, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
+    poisson_x_k<true, L><<<grid, tpb, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0]); \
   else                                                                                                    \
-    poisson_x_k<false, 0><<<grid, PFFT_TPB, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0])
+    poisson_x_k<false, 0><<<grid, tpb, lds, c->stream>>>(fl, n0, c->n[1], c->n2h, c->n2p, B, kt, c->tw[0])
   PMX_CT_SWITCH(ln, PX);
 #undef PX
   pmx_toc(c, PMX_T_POISSON);
@@ -1499,10 +1867,9 @@ int pmx_poisson_ctx(pmx_ctx* c, float coef, int deferred) {
   if ((rc = pmx_fft_strided(c, f, 1, 1, 1, 0))) return rc;
   if ((rc = pmx_fft_ypair(c, f, 1, 1))) return rc;
   float scale = (float)(1.0 / (double)c->M);
-  if ((rc = pmx_fft_c2r_inplace(c, (float*)f[1], scale, 0))) return rc;
-  if ((rc = pmx_fft_c2r_inplace(c, (float*)f[2], scale, 1))) return rc;
-  if ((rc = pmx_fft_c2r_inplace(c, (float*)f[0], scale, 1))) return rc;
-  return PMX_OK;
+  float* z[3] = {(float*)f[1], (float*)f[2], (float*)f[0]};
+  const int rev[3] = {0, 1, 1};
+  return pmx_fft_c2r_inplace(c, z, 3, scale, rev);
 }
 
 // Adjoint Poisson on the context buffers: cbuf[0..2] hold the three
@@ -1518,12 +1885,10 @@ int pmx_poisson_adj_ctx(pmx_ctx* c, float scale_out, int deferred) {
 int pmx_poisson_adj_bufs(pmx_ctx* c, float2* const* f, float scale_out, int deferred) {
   int rc;
   const bool fold = deferred && pmx_fold_deferrable(c);
-  const long long hstride = c->ntiles * c->tg.shell;
   // block directions alternate as in pmx_poisson_ctx
-  for (int d = 0; d < 3; ++d)
-    if ((rc = pmx_fft_r2c_inplace(c, (float*)f[d], 0, 0.f, fold ? c->halo + d * hstride : nullptr,
-                                  1)))
-      return rc;
+  float* z[3] = {(float*)f[0], (float*)f[1], (float*)f[2]};
+  const int rev[3] = {1, 1, 1};
+  if ((rc = pmx_fft_r2c_inplace(c, z, 3, 0, 0.f, fold ? c->halo : nullptr, rev))) return rc;
   if ((rc = pmx_fft_strided(c, f, 1, 1, -1, 0))) return rc;
   if ((rc = pmx_fft_ypair(c, f, -1, 0))) return rc;
   if ((rc = pmx_poisson_x(c, f, 1, 0, 1))) return rc;

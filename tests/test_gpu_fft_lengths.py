@@ -1,0 +1,67 @@
+"""The real FFT and the Poisson solve over the lengths their stages split on:
+each radix and prime stage, odd rows (two a pencil, an odd row left over),
+half-length rows of any length, small and large row and column blocks."""
+import numpy as np
+import pytest
+import scipy.fft as sfft
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# every radix in each axis: 6, 9, 10; 2 x 7, 15, 2 x 9; primes 11, 13, 17, 19,
+# 31, 127; prime squares; 8 x 3 and 3 x 2^k meshes; 180 = 4 9 5, 210 = 6 5 7;
+# fixed lengths 32 and up in small and large row blocks; a single row pair
+SHAPES = [(6, 9, 10), (14, 15, 18), (11, 26, 13), (17, 34, 51), (19, 62, 127), (49, 121, 25),
+          (24, 96, 48), (150, 45, 30), (20, 180, 210), (32, 32, 64), (33, 32, 64), (3, 5, 64),
+          (8, 512, 128), (96, 192, 66), (1, 3, 375), (1, 1, 9), (5, 1, 2), (2, 2, 4095)]
+
+
+def _rel(a, b):
+    return np.linalg.norm(np.asarray(a, np.complex128) - b) / np.linalg.norm(b)
+
+
+# a stage of radix r rounds each output about sqrt(r) times at 2^-24; over
+# the stages of three axes here that stays below 1e-6, twice that is allowed
+TOL = 2e-6
+
+
+@pytest.mark.parametrize('shape', SHAPES)
+def test_transforms_match_float64(dev, shape):
+    from pmwd_amd.pm_util import fftfwd, fftinv
+    x = np.random.default_rng(5).standard_normal(shape).astype(np.float32)
+    want = sfft.rfftn(x.astype(np.float64))
+    assert _rel(fftfwd(torch.as_tensor(x, device=dev)).cpu().numpy(), want) < TOL
+    spec = want.astype(np.complex64)
+    # imaginary parts of the self-conjugate planes are dropped, as irfftn does
+    spec[..., 0] += 0.5j
+    if shape[2] % 2 == 0:
+        spec[..., -1] += 0.25j
+    back = fftinv(torch.as_tensor(spec, device=dev), shape=shape).cpu().numpy()
+    assert _rel(back, sfft.irfftn(spec.astype(np.complex128), s=shape)) < TOL
+
+
+@pytest.mark.parametrize('shape', [(14, 15, 18), (11, 26, 13), (24, 96, 48), (15, 20, 25),
+                                   (32, 64, 64), (20, 180, 42)])
+def test_poisson_and_its_adjoint(dev, shape):
+    """The solve against a float64 one, and its adjoint by the inner product."""
+    from pmwd_amd import _lib
+    from oracle import pm as opm
+    rng = np.random.default_rng(6)
+    dens = (1 + 0.3 * rng.standard_normal(shape)).astype(np.float32)
+    cot = rng.standard_normal((3,) + shape).astype(np.float32)
+    coef = float(np.float32(1.5) * np.float32(0.3))
+    c = _lib.context(shape, 1.5, dev)
+    to = lambda a: torch.as_tensor(a, device=dev)
+    grad, back = to(np.empty_like(cot)), to(np.empty_like(dens))
+    d, g = to(dens), to(cot)
+    _lib.check(_lib.lib().pmx_poisson_grad(c.bind(), _lib.ptr(d), coef, _lib.ptr(grad)))
+    _lib.check(_lib.lib().pmx_poisson_grad_adj(c.bind(), _lib.ptr(g), coef, _lib.ptr(back)))
+    want = opm.gravity_mesh(dens, 0.3, 1.5, shape)
+    for a in range(3):
+        assert _rel(grad[a].cpu().numpy(), np.asarray(want[a], np.complex128)) < 5e-6
+    # <cot, G (dens - 1)> = <G^T cot, dens - 1>; each side a sum over the mesh
+    # of terms rounded at 1e-6
+    lhs = float((g.double() * grad.double()).sum())
+    rhs = float((back.double() * (d.double() - 1)).sum())
+    scale = float((g.double() * grad.double()).abs().sum())
+    assert abs(lhs - rhs) < 5e-6 * scale
