@@ -2,7 +2,9 @@
 // offsets, a different output cell size (enmesh's a2 branch, computed in
 // float64 as the reference does), target shapes with dropped indices,
 // channels and 1-3 spatial dimensions.  Not the hot path: global float
-// atomics are used for the scatter-type outputs.
+// atomics are used for the scatter-type outputs.  The entry points hand the
+// default geometry with up to three channels to the kernels of
+// pmx_values.hip, which do the same float operations.
 #include "pmx_internal.h"
 
 #include <math.h>
@@ -322,6 +324,8 @@ extern "C" int pmx_scatter_cic(pmx_ctx* c, const pmx_cic_geom* g, const int16_t*
   if (rc) return rc;
   if (n == 0) return PMX_OK;
   PMX_REQUIRE(pmid && disp, "pmx_scatter_cic: NULL particle arrays");
+  if (pmx_values_fit(c, g, nchan) && pmx_values_scatter_ready(c, n))
+    return pmx_values_scatter(c, pmid, disp, n, val, val_scalar, nchan, mesh);
   gen_scatter_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(G, pmid, disp, n, val, val_scalar, nchan,
                                                           mesh);
   PMX_LAUNCH_CHECK();
@@ -338,6 +342,8 @@ extern "C" int pmx_gather_cic(pmx_ctx* c, const pmx_cic_geom* g, const int16_t* 
   if (rc) return rc;
   if (n == 0) return PMX_OK;
   PMX_REQUIRE(pmid && disp && mesh && out, "pmx_gather_cic: NULL pointer");
+  if (pmx_values_fit(c, g, nchan))
+    return pmx_values_gather(c, pmid, disp, n, mesh, nchan, val, val_scalar, out);
   gen_gather_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(G, pmid, disp, n, mesh, nchan, val,
                                                          val_scalar, out);
   PMX_LAUNCH_CHECK();
@@ -355,6 +361,8 @@ extern "C" int pmx_scatter_cic_adj(pmx_ctx* c, const pmx_cic_geom* g, const int1
   if (rc) return rc;
   if (n == 0) return PMX_OK;
   PMX_REQUIRE(pmid && disp && mesh_cot, "pmx_scatter_cic_adj: NULL pointer");
+  if (pmx_values_fit(c, g, nchan))
+    return pmx_values_adj(c, pmid, disp, n, mesh_cot, nchan, val, val_scalar, disp_cot, val_cot);
   gen_scatter_adj_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(G, pmid, disp, n, mesh_cot, val,
                                                               val_scalar, nchan, disp_cot, val_cot);
   PMX_LAUNCH_CHECK();
@@ -372,6 +380,14 @@ extern "C" int pmx_gather_cic_adj(pmx_ctx* c, const pmx_cic_geom* g, const int16
   if (rc) return rc;
   if (n == 0) return PMX_OK;
   PMX_REQUIRE(pmid && disp && mesh && val_cot, "pmx_gather_cic_adj: NULL pointer");
+  if (pmx_values_fit(c, g, nchan)) {
+    if (disp_cot && (rc = pmx_values_adj(c, pmid, disp, n, mesh, nchan, val_cot, 0.f, disp_cot, nullptr)))
+      return rc;
+    disp_cot = nullptr;
+    if (!mesh_cot) return PMX_OK;
+    if (pmx_values_scatter_ready(c, n))
+      return pmx_values_scatter(c, pmid, disp, n, val_cot, 0.f, nchan, mesh_cot);
+  }
   gen_gather_adj_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(G, pmid, disp, n, mesh, val_cot, nchan,
                                                              disp_cot, mesh_cot);
   PMX_LAUNCH_CHECK();

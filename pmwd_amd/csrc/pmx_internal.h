@@ -951,6 +951,15 @@ int pmx_kd_adj_bin(pmx_ctx* c, const int16_t* pmid, float* disp, float* vel, con
                    int cap, double* part);
 int pmx_deposit_binned3(pmx_ctx* c, long long n, float* const* mesh, int mrs, int defer = 0);
 int pmx_ensure_halo(pmx_ctx* c, int nch);
+// default-geometry CIC of one to three value channels (pmx_values.hip)
+bool pmx_values_fit(const pmx_ctx* c, const pmx_cic_geom* g, int nchan);
+bool pmx_values_scatter_ready(pmx_ctx* c, long long n);
+int pmx_values_gather(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
+                      const float* mesh, int nchan, const float* val, float vs, float* out);
+int pmx_values_adj(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n, const float* f,
+                   int nchan, const float* val, float vs, float* disp_cot, float* val_cot);
+int pmx_values_scatter(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
+                       const float* val, float vs, int nchan, float* mesh);
 int pmx_poisson_ctx(pmx_ctx* c, float coef, int deferred = 0);
 // FFT passes on meshes in the context's padded layout (pmx_fft.hip):
 // in-place z r2c (pre: (x - 1) * coef on load; halo: the deposit's fold

@@ -23,18 +23,25 @@ class _ScatterFn(torch.autograd.Function):
         L = _lib.lib()
         dim = conf.dim
         n = pmid.shape[0]
-        chan = tuple(mesh.shape[dim:])
+        fresh = mesh is None   # zeros of the mesh shape
+        chan = tuple(val.shape[1:]) if fresh and val is not None else ()
+        shape = tuple(conf.mesh_shape) + chan if fresh else tuple(mesh.shape)
+        sshape, chan = shape[:dim], shape[dim:]
         nchan = int(np.prod(chan)) if chan else 1
-        sshape = tuple(mesh.shape[:dim])
-        out = mesh.detach().clone().contiguous()
         disp_c = disp.detach().contiguous()
         val_c = val.detach().contiguous() if val is not None else None
         # the backward uses this context too: autograd may run it on another
         # thread, where context() would not see the caller's context provider
         c = _lib.context(conf.mesh_shape, conf.cell_size, disp.device)
-        if val_c is None and nchan == 1 and is_default_cic(conf, sshape, offset, cell_size):
+        mass = val_c is None and nchan == 1 and is_default_cic(conf, sshape, offset, cell_size)
+        if not fresh:
+            out = mesh.detach().clone().contiguous()
+        else:   # the mass scatter writes every cell
+            make = torch.empty if mass else torch.zeros
+            out = make(shape, dtype=conf.float_dtype, device=disp.device)
+        if mass:
             _lib.check(L.pmx_scatter_mass(c.bind(), _lib.ptr(pmid), _lib.ptr(disp_c), n,
-                                          float(val_scalar), _lib.ptr(out), 1))
+                                          float(val_scalar), _lib.ptr(out), int(not fresh)))
         else:
             g = cic_geom(conf, sshape, offset, cell_size)
             _lib.check(L.pmx_scatter_cic(c.bind(), g, _lib.ptr(pmid), _lib.ptr(disp_c), n,
@@ -86,11 +93,9 @@ def scatter(ptcl, conf, mesh=None, val=None, offset=0, cell_size=None):
     else:
         val_scalar = float(val)
     chan = tuple(val_t.shape[1:]) if val_t is not None else ()
-    if mesh is None:
-        mesh = torch.zeros(tuple(conf.mesh_shape) + chan, dtype=conf.float_dtype, device=dev)
-    else:
+    if mesh is not None:
         mesh = torch.as_tensor(mesh).to(device=dev, dtype=conf.float_dtype)
-    if tuple(mesh.shape[conf.dim:]) != chan:
-        raise ValueError(f'channel shape mismatch: {tuple(mesh.shape[conf.dim:])} != {chan}')
+        if tuple(mesh.shape[conf.dim:]) != chan:
+            raise ValueError(f'channel shape mismatch: {tuple(mesh.shape[conf.dim:])} != {chan}')
     return _ScatterFn.apply(disp, mesh, val_t, pmid.contiguous(), conf, offset, cell_size,
                             val_scalar)
