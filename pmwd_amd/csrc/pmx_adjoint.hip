@@ -296,66 +296,68 @@ extern "C" int pmx_drift_adj(pmx_ctx* c, long long n, float* disp, const float* 
 // (disp replaced by snap when given, a stored checkpoint), with per-block
 // partials of disp_cot.vel (the drift's cosmology term).  A kick's own
 // vel_cot.acc equals the dot of the force VJP that produced acc.
+// One particle a thread, one global atomic per tile and workgroup (TileTable).
 template <int HAS_KP, bool CAP>
-__global__ void __launch_bounds__(PMX_TPB)
+__global__ void __launch_bounds__(KD_ADJ_TPB)
     kd_adj_bin_k(const int16_t* __restrict__ pmid, float* __restrict__ disp, float* __restrict__ vel,
                  const float* __restrict__ acc, float* __restrict__ disp_cot,
                  float* __restrict__ vel_cot, const float* __restrict__ acc_cot,
                  const float* __restrict__ snap, long long n, float kp, float ka, float d,
                  MeshGeom g, TileGeom tg, uint32_t* __restrict__ tile_count, BinOut o,
                  double* __restrict__ part, int keep_x) {
-  constexpr int T3 = 3 * PMX_TPB;
-  // vel | acc | disp | disp_cot | vel_cot | acc_cot, staged through LDS
-  __shared__ __align__(16) float sh[6 * T3];
-  __shared__ __align__(16) int16_t sp[T3];
-  const long long b0 = (long long)blockIdx.x * PMX_TPB;
-  const int cnt = (int)(n - b0 < PMX_TPB ? n - b0 : PMX_TPB);
-  pmx_stage_in3<6, PMX_TPB>(sh, {{vel, acc, disp, disp_cot, vel_cot, acc_cot}}, b0, cnt);
-  pmx_stage_pmid<PMX_TPB>(sp, pmid, b0, cnt);
-  __syncthreads();
-  const int q = threadIdx.x;
-  const bool active = q < cnt;
-  double s = 0;
-  uint32_t t = 0;
-  CicAxis ax[3];
-  float dp[3];
+  constexpr int TPB = KD_ADJ_TPB;
+  __shared__ TileTable<2 * TPB> T;
+  tt_clear<2 * TPB, TPB>(T);
+  const long long i = (long long)blockIdx.x * TPB + threadIdx.x;
+  const bool active = i < n;
+  int pm[3];
+  float x[3], v[3], dc[3], vc[3], ac[3], at[3], sn[3];
   if (active) {
-    int pm[3];
+    load_ptcl(pmid, disp, i, pm, x);
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const int e = 3 * q + a;
-      pm[a] = sp[e];
-      const float ac = sh[T3 + e], acot = sh[5 * T3 + e];
-      float v = sh[e];
-      float dc = sh[3 * T3 + e];
-      if (HAS_KP) {
-        v = v + ac * kp;
-        dc = dc - acot * kp;
-      }
-      v = v + ac * ka;
-      dc = dc - acot * ka;
-      float x = sh[2 * T3 + e];
-      // keep_x: disp already holds the stored state the drift would be replaced by
-      if (!keep_x) x = x + v * d;
-      float vc = sh[4 * T3 + e];
-      vc = vc - dc * d;
-      s += (double)dc * v;
-      if (snap) x = snap[3 * (b0 + q) + a];
-      sh[e] = v;
-      sh[2 * T3 + e] = x;
-      sh[3 * T3 + e] = dc;
-      sh[4 * T3 + e] = vc;
-      dp[a] = x;
+      v[a] = vel[3 * i + a];
+      ac[a] = acc[3 * i + a];
+      dc[a] = disp_cot[3 * i + a];
+      vc[a] = vel_cot[3 * i + a];
+      at[a] = acc_cot[3 * i + a];
+      if (snap) sn[a] = snap[3 * i + a];
     }
-    cic_setup(pm, dp, g, ax);
-    t = tile_of(ax, tg);
   }
-  const uint32_t r = agg_slot(tile_count, t, active);
-  if (active) pmx_bin_emit<CAP>(o, b0 + q, t, r, ax, tg);
   __syncthreads();
-  pmx_stage_out3<1, PMX_TPB>({{vel}}, sh, b0, cnt);
-  pmx_stage_out3<3, PMX_TPB>({{disp, disp_cot, vel_cot}}, sh + 2 * T3, b0, cnt);
-  block_sum_store<PMX_TPB>(s, part);
+  double s = 0;
+  uint32_t t = 0, rank = 0;
+  int slot = -1;
+  CicAxis ax[3];
+  if (active) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      if (HAS_KP) {
+        v[a] = v[a] + ac[a] * kp;
+        dc[a] = dc[a] - at[a] * kp;
+      }
+      v[a] = v[a] + ac[a] * ka;
+      dc[a] = dc[a] - at[a] * ka;
+      // keep_x: disp already holds the stored state the drift would be replaced by
+      if (!keep_x) x[a] = x[a] + v[a] * d;
+      vc[a] = vc[a] - dc[a] * d;
+      s += (double)dc[a] * v[a];
+      if (snap) x[a] = sn[a];
+      vel[3 * i + a] = v[a];
+      disp[3 * i + a] = x[a];
+      disp_cot[3 * i + a] = dc[a];
+      vel_cot[3 * i + a] = vc[a];
+    }
+    cic_setup(pm, x, g, ax);
+    t = tile_of(ax, tg);
+    slot = tt_count<2 * TPB>(T, t, rank);
+    if (slot < 0) rank = atomicAdd(&tile_count[t], 1u);
+  }
+  __syncthreads();
+  tt_reserve<2 * TPB, TPB, true>(T, tile_count);
+  __syncthreads();
+  if (active) pmx_bin_emit<CAP>(o, i, t, rank + (slot < 0 ? 0u : T.base[slot]), ax, tg);
+  block_sum_store<TPB>(s, part);
 }
 
 int pmx_kd_adj_bin(pmx_ctx* c, const int16_t* pmid, float* disp, float* vel, const float* acc,
@@ -363,12 +365,12 @@ int pmx_kd_adj_bin(pmx_ctx* c, const int16_t* pmid, float* disp, float* vel, con
                    long long n, float kp, float ka, float d, uint32_t* count, const BinOut& o,
                    int cap, double* part) {
   const MeshGeom g = pmx_geom_padded(c);
-  const unsigned nb1 = pmx_blocks(n);
+  const unsigned nb1 = pmx_kd_adj_blocks(n);
   // a snapshot already copied into disp: the drift's disp update is skipped
   const int keep_x = disp_snap != nullptr && disp_snap == disp;
   const float* snap = keep_x ? nullptr : disp_snap;
 #define KD_ADJ_LAUNCH(KP, CAPV, KPV)                                                          \
-  kd_adj_bin_k<KP, CAPV><<<nb1, PMX_TPB, 0, c->stream>>>(pmid, disp, vel, acc, disp_cot,       \
+  kd_adj_bin_k<KP, CAPV><<<nb1, KD_ADJ_TPB, 0, c->stream>>>(pmid, disp, vel, acc, disp_cot,       \
                                                          vel_cot, acc_cot, snap, n, KPV, ka, \
                                                          d, g, c->tg, count, o, part, keep_x)
   pmx_tic(c, PMX_T_KDADJ);
@@ -399,7 +401,7 @@ extern "C" int pmx_nbody_step_adj(pmx_ctx* c, const int16_t* pmid, float* disp, 
     return PMX_OK;
   }
   int rc, cap;
-  const unsigned nb1 = pmx_blocks(n);
+  const unsigned nb1 = pmx_kd_adj_blocks(n);
   // every allocation (the force VJP's value channels and three-channel halo
   // shells included) before the first kernel writes the caller's arrays, so
   // that PMX_ENOMEM leaves them as they were

@@ -1,8 +1,8 @@
 // Cloud-in-cell scatter/gather, gravity and time stepping (gfx950).
 //
 // Hot scatter (pmx_scatter_mass): particles are binned by the mesh tile that
-// holds their lower CIC corner (count with wave-aggregated integer atomics,
-// exclusive scan, fill), then one workgroup per tile accumulates its
+// holds their lower CIC corner (wave-aggregated integer atomics over a
+// capacity layout, or count, scan and emit), then one workgroup per tile accumulates its
 // particles into an LDS copy of the tile plus a +1 halo shell and writes the
 // tile interior with plain stores and the shell to a halo buffer; a fold
 // pass adds each tile's incoming shells.  No float atomics touch global
@@ -16,7 +16,7 @@
 
 __global__ void fill_u32_k(uint32_t* __restrict__ p, long long n, uint32_t v,
                            const uint32_t* __restrict__ cond) {
-  if (cond && *cond == 0) return;
+  if (pmx_cond_off(cond)) return;
   for (long long i = (long long)blockIdx.x * PMX_TPB + threadIdx.x; i < n;
        i += (long long)gridDim.x * PMX_TPB)
     p[i] = v;
@@ -83,73 +83,107 @@ extern "C" int pmx_tile_keys(pmx_ctx* c, const int16_t* pmid, const float* disp,
 }
 
 // ---------------------------------------------------- binned scatter --
-// The binning kernels below run over blocks of PMX_TPB particles, grid-
-// striding when the grid is capped (the exact re-binning after a capacity
-// overflow, launched before the device knows whether it is needed, exits at
-// once unless *cond != 0).
-template <bool CAP>
-__global__ void __launch_bounds__(PMX_TPB)
-    bin_count_k(const int16_t* __restrict__ pmid, const float* __restrict__ disp, long long n,
-                MeshGeom g, TileGeom tg, uint32_t* __restrict__ tile_count, BinOut o,
-                const uint32_t* __restrict__ cond) {
-  if (cond && *cond == 0) return;
-  __shared__ __align__(16) float sd[3 * PMX_TPB];
-  __shared__ __align__(16) int16_t sp[3 * PMX_TPB];
-  for (long long b0 = (long long)blockIdx.x * PMX_TPB; b0 < n;
-       b0 += (long long)gridDim.x * PMX_TPB) {
-    const int cnt = (int)(n - b0 < PMX_TPB ? n - b0 : PMX_TPB);
-    pmx_stage_in3<1, PMX_TPB>(sd, {{disp}}, b0, cnt);
-    pmx_stage_pmid<PMX_TPB>(sp, pmid, b0, cnt);
-    __syncthreads();
-    const int q = threadIdx.x;
-    const bool active = q < cnt;
-    uint32_t t = 0;
-    CicAxis ax[3];
-    float dp[3];
-    if (active) {
-      const int pm[3] = {sp[3 * q], sp[3 * q + 1], sp[3 * q + 2]};
-      dp[0] = sd[3 * q];
-      dp[1] = sd[3 * q + 1];
-      dp[2] = sd[3 * q + 2];
-      cic_setup(pm, dp, g, ax);
-      t = tile_of(ax, tg);
+// One binning pass over the particles, TPB * U of them a workgroup:
+//   BIN_COUNT  tile counts only: there are no counts to size the tiles by, or
+//              (with cond) flags[1] says that the last layout did not hold;
+//   BIN_FIRST  the capacity layout: counts and emits at once, unless flags[1]
+//              leaves it to BIN_COUNT;
+//   BIN_BOTH   either, as flags[1] says (one launch, for few particles);
+//   BIN_EMIT   the exact layout: emits by the cursors in ctr, unless (with
+//              cond) the first pass already did.
+// Global atomics bound this pass when each wave takes its own (17 M for 512^3
+// particles, at about 20 per ns), so the workgroup counts its tiles in LDS
+// (TileTable) and takes one per tile: consecutive particles share few tiles,
+// 8192 of them about 200 against eight per wave of 64.  Its records for a
+// tile are then one run of the tile, long enough to fill cache lines.  512^3
+// particles: count 0.55 ms, emit 1.5 ms; with atomics per wave 1.0 ms for the
+// counts and ranks and 2.2 ms for a separate fill.
+enum { BIN_COUNT = 0, BIN_FIRST = 1, BIN_EMIT = 2, BIN_BOTH = 3 };
+
+template <int KIND, int TPB, int U>
+__global__ void __launch_bounds__(TPB)
+    bin_k(const int16_t* __restrict__ pmid, const float* __restrict__ disp, long long n,
+          MeshGeom g, TileGeom tg, uint32_t* __restrict__ ctr, BinOut o,
+          const uint32_t* __restrict__ cond) {
+  if (KIND == BIN_EMIT && pmx_cond_off(cond)) return;
+  if (KIND == BIN_COUNT && cond && cond[1] == 0u) return;
+  if (KIND == BIN_FIRST && cond[1] != 0u) return;
+  const bool count = KIND == BIN_COUNT || (KIND == BIN_BOTH && cond[1] != 0u);
+  __shared__ TileTable<2 * TPB> T;
+  const unsigned nchunk = (unsigned)((n + U * TPB - 1) / (U * TPB));
+  for (unsigned cb = blockIdx.x; cb < nchunk; cb += gridDim.x) {
+    const long long c0 = (long long)cb * U * TPB;
+    tt_clear<2 * TPB, TPB>(T);
+    int pm[U][3];
+    float dp[U][3];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long i = c0 + u * TPB + threadIdx.x;
+      if (i < n) load_ptcl(pmid, disp, i, pm[u], dp[u]);
     }
-    const uint32_t r = agg_slot(tile_count, t, active);
-    if (active) pmx_bin_emit<CAP>(o, b0 + q, t, r, ax, tg);
+    __syncthreads();
+    float4 rec[U];
+    uint32_t t[U], rank[U];
+    int slot[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long i = c0 + u * TPB + threadIdx.x;
+      if (i < n) {
+        CicAxis ax[3];
+        cic_setup(pm[u], dp[u], g, ax);
+        t[u] = tile_of(ax, tg);
+        rec[u] = pmx_make_record(ax, tg);
+        slot[u] = tt_count<2 * TPB>(T, t[u], rank[u]);
+        if (slot[u] < 0) rank[u] = atomicAdd(&ctr[t[u]], 1u);
+      }
+    }
+    __syncthreads();
+    if (count) {
+      tt_reserve<2 * TPB, TPB, false>(T, ctr);
+    } else {
+      tt_reserve<2 * TPB, TPB, true>(T, ctr);
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const long long i = c0 + u * TPB + threadIdx.x;
+        if (i < n) {
+          const uint32_t r = rank[u] + (slot[u] < 0 ? 0u : T.base[slot[u]]);
+          const uint32_t b = o.start[t[u]], e = o.start[t[u] + 1];
+          if (r < e - b) {
+            o.rec[b + r] = rec[u];
+            o.pidx[b + r] = (uint32_t)i;
+          } else {
+            o.flag[0] = 1u;
+          }
+        }
+      }
+    }
     __syncthreads();
   }
 }
 
-// Writes the record (pmx_make_record) and index of each particle at
-// tile_start[tile] + rank once the tile counts are scanned.
-__global__ void __launch_bounds__(PMX_TPB)
-    bin_fill_k(const int16_t* __restrict__ pmid, const float* __restrict__ disp, long long n,
-               MeshGeom g, TileGeom tg, const uint32_t* __restrict__ ptile,
-               const uint32_t* __restrict__ prank, const uint32_t* __restrict__ tile_start,
-               float4* __restrict__ rec, uint32_t* __restrict__ pidx,
-               const uint32_t* __restrict__ cond) {
-  if (cond && *cond == 0) return;
-  __shared__ __align__(16) float sd[3 * PMX_TPB];
-  __shared__ __align__(16) int16_t sp[3 * PMX_TPB];
-  for (long long b0 = (long long)blockIdx.x * PMX_TPB; b0 < n;
-       b0 += (long long)gridDim.x * PMX_TPB) {
-    const int cnt = (int)(n - b0 < PMX_TPB ? n - b0 : PMX_TPB);
-    pmx_stage_in3<1, PMX_TPB>(sd, {{disp}}, b0, cnt);
-    pmx_stage_pmid<PMX_TPB>(sp, pmid, b0, cnt);
-    __syncthreads();
-    const int q = threadIdx.x;
-    const long long i = b0 + q;
-    if (q < cnt) {
-      const int pm[3] = {sp[3 * q], sp[3 * q + 1], sp[3 * q + 2]};
-      const float dp[3] = {sd[3 * q], sd[3 * q + 1], sd[3 * q + 2]};
-      CicAxis ax[3];
-      cic_setup(pm, dp, g, ax);
-      const uint32_t slot = tile_start[ptile[i]] + prank[i];
-      rec[slot] = pmx_make_record(ax, tg);
-      pidx[slot] = (uint32_t)i;
-    }
-    __syncthreads();
-  }
+// Launches a pass; few particles take small workgroups, so that every CU has
+// some.  Counting keeps little per particle and takes 8192 a workgroup, the
+// emitting kinds 2048 (with 8192 their records spill).  capped: the grid of a
+// pass that mostly returns at once.
+template <int KIND>
+static void bin_launch(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
+                       uint32_t* ctr, const uint32_t* cond, bool capped) {
+  const MeshGeom g = pmx_geom_padded(c);
+  const BinOut o = pmx_bin_out(c);
+  auto go = [&](auto tpb, auto u) {
+    constexpr int TPB = decltype(tpb)::value, U = decltype(u)::value;
+    const unsigned nb = pmx_blocks(n, TPB * U), cap = PMX_REBIN_GRID * PMX_TPB / TPB;
+    bin_k<KIND, TPB, U><<<capped && nb > cap ? cap : nb, TPB, 0, c->stream>>>(
+        pmid, disp, n, g, c->tg, ctr, o, cond);
+  };
+  using std::integral_constant;
+  if (n < PMX_BIN_SMALL)
+    go(integral_constant<int, 256>{}, integral_constant<int, 1>{});
+  else if constexpr (KIND == BIN_COUNT)
+    go(integral_constant<int, 1024>{}, integral_constant<int, 8>{});
+  else
+    go(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
 }
 
 __device__ __forceinline__ int shell_index(int qx, int qy, int qz, int sx, int sy, int sz) {
@@ -529,78 +563,38 @@ __global__ void __launch_bounds__(PMX_TPB)
   }
 }
 
-// Writes the binned records once the tile counts are scanned.
-int pmx_bin_fill(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
-                 const uint32_t* cond) {
-  if (n == 0) return PMX_OK;
-  const MeshGeom g = pmx_geom_padded(c);
-  const unsigned nb = cond ? pmx_blocks_capped(n, PMX_REBIN_GRID) : pmx_blocks(n);
-  pmx_tic(c, PMX_T_FILL);
-  bin_fill_k<<<nb, PMX_TPB, 0, c->stream>>>(pmid, disp, n, g, c->tg, c->pkey, c->prank,
-                                            c->tile_start, c->rec, c->pidx, cond);
-  pmx_toc(c, PMX_T_FILL);
-  PMX_LAUNCH_CHECK();
-  return PMX_OK;
-}
-
-int pmx_scan_tiles(pmx_ctx* c, const uint32_t* cond) {
-  pmx_tic(c, PMX_T_SCAN);
-  int rc = pmx_scan_exclusive(c, c->tile_count, c->tile_start, c->ntiles + 1, cond);
-  pmx_toc(c, PMX_T_SCAN);
-  return rc;
-}
-
-// Capacities from the counts of the last binning: count + slack per tile
-// (0 for the end slot), then the counts and the overflow flag are cleared.
-__global__ void tile_caps_k(uint32_t* __restrict__ count, uint32_t* __restrict__ cap, long long nt,
-                            uint32_t* __restrict__ flag) {
-  const long long i = (long long)blockIdx.x * PMX_TPB + threadIdx.x;
-  if (i <= nt) {
-    const uint32_t k = count[i];
-    cap[i] = i < nt ? k + pmx_tile_slack(k) : 0u;
-    count[i] = 0u;
-  }
-  if (i == 0) flag[0] = 0u;
-}
-
-int pmx_bin_begin(pmx_ctx* c, long long n, int* cap) {
+int pmx_bin_begin(pmx_ctx* c, long long n, int* cap, int may_count) {
   int rc;
   if ((rc = pmx_ensure_ptcl(c, n))) return rc;
   // the capacities of caps_n particles fit the record slots and 32-bit slots
   *cap = c->caps_valid && c->caps_n <= c->ptcl_cap && c->rec_cap < (1LL << 32) - 1;
   c->caps_valid = 0;  // until pmx_bin_end has exact counts again
-  if (!*cap) return pmx_fill_u32(c, c->tile_count, c->ntiles + 1, 0u);
+  if (!*cap) {
+    // the first capacity pass after this one emits
+    if ((rc = pmx_fill_u32(c, c->flags, 2, 0u))) return rc;
+    return pmx_fill_u32(c, c->tile_count, c->ntiles + 1, 0u);
+  }
   pmx_tic(c, PMX_T_SCAN);
-  tile_caps_k<<<pmx_blocks(c->ntiles + 1), PMX_TPB, 0, c->stream>>>(c->tile_count, c->tile_cap,
-                                                                    c->ntiles, c->flags);
-  PMX_LAUNCH_CHECK();
-  rc = pmx_scan_exclusive(c, c->tile_cap, c->tile_start, c->ntiles + 1);
+  rc = pmx_tile_caps(c, c->tile_count, c->tile_count, c->tile_start, may_count);
   pmx_toc(c, PMX_T_SCAN);
   return rc;
 }
 
 BinOut pmx_bin_out(pmx_ctx* c) {
-  return BinOut{c->pkey, c->prank, c->tile_start, c->rec, c->pidx, c->flags};
+  return BinOut{nullptr, nullptr, c->tile_start, c->rec, c->pidx, c->flags};
 }
 
 int pmx_bin_end(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n, int cap) {
   int rc;
-  if (!cap) {
-    if ((rc = pmx_scan_tiles(c))) return rc;
-    if ((rc = pmx_bin_fill(c, pmid, disp, n))) return rc;
-  } else if (n > 0) {
-    // a tile overflowed its capacity: count, scan and fill exactly, all
-    // conditional on the device-side flag
-    const uint32_t* f = c->flags;
-    const MeshGeom g = pmx_geom_padded(c);
-    if ((rc = pmx_fill_u32(c, c->tile_count, c->ntiles + 1, 0u, f))) return rc;
-    pmx_tic(c, PMX_T_BIN);
-    bin_count_k<false><<<pmx_blocks_capped(n, PMX_REBIN_GRID), PMX_TPB, 0, c->stream>>>(
-        pmid, disp, n, g, c->tg, c->tile_count, pmx_bin_out(c), f);
-    pmx_toc(c, PMX_T_BIN);
+  pmx_tic(c, PMX_T_SCAN);
+  rc = pmx_tile_exact(c, c->tile_count, c->tile_start, cap);
+  pmx_toc(c, PMX_T_SCAN);
+  if (rc) return rc;
+  if (n > 0) {
+    pmx_tic(c, PMX_T_FILL);
+    bin_launch<BIN_EMIT>(c, pmid, disp, n, c->tile_cap, cap ? c->flags : nullptr, cap != 0);
+    pmx_toc(c, PMX_T_FILL);
     PMX_LAUNCH_CHECK();
-    if ((rc = pmx_scan_tiles(c, f))) return rc;
-    if ((rc = pmx_bin_fill(c, pmid, disp, n, f))) return rc;
   }
   c->caps_valid = 1;
   c->caps_n = n;
@@ -610,17 +604,16 @@ int pmx_bin_end(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
 // Bins the particles by tile (c->rec, c->tile_start, c->tile_count).
 int pmx_bin_particles(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n) {
   int rc, cap;
-  if ((rc = pmx_bin_begin(c, n, &cap))) return rc;
+  if ((rc = pmx_bin_begin(c, n, &cap, 1))) return rc;
   if (n > 0) {
-    const MeshGeom g = pmx_geom_padded(c);
-    const BinOut o = pmx_bin_out(c);
     pmx_tic(c, PMX_T_BIN);
-    if (cap)
-      bin_count_k<true><<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(pmid, disp, n, g, c->tg,
-                                                                  c->tile_count, o, nullptr);
-    else
-      bin_count_k<false><<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(pmid, disp, n, g, c->tg,
-                                                                   c->tile_count, o, nullptr);
+    if (cap && n < PMX_BIN_SMALL) {
+      bin_launch<BIN_BOTH>(c, pmid, disp, n, c->tile_count, c->flags, false);
+    } else if (cap) {
+      bin_launch<BIN_FIRST>(c, pmid, disp, n, c->tile_count, c->flags, false);
+      bin_launch<BIN_COUNT>(c, pmid, disp, n, c->tile_count, c->flags, true);
+    } else
+      bin_launch<BIN_COUNT>(c, pmid, disp, n, c->tile_count, nullptr, false);
     pmx_toc(c, PMX_T_BIN);
     PMX_LAUNCH_CHECK();
   }
@@ -821,10 +814,11 @@ extern "C" int pmx_drift(pmx_ctx* c, long long n, float* disp, const float* vel,
   return PMX_OK;
 }
 
-// kick (k1) + drift (d) fused with the binning of the drifted particles;
-// the block's vel, acc and disp rows are staged through LDS
-template <bool CAP>
-__global__ void __launch_bounds__(PMX_TPB)
+// kick (k1) + drift (d) fused with the binning of the drifted particles, TPB *
+// U of them a workgroup with one global atomic per tile (as bin_k).  The
+// longer runs of a workgroup's ranks also make the fill after it faster.
+template <bool CAP, int TPB, int U>
+__global__ void __launch_bounds__(TPB)
     kick_drift_bin_k(const int16_t* __restrict__ pmid, float* __restrict__ disp,
                      float* __restrict__ vel, const float* __restrict__ acc, long long n, float k1,
                      float dd, MeshGeom g, TileGeom tg, uint32_t* __restrict__ tile_count,
@@ -834,40 +828,53 @@ __global__ void __launch_bounds__(PMX_TPB)
     k1 = fdev[0];
     dd = fdev[1];
   }
-  constexpr int T3 = 3 * PMX_TPB;
-  __shared__ __align__(16) float sh[3 * T3];  // vel | acc | disp
-  __shared__ __align__(16) int16_t sp[T3];
-  const long long b0 = (long long)blockIdx.x * PMX_TPB;
-  const int cnt = (int)(n - b0 < PMX_TPB ? n - b0 : PMX_TPB);
-  pmx_stage_in3<3, PMX_TPB>(sh, {{vel, acc, disp}}, b0, cnt);
-  pmx_stage_pmid<PMX_TPB>(sp, pmid, b0, cnt);
-  __syncthreads();
-  const int q = threadIdx.x;
-  const bool active = q < cnt;
-  uint32_t t = 0;
-  CicAxis ax[3];
-  float dp[3];
-  if (active) {
-    int pm[3];
+  __shared__ TileTable<2 * TPB> T;
+  tt_clear<2 * TPB, TPB>(T);
+  const long long c0 = (long long)blockIdx.x * U * TPB;
+  int pm[U][3];
+  float x[U][3], v[U][3], w[U][3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      pm[a] = sp[3 * q + a];
-      float v = sh[3 * q + a];
-      v = v + sh[T3 + 3 * q + a] * k1;
-      float x = sh[2 * T3 + 3 * q + a];
-      x = x + v * dd;
-      sh[3 * q + a] = v;
-      sh[2 * T3 + 3 * q + a] = x;
-      dp[a] = x;
+  for (int u = 0; u < U; ++u) {
+    const long long i = c0 + u * TPB + threadIdx.x;
+    if (i < n) {
+      load_ptcl(pmid, disp, i, pm[u], x[u]);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        v[u][a] = vel[3 * i + a];
+        w[u][a] = acc[3 * i + a];
+      }
     }
-    cic_setup(pm, dp, g, ax);
-    t = tile_of(ax, tg);
   }
-  const uint32_t r = agg_slot(tile_count, t, active);
-  if (active) pmx_bin_emit<CAP>(o, b0 + q, t, r, ax, tg);
   __syncthreads();
-  pmx_stage_out3<1, PMX_TPB>({{vel}}, sh, b0, cnt);
-  pmx_stage_out3<1, PMX_TPB>({{disp}}, sh + 2 * T3, b0, cnt);
+  CicAxis ax[U][3];
+  uint32_t t[U], rank[U];
+  int slot[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const long long i = c0 + u * TPB + threadIdx.x;
+    if (i < n) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        v[u][a] = v[u][a] + w[u][a] * k1;
+        x[u][a] = x[u][a] + v[u][a] * dd;
+        vel[3 * i + a] = v[u][a];
+        disp[3 * i + a] = x[u][a];
+      }
+      cic_setup(pm[u], x[u], g, ax[u]);
+      t[u] = tile_of(ax[u], tg);
+      slot[u] = tt_count<2 * TPB>(T, t[u], rank[u]);
+      if (slot[u] < 0) rank[u] = atomicAdd(&tile_count[t[u]], 1u);
+    }
+  }
+  __syncthreads();
+  tt_reserve<2 * TPB, TPB, true>(T, tile_count);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const long long i = c0 + u * TPB + threadIdx.x;
+    if (i < n)
+      pmx_bin_emit<CAP>(o, i, t[u], rank[u] + (slot[u] < 0 ? 0u : T.base[slot[u]]), ax[u], tg);
+  }
 }
 
 int pmx_kick_drift_bin(pmx_ctx* c, const int16_t* pmid, float* disp, float* vel, const float* acc,
@@ -876,12 +883,17 @@ int pmx_kick_drift_bin(pmx_ctx* c, const int16_t* pmid, float* disp, float* vel,
   // the first kick and drift of a call: entries 1 and 2 of a device table
   const float* fdev = c->dfac ? c->dfac + 1 : nullptr;
   pmx_tic(c, PMX_T_BIN);
-  if (cap)
-    kick_drift_bin_k<true><<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(pmid, disp, vel, acc, n, k1, d,
-                                                                     g, c->tg, count, o, fdev);
-  else
-    kick_drift_bin_k<false><<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(pmid, disp, vel, acc, n, k1,
-                                                                      d, g, c->tg, count, o, fdev);
+#define KD_GO(CAP, TPB, U)                                                                       \
+  kick_drift_bin_k<CAP, TPB, U><<<pmx_blocks(n, TPB * U), TPB, 0, c->stream>>>(                   \
+      pmid, disp, vel, acc, n, k1, d, g, c->tg, count, o, fdev)
+  if (n < PMX_BIN_SMALL) {
+    if (cap) KD_GO(true, 256, 1);
+    else KD_GO(false, 256, 1);
+  } else {
+    if (cap) KD_GO(true, 1024, 2);
+    else KD_GO(false, 1024, 2);
+  }
+#undef KD_GO
   pmx_toc(c, PMX_T_BIN);
   PMX_LAUNCH_CHECK();
   return PMX_OK;

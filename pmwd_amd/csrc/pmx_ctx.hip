@@ -335,7 +335,7 @@ extern "C" int pmx_ctx_destroy(pmx_ctx* c) {
                 c->red_out, c->sort_k[0], c->sort_k[1], c->sort_v[0], c->sort_v[1], c->sort_hist,
                 c->scan_tmp};
   for (void* p : ps) rel(p);
-  // pl[1], al[1], pl_tile and pl_rank alias the scratch freed above
+  // pl[1] and al[1] alias the scratch freed above
   void* qs[] = {c->pl[0].s0, c->pl[0].s1, c->pl_count[0], c->pl_start[0], c->pl_count[1],
                 c->pl_start[1], c->al[0].p.s0, c->al[0].p.s1, c->al[0].c0, c->al[0].c1,
                 c->abuf[0], c->abuf[1], c->abuf[2], c->al_dots, c->lbuf, c->tab};
@@ -402,7 +402,6 @@ extern "C" int pmx_ctx_trim(pmx_ctx* c, int what) {
   dev_free(c, (void**)&c->pl[0].s0, c->pl_cap * 16);
   dev_free(c, (void**)&c->pl[0].s1, c->pl_cap * 16);
   c->pl[1] = PState{};
-  c->pl_tile = c->pl_rank = nullptr;
   c->ptcl_cap = c->rec_cap = c->vrec_cap = c->pl_cap = 0;
   c->caps_valid = 0;
   if (c->halo_nch > 1) {
@@ -435,7 +434,7 @@ int pmx_ensure_ptcl(pmx_ctx* c, long long n) {
   free_adj_state(c);
   c->ptcl_cap = c->rec_cap = c->vrec_cap = c->pl_cap = 0;
   c->caps_valid = 0;
-  // pkey/prank hold a tile and rank per particle, or (multi-step re-bin) per record slot
+  // pkey/prank hold a tile and rank per particle
   int rc = dev_alloc(c, (void**)&c->rec, rcap * 16);
   rc |= dev_alloc(c, (void**)&c->pidx, rcap * 4);
   rc |= dev_alloc(c, (void**)&c->pkey, rcap * 4);
@@ -465,9 +464,8 @@ int pmx_ensure_halo(pmx_ctx* c, int nch) {
 
 // The multi-step pipeline's two tile-ordered particle copies of rec_cap
 // slots: the first is its own memory, the second lives in the per-step
-// path's scratch (s0 in rec, s1 in the four vrec channels), and
-// the exact re-bin's per-slot tile and rank in pkey/prank.  The per-step
-// path rewrites all of these before it reads them.
+// path's scratch (s0 in rec, s1 in the four vrec channels).  The per-step
+// path rewrites these before it reads them.
 int pmx_ensure_state(pmx_ctx* c) {
   int rc;
   if ((rc = pmx_ensure_vrec(c))) return rc;
@@ -492,8 +490,6 @@ int pmx_ensure_state(pmx_ctx* c) {
   }
   c->pl[1].s0 = c->rec;
   c->pl[1].s1 = reinterpret_cast<float4*>(c->vrec);
-  c->pl_tile = c->pkey;
-  c->pl_rank = c->prank;
   return PMX_OK;
 }
 
@@ -613,11 +609,11 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
   return incl - v;
 }
 
-// The scan kernels return at once when cond is given and *cond == 0 (a
-// device-side decision, no host round trip).
+// The scan kernels return at once when cond is given and both of its
+// flags are 0 (a device-side decision, no host round trip).
 __global__ void scan_reduce_k(const uint32_t* __restrict__ in, long long n, uint32_t* __restrict__ bsum,
                               const uint32_t* __restrict__ cond) {
-  if (cond && *cond == 0) return;
+  if (pmx_cond_off(cond)) return;
   __shared__ uint32_t sh[PMX_TPB];
   long long base = (long long)blockIdx.x * SCAN_TILE;
   uint32_t s = 0;
@@ -632,7 +628,7 @@ __global__ void scan_reduce_k(const uint32_t* __restrict__ in, long long n, uint
 
 __global__ void scan_single_k(uint32_t* __restrict__ data, long long n,
                               const uint32_t* __restrict__ cond) {
-  if (cond && *cond == 0) return;
+  if (pmx_cond_off(cond)) return;
   __shared__ uint32_t sh[PMX_TPB];
   uint32_t carry = 0;
   for (long long base = 0; base < n; base += PMX_TPB) {
@@ -648,7 +644,7 @@ __global__ void scan_single_k(uint32_t* __restrict__ data, long long n,
 __global__ void scan_apply_k(const uint32_t* __restrict__ in, long long n,
                              const uint32_t* __restrict__ boff, uint32_t* __restrict__ out,
                              const uint32_t* __restrict__ cond) {
-  if (cond && *cond == 0) return;
+  if (pmx_cond_off(cond)) return;
   __shared__ uint32_t sh[PMX_TPB];
   long long base = (long long)blockIdx.x * SCAN_TILE + (long long)threadIdx.x * SCAN_ITEMS;
   uint32_t v[SCAN_ITEMS];
@@ -697,6 +693,137 @@ int pmx_scan_exclusive(pmx_ctx* c, const uint32_t* in, uint32_t* out, long long 
   scan_apply_k<<<(unsigned)nb, PMX_TPB, 0, c->stream>>>(in, n, c->scan_tmp, out, cond);
   PMX_LAUNCH_CHECK();
   return PMX_OK;
+}
+
+// ------------------------------------------------------- tile layouts --
+// The capacity or exact layout in one workgroup (pmx_tile_caps, _exact):
+// each binning pass and pipeline step makes both, and at few tiles the three
+// kernels of a scan and one for the capacities cost their launches (2 to 5 us
+// each).  1024 threads scan 4096 tiles a round, about 4 us: 513 and 4097
+// entries take 4 and 7 us against 7 to 19, but 32769 (a 512^3 mesh) 35.
+#define TILE_SCAN_TPB 1024
+#define TILE_SCAN_MAX 8193
+
+struct TileLayout {
+  const uint32_t* in;   // counts
+  uint32_t* clear;      // counts to clear (capacities only)
+  uint32_t* cap;
+  uint32_t* start;
+  uint32_t* flags;
+  long long n;          // entries, the end slot last
+};
+
+template <bool CAPS>
+__global__ void __launch_bounds__(TILE_SCAN_TPB)
+    tile_layout_k(TileLayout L, int may_count, int conditional) {
+  constexpr int I = 4;
+  __shared__ uint32_t wsum[TILE_SCAN_TPB / 64];
+  __shared__ uint32_t s_over;
+  const uint32_t f0 = L.flags[0], f1 = L.flags[1];
+  if (!CAPS && conditional && (f0 | f1) == 0u) return;
+  if (threadIdx.x == 0) s_over = 0u;
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t carry = 0;
+  for (long long base = 0; base < L.n; base += TILE_SCAN_TPB * I) {
+    const long long i0 = base + (long long)threadIdx.x * I;
+    uint32_t v[I], sum = 0;
+#pragma unroll
+    for (int k = 0; k < I; ++k) {
+      const long long i = i0 + k;
+      v[k] = 0u;
+      if (i < L.n) {
+        const uint32_t q = L.in[i];
+        v[k] = CAPS ? (i + 1 < L.n ? q + pmx_tile_slack(q) : 0u) : q;
+        if (CAPS) {
+          L.cap[i] = v[k];
+          L.clear[i] = 0u;
+        } else {
+          if (conditional && f1 && i + 1 < L.n && q > L.cap[i]) s_over = 1u;
+          L.cap[i] = 0u;
+        }
+      }
+      sum += v[k];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t x = __shfl_up(incl, o);
+      if (lane >= o) incl += x;
+    }
+    __syncthreads();  // wsum of the round before has been read
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    uint32_t off = carry, tot = 0;
+#pragma unroll
+    for (int w = 0; w < TILE_SCAN_TPB / 64; ++w) {
+      if (w < wave) off += wsum[w];
+      tot += wsum[w];
+    }
+    carry += tot;
+    uint32_t ex = off + incl - sum;
+#pragma unroll
+    for (int k = 0; k < I; ++k) {
+      if (i0 + k < L.n) L.start[i0 + k] = ex;
+      ex += v[k];
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  if (CAPS) {
+    L.flags[1] = may_count ? f0 : 0u;
+    L.flags[0] = 0u;
+  } else if (conditional && f1) {
+    L.flags[0] = s_over;
+  }
+}
+
+// The parts besides the scan, for more tiles than one workgroup takes.
+__global__ void tile_caps_k(TileLayout L, int may_count) {
+  const long long i = (long long)blockIdx.x * PMX_TPB + threadIdx.x;
+  if (i < L.n) {
+    const uint32_t k = L.in[i];
+    L.cap[i] = i + 1 < L.n ? k + pmx_tile_slack(k) : 0u;
+    L.clear[i] = 0u;
+  }
+  if (i == 0) {
+    L.flags[1] = may_count ? L.flags[0] : 0u;
+    L.flags[0] = 0u;
+  }
+}
+
+__global__ void tile_cursors_k(TileLayout L, int conditional) {
+  if (conditional && (L.flags[0] | L.flags[1]) == 0u) return;
+  const long long i = (long long)blockIdx.x * PMX_TPB + threadIdx.x;
+  if (i >= L.n) return;
+  if (conditional && L.flags[1] && i + 1 < L.n && L.in[i] > L.cap[i]) L.flags[0] = 1u;
+  L.cap[i] = 0u;
+}
+
+int pmx_tile_caps(pmx_ctx* c, const uint32_t* count_in, uint32_t* count_out, uint32_t* start,
+                  int may_count, int flag0) {
+  const TileLayout L = {count_in, count_out, c->tile_cap, start, c->flags + flag0, c->ntiles + 1};
+  if (L.n <= TILE_SCAN_MAX) {
+    tile_layout_k<true><<<1, TILE_SCAN_TPB, 0, c->stream>>>(L, may_count, 0);
+    PMX_LAUNCH_CHECK();
+    return PMX_OK;
+  }
+  tile_caps_k<<<pmx_blocks(L.n), PMX_TPB, 0, c->stream>>>(L, may_count);
+  PMX_LAUNCH_CHECK();
+  return pmx_scan_exclusive(c, c->tile_cap, start, L.n);
+}
+
+int pmx_tile_exact(pmx_ctx* c, const uint32_t* count, uint32_t* start, int conditional,
+                   int flag0) {
+  const TileLayout L = {count, nullptr, c->tile_cap, start, c->flags + flag0, c->ntiles + 1};
+  if (L.n <= TILE_SCAN_MAX) {
+    tile_layout_k<false><<<1, TILE_SCAN_TPB, 0, c->stream>>>(L, 0, conditional);
+    PMX_LAUNCH_CHECK();
+    return PMX_OK;
+  }
+  tile_cursors_k<<<pmx_blocks(L.n), PMX_TPB, 0, c->stream>>>(L, conditional);
+  PMX_LAUNCH_CHECK();
+  return pmx_scan_exclusive(c, count, start, L.n, conditional ? L.flags : nullptr);
 }
 
 // -------------------------------------------------------------- dot ---

@@ -168,19 +168,19 @@ struct pmx_ctx {
   // plus slack (tile_cap), tile_start the scan of the capacities, and the
   // binning kernel writes the records itself; flags[0] is set on the device
   // when a tile overflows, which runs the exact count/scan/fill after it.
+  // tile_cap then serves as the cursors of an exact emission.  flags[0]: the
+  // last capacity layout did not hold its particles; flags[1]: the pass under
+  // way only counts (see pmx_bin_begin); flags[2..3]: the pipelines' pair.
   uint32_t* tile_cap;
   uint32_t* flags;
   int caps_valid;      // host: tile_count holds the exact counts of caps_n particles
   long long caps_n;
   long long rec_cap;   // record slots of rec/pidx (and the vrec channel stride)
   // multi-step pipeline: two tile-ordered particle copies of rec_cap slots
-  // (the second aliases rec/vrec/pidx), their tile counts and starts, and
-  // the per-slot tile/rank of an exact re-bin (aliases pkey/prank)
+  // (the second aliases rec/vrec/pidx), their tile counts and starts
   PState pl[2];
   uint32_t* pl_count[2];
   uint32_t* pl_start[2];
-  uint32_t* pl_tile;
-  uint32_t* pl_rank;
   long long pl_cap;    // slots of the pipeline's own copy
   // reverse-time pipeline: its own particle copy (the second aliases rec,
   // vrec, pidx and the forward pipeline's copy) and three mesh buffers
@@ -271,6 +271,20 @@ int pmx_dev_alloc(pmx_ctx* c, void** p, size_t bytes);
 void pmx_dev_free(pmx_ctx* c, void** p, size_t bytes);
 int pmx_scan_exclusive(pmx_ctx* c, const uint32_t* in, uint32_t* out, long long n,
                        const uint32_t* cond = nullptr);
+// The capacity layout of the next binning: cap = count_in + slack per tile,
+// start their scan, count_out (may be count_in) cleared, flags[1] the last
+// verdict when may_count, flags[0] cleared.  And the exact layout after a
+// pass whose counts are complete: start the scan of count and the cursors
+// cap cleared; with conditional, only when flags[0] or flags[1] is set, and
+// then flags[0] also says whether the capacities would have held a pass that
+// only counted.
+// flag0: which pair of flags (the pipelines keep theirs apart, so that the
+// verdict of the single passes outlives a run).
+#define PMX_FLAG_PL 2
+int pmx_tile_caps(pmx_ctx* c, const uint32_t* count_in, uint32_t* count_out, uint32_t* start,
+                  int may_count, int flag0 = 0);
+int pmx_tile_exact(pmx_ctx* c, const uint32_t* count, uint32_t* start, int conditional,
+                   int flag0 = 0);
 
 // Slack of a tile's capacity over its last count, and the record slots the
 // capacities of n particles can take (sum over tiles of count + slack).
@@ -422,9 +436,10 @@ __device__ __forceinline__ float4 pmx_make_record(const CicAxis ax[3], const Til
 }
 
 // Where a binning kernel puts particle i of tile t with rank r.  Exact mode
-// (CAP false): the tile and rank, for the fill after the scan of the counts.
-// Capacity mode: the record itself at start[t] + r when r is below the
-// tile's capacity start[t+1] - start[t], else the overflow flag.
+// (CAP false): the tile and rank, for a fill after the scan of the counts
+// (where the caller's fill takes them from there).  Capacity mode: the record
+// itself at start[t] + r when r is below the tile's capacity start[t+1] -
+// start[t], else the overflow flag.
 struct BinOut {
   uint32_t* ptile;
   uint32_t* prank;
@@ -438,8 +453,10 @@ template <bool CAP>
 __device__ __forceinline__ void pmx_bin_emit(const BinOut& o, long long i, uint32_t t, uint32_t r,
                                              const CicAxis ax[3], const TileGeom& tg) {
   if (!CAP) {
-    o.ptile[i] = t;
-    o.prank[i] = r;
+    if (o.ptile) {
+      o.ptile[i] = t;
+      o.prank[i] = r;
+    }
     return;
   }
   const uint32_t b = o.start[t], e = o.start[t + 1];
@@ -451,31 +468,112 @@ __device__ __forceinline__ void pmx_bin_emit(const BinOut& o, long long i, uint3
   }
 }
 
+// A conditional kernel's exit: neither flag is set.
+__device__ __forceinline__ bool pmx_cond_off(const uint32_t* cond) {
+  return cond && (cond[0] | cond[1]) == 0u;
+}
+
+// The lanes of a wave grouped by key with ballots: each lane's group leader
+// and rank in its group, and the leader's group size (0 elsewhere).
+struct AggGroup {
+  int leader;
+  uint32_t rank, size;
+};
+__device__ __forceinline__ AggGroup agg_group(uint32_t key, bool active) {
+  unsigned long long pending = __ballot(active);
+  const int lane = __lane_id();
+  AggGroup a = {lane, 0u, 0u};
+  while (pending) {
+    const int leader = __ffsll((long long)pending) - 1;  // wave-uniform
+    const uint32_t lkey = (uint32_t)__builtin_amdgcn_readlane((int)key, leader);
+    const unsigned long long peers = __ballot(active && key == lkey) & pending;
+    if (active && key == lkey) {
+      a.leader = leader;
+      a.rank = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+    }
+    if (lane == leader) a.size = (uint32_t)__popcll(peers);
+    pending &= ~peers;
+  }
+  return a;
+}
+
 // Wave-aggregated atomicAdd(&ctr[key], 1): returns this lane's slot.
 // Every lane of the wave must call it (inactive lanes pass active=false).
 // The lanes are grouped by key with ballots first; then each group's leader
 // adds the group size, all leaders in one instruction, so the wave waits for
 // a single atomic round trip however many keys it holds.
 __device__ __forceinline__ uint32_t agg_slot(uint32_t* __restrict__ ctr, uint32_t key, bool active) {
-  unsigned long long pending = __ballot(active);
-  const int lane = __lane_id();
-  int my_leader = lane;
-  uint32_t my_rank = 0, group = 0;
-  while (pending) {
-    const int leader = __ffsll((long long)pending) - 1;  // wave-uniform
-    const uint32_t lkey = (uint32_t)__builtin_amdgcn_readlane((int)key, leader);
-    const unsigned long long peers = __ballot(active && key == lkey) & pending;
-    if (active && key == lkey) {
-      my_leader = leader;
-      my_rank = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
-    }
-    if (lane == leader) group = (uint32_t)__popcll(peers);
-    pending &= ~peers;
-  }
+  const AggGroup a = agg_group(key, active);
   uint32_t base = 0;
-  if (group) base = atomicAdd(&ctr[key], group);
-  base = __shfl(base, my_leader);
-  return base + my_rank;
+  if (a.size) base = atomicAdd(&ctr[key], a.size);
+  base = __shfl(base, a.leader);
+  return base + a.rank;
+}
+
+// Tile counters of a workgroup's particles in LDS: an open-addressing table
+// of S (a power of two) tiles with their counts here and, once reserved, the
+// workgroup's base in the global counters, so that a tile costs one global
+// atomic per workgroup.  A particle whose tile finds no place in PROBES steps
+// (particles in no spatial order) takes its slot from the global counter.
+template <int S>
+struct TileTable {
+  uint32_t key[S], cnt[S], base[S];
+};
+#define PMX_NO_TILE 0xffffffffu
+// particles below which the binning passes take small workgroups
+#define PMX_BIN_SMALL (1 << 20)
+
+template <int S, int TPB>
+__device__ __forceinline__ void tt_clear(TileTable<S>& T) {
+  for (int i = threadIdx.x; i < S; i += TPB) {
+    T.key[i] = PMX_NO_TILE;
+    T.cnt[i] = 0u;
+  }
+}
+
+// Counts one particle of tile t: its place in the table (or -1) and its rank
+// among the workgroup's particles there.
+template <int S>
+__device__ __forceinline__ int tt_count(TileTable<S>& T, uint32_t t, uint32_t& rank) {
+  constexpr int PROBES = 8;
+  uint32_t h = (t * 0x9E3779B1u) & (S - 1);
+  for (int p = 0; p < PROBES; ++p) {
+    uint32_t k = T.key[h];
+    if (k == PMX_NO_TILE) {
+      k = atomicCAS(&T.key[h], PMX_NO_TILE, t);
+      if (k == PMX_NO_TILE) k = t;
+    }
+    if (k == t) {
+      rank = atomicAdd(&T.cnt[h], 1u);
+      return (int)h;
+    }
+    h = (h + 1) & (S - 1);
+  }
+  return -1;
+}
+
+// Reserves every tile's particles in the global counters (between barriers);
+// with RET false the base is not wanted.
+template <int S, int TPB, bool RET>
+__device__ __forceinline__ void tt_reserve(TileTable<S>& T, uint32_t* __restrict__ ctr) {
+  constexpr int N = (S + TPB - 1) / TPB;
+  uint32_t b[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const int i = threadIdx.x + k * TPB;
+    b[k] = 0u;
+    if (i < S && T.cnt[i]) {
+      if (RET)
+        b[k] = atomicAdd(&ctr[T.key[i]], T.cnt[i]);
+      else
+        atomicAdd(&ctr[T.key[i]], T.cnt[i]);
+    }
+  }
+  if (RET) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if ((int)threadIdx.x + k * TPB < S) T.base[threadIdx.x + k * TPB] = b[k];
+  }
 }
 
 // ------------------------------------------------ AoS staging through LDS --
@@ -906,17 +1004,16 @@ __device__ __forceinline__ void pmx_unpack_local(float w, int& lx, int& ly, int&
 // ------------------------------------------------- shared host drivers --
 // with cond, the fill, scan and binning kernels do nothing unless *cond != 0
 int pmx_fill_u32(pmx_ctx* c, uint32_t* p, long long n, uint32_t v, const uint32_t* cond = nullptr);
-int pmx_scan_tiles(pmx_ctx* c, const uint32_t* cond = nullptr);
-int pmx_bin_fill(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
-                 const uint32_t* cond = nullptr);
 int pmx_bin_particles(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n);
-// A binning pass in three parts: pmx_bin_begin zeroes the counts and, when
-// the counts of the last pass can size the tiles, sets up the capacity
-// layout (returns *cap = 1); the caller's binning kernel then counts the
-// particles and emits them (pmx_bin_out gives its BinOut); pmx_bin_end
-// finishes the exact path, or re-bins exactly on the device when a tile
-// overflowed, and records the counts for the next pass.
-int pmx_bin_begin(pmx_ctx* c, long long n, int* cap);
+// A binning pass in three parts.  pmx_bin_begin clears the counts and, when
+// the counts of the last pass can size the tiles, sets up the capacity layout
+// (returns *cap = 1); the caller's binning kernel then counts the particles
+// and, in the capacity layout, emits them (pmx_bin_out gives its BinOut).  A
+// kernel that obeys flags[1] (may_count) only counts where the last layout
+// did not hold, as for a state unrelated to the last one.  pmx_bin_end lays
+// the tiles out by the counts and emits the particles where the pass did
+// not, decided on the device, and the counts are there for the next pass.
+int pmx_bin_begin(pmx_ctx* c, long long n, int* cap, int may_count = 0);
 BinOut pmx_bin_out(pmx_ctx* c);
 int pmx_bin_end(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n, int cap);
 // The r2c row pass of the Poisson solve can add the deposit's halo shells as
@@ -944,7 +1041,9 @@ int pmx_ensure_state(pmx_ctx* c);
 int pmx_ensure_adj_state(pmx_ctx* c, int nsteps);
 // reverse kick(s) and drift of the caller's arrays (pending closing kick kp
 // first when nonzero), binned into count/o; per-block partials of the drift
-// dot product at part[0, pmx_blocks(n))
+// dot product at part[0, pmx_kd_adj_blocks(n))
+#define KD_ADJ_TPB 512
+inline unsigned pmx_kd_adj_blocks(long long n) { return pmx_blocks(n, KD_ADJ_TPB); }
 int pmx_kd_adj_bin(pmx_ctx* c, const int16_t* pmid, float* disp, float* vel, const float* acc,
                    float* disp_cot, float* vel_cot, const float* acc_cot, const float* disp_snap,
                    long long n, float kp, float ka, float d, uint32_t* count, const BinOut& o,

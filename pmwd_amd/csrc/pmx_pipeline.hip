@@ -12,8 +12,8 @@
 // counts).  The deposit of the next step reads the new copy in tile order.
 // Only the first kick/drift and the last closing kick touch the caller's
 // arrays.  A tile that overflows its capacity makes the device redo the step
-// exactly (count, scan, write), all launched unconditionally and skipped on
-// the device unless the overflow flag is set.
+// exactly (scan of the counts, write), launched unconditionally and skipped
+// on the device unless the overflow flag is set.
 //
 // Every floating-point operation is the one pmx_nbody_step performs, in the
 // same order, so the results are bitwise those of nsteps pmx_nbody_step calls
@@ -33,15 +33,14 @@
 // tile overflowed
 #define PL_REBIN_GRID 2048u
 
-enum { PL_CAP = 0, PL_COUNT = 1, PL_WRITE = 2, PL_LAST = 3 };
+enum { PL_CAP = 0, PL_WRITE = 2, PL_LAST = 3 };
 
 // Destination of a pipeline step.
 struct PlOut {
   PState st;
-  uint32_t* count;        // per-tile counts of the destination (atomics)
+  uint32_t* count;        // per-tile counts of the destination (atomics); the
+                          // exact re-bin: its cursors
   const uint32_t* start;  // per-tile starts of the destination
-  uint32_t* ptile;        // exact re-bin: tile and rank per source slot
-  uint32_t* prank;
   uint32_t* flag;         // overflow flag
 };
 
@@ -58,55 +57,52 @@ __device__ __forceinline__ void pl_put(const PState& st, uint32_t slot, float4 s
 }
 
 // Writes particle i (after the first kick and drift) to the slot
-// start[ptile[i]] + prank[i] of st, pm reduced mod the mesh extent.
-__global__ void __launch_bounds__(PMX_TPB)
+// start[ptile[i]] + prank[i] of st, pm reduced mod the mesh extent.  TPB * U
+// particles a workgroup as in the kick and drift that ranked them: their
+// runs of a tile then complete their cache lines in one L2 (512^3: 2.92 ms
+// when eight workgroups on eight XCDs share a run).
+template <int TPB, int U>
+__global__ void __launch_bounds__(TPB)
     pl_fill_k(const int16_t* __restrict__ pmid, const float* __restrict__ disp,
               const float* __restrict__ vel, long long n, MeshGeom g,
               const uint32_t* __restrict__ ptile, const uint32_t* __restrict__ prank,
               const uint32_t* __restrict__ start, PState st) {
-  constexpr int T3 = 3 * PMX_TPB;
-  __shared__ __align__(16) float sh[2 * T3];  // disp | vel
-  __shared__ __align__(16) int16_t sp[T3];
-  const long long b0 = (long long)blockIdx.x * PMX_TPB;
-  const int cnt = (int)(n - b0 < PMX_TPB ? n - b0 : PMX_TPB);
-  pmx_stage_in3<2, PMX_TPB>(sh, {{disp, vel}}, b0, cnt);
-  pmx_stage_pmid<PMX_TPB>(sp, pmid, b0, cnt);
-  __syncthreads();
-  const int q = threadIdx.x;
-  if (q >= cnt) return;
-  const long long i = b0 + q;
-  const uint32_t px = (uint32_t)pmx_wrap(sp[3 * q], g.n0);
-  const uint32_t py = (uint32_t)pmx_wrap(sp[3 * q + 1], g.n1);
-  const uint32_t pz = (uint32_t)pmx_wrap(sp[3 * q + 2], g.n2);
-  const float4 s0 = make_float4(sh[3 * q], sh[3 * q + 1], sh[3 * q + 2],
-                                __uint_as_float(pmx_state_pack(px, py, pz)));
-  const float4 s1 = make_float4(sh[T3 + 3 * q], sh[T3 + 3 * q + 1], sh[T3 + 3 * q + 2],
-                                __uint_as_float((uint32_t)i));
-  pl_put(st, start[ptile[i]] + prank[i], s0, s1);
-}
-
-// Capacities of the next copy from the counts of the current one; clears
-// the next copy's counts and the overflow flag.
-__global__ void pl_caps_k(const uint32_t* __restrict__ count_in, uint32_t* __restrict__ cap,
-                          uint32_t* __restrict__ count_out, long long nt,
-                          uint32_t* __restrict__ flag) {
-  const long long i = (long long)blockIdx.x * PMX_TPB + threadIdx.x;
-  if (i <= nt) {
-    const uint32_t k = count_in[i];
-    cap[i] = i < nt ? k + pmx_tile_slack(k) : 0u;
-    count_out[i] = 0u;
+  const long long c0 = (long long)blockIdx.x * U * TPB;
+  int pm[U][3];
+  float x[U][3], v[U][3];
+  uint32_t slot[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const long long i = c0 + u * TPB + threadIdx.x;
+    if (i < n) {
+      slot[u] = start[ptile[i]] + prank[i];
+      load_ptcl(pmid, disp, i, pm[u], x[u]);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) v[u][a] = vel[3 * i + a];
+    }
   }
-  if (i == 0) flag[0] = 0u;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const long long i = c0 + u * TPB + threadIdx.x;
+    if (i < n) {
+      const uint32_t px = (uint32_t)pmx_wrap(pm[u][0], g.n0);
+      const uint32_t py = (uint32_t)pmx_wrap(pm[u][1], g.n1);
+      const uint32_t pz = (uint32_t)pmx_wrap(pm[u][2], g.n2);
+      pl_put(st, slot[u],
+             make_float4(x[u][0], x[u][1], x[u][2], __uint_as_float(pmx_state_pack(px, py, pz))),
+             make_float4(v[u][0], v[u][1], v[u][2], __uint_as_float((uint32_t)i)));
+    }
+  }
 }
 
 // One workgroup per tile of the source copy: gather, closing kick k2; then
 // (not LAST) opening kick k1n and drift dn of the next step and the move to
 // the new tile:
 //   PL_CAP    capacity slot in the destination, or the overflow flag;
-//   PL_COUNT  exact re-bin, pass 1: tile and rank per source slot;
-//   PL_WRITE  exact re-bin, pass 2: the particle to its exact slot;
+//   PL_WRITE  exact re-bin: the particle to the next slot of its tile in the
+//             layout of PL_CAP's counts;
 //   PL_LAST   acc, vel and disp to the caller's arrays at the particle index.
-// PL_COUNT and PL_WRITE return at once unless the overflow flag is set.
+// PL_WRITE returns at once unless the overflow flag is set.
 template <int MODE, int FULL = 0>
 __global__ void __launch_bounds__(PL_TPB, PL_MINB)
     pl_step_k(PState in, const uint32_t* __restrict__ in_start,
@@ -114,7 +110,7 @@ __global__ void __launch_bounds__(PL_TPB, PL_MINB)
               const float* __restrict__ F0, const float* __restrict__ F1,
               const float* __restrict__ F2, float k2, float k1n, float dn, PlOut out,
               PlUser user, const float* __restrict__ fdev) {
-  if ((MODE == PL_COUNT || MODE == PL_WRITE) && out.flag[0] == 0u) return;
+  if (MODE == PL_WRITE && out.flag[0] == 0u) return;
   // factors from the device table when the call has one: this step's
   // {k1, d, k2} then the next step's {k1, d}
   if (fdev) {
@@ -128,7 +124,7 @@ __global__ void __launch_bounds__(PL_TPB, PL_MINB)
   // PL_CAP: runs per neighbour tile and round (pl_nbr_code, pl_round_bases),
   // so a round's stores into a tile are one run instead of one per wave
   __shared__ uint32_t s_cnt[27], s_base[27];
-  // the exact re-bin (COUNT, WRITE: rare) walks the tiles with a small grid,
+  // the exact re-bin (WRITE: rare) walks the tiles with a small grid,
   // so that it costs little when the overflow flag is clear
   auto tile = [&](const int t) {
     int o[3], s[3], ti[3];
@@ -202,20 +198,8 @@ __global__ void __launch_bounds__(PL_TPB, PL_MINB)
   #pragma unroll
         for (int u = 0; u < PL_U; ++u) {
           const uint32_t q = q0 + u * PL_TPB + threadIdx.x;
-          if (q < cnt)
-            pl_put(out.st, out.start[out.ptile[start + q]] + out.prank[start + q], n0[u], n1[u]);
-        }
-        continue;
-      }
-      if (MODE == PL_COUNT) {
-  #pragma unroll
-        for (int u = 0; u < PL_U; ++u) {
-          const uint32_t q = q0 + u * PL_TPB + threadIdx.x;
           const uint32_t r = agg_slot(out.count, nt[u], q < cnt);
-          if (q < cnt) {
-            out.ptile[start + q] = nt[u];
-            out.prank[start + q] = r;
-          }
+          if (q < cnt) pl_put(out.st, out.start[nt[u]] + r, n0[u], n1[u]);
         }
         continue;
       }
@@ -245,7 +229,7 @@ __global__ void __launch_bounds__(PL_TPB, PL_MINB)
       }
     }
   };
-  if (MODE == PL_COUNT || MODE == PL_WRITE) {
+  if (MODE == PL_WRITE) {
     const unsigned ntl = (unsigned)tg.ntx * tg.nty * tg.ntz;
     for (unsigned tb = blockIdx.x; tb < ntl; tb += gridDim.x) {
       tile((int)pmx_xcd_block(tb, ntl));
@@ -263,7 +247,7 @@ static void pl_launch(pmx_ctx* c, int src, PlOut out, PlUser user, float k2, flo
   const MeshGeom g = pmx_geom_padded(c);
   const TileGeom& tg = c->tg;
   const size_t lds = (size_t)3 * (tg.tx + 1) * (tg.ty + 1) * (tg.tz + 1) * sizeof(float);
-  const bool rebin = MODE == PL_COUNT || MODE == PL_WRITE;
+  const bool rebin = MODE == PL_WRITE;
   const unsigned grid = rebin && c->ntiles > PL_REBIN_GRID ? PL_REBIN_GRID : (unsigned)c->ntiles;
   // tile strides as constants when every tile is a full 16^3 tile
   if (pmx_full16(c))
@@ -306,8 +290,12 @@ static int nbody_steps_run(pmx_ctx* c, const int16_t* pmid, float* disp, float* 
   pmx_toc(c, PMX_T_SCAN);
   if (rc) return rc;
   pmx_tic(c, PMX_T_FILL);
-  pl_fill_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(pmid, disp, vel, n, g, c->pkey, c->prank,
-                                                      c->pl_start[A], c->pl[A]);
+#define PL_FILL(TPB, U)                                                                      \
+  pl_fill_k<TPB, U><<<pmx_blocks(n, TPB * U), TPB, 0, c->stream>>>(                           \
+      pmid, disp, vel, n, g, c->pkey, c->prank, c->pl_start[A], c->pl[A])
+  if (n < PMX_BIN_SMALL) PL_FILL(256, 1);
+  else PL_FILL(1024, 2);
+#undef PL_FILL
   pmx_toc(c, PMX_T_FILL);
   PMX_LAUNCH_CHECK();
 
@@ -326,24 +314,20 @@ static int nbody_steps_run(pmx_ctx* c, const int16_t* pmid, float* disp, float* 
     }
     const int B = 1 - A;
     pmx_tic(c, PMX_T_SCAN);
-    pl_caps_k<<<pmx_blocks(nt + 1), PMX_TPB, 0, c->stream>>>(c->pl_count[A], c->tile_cap,
-                                                             c->pl_count[B], nt, c->flags);
-    PMX_LAUNCH_CHECK();
-    rc = pmx_scan_exclusive(c, c->tile_cap, c->pl_start[B], nt + 1);
+    rc = pmx_tile_caps(c, c->pl_count[A], c->pl_count[B], c->pl_start[B], 0, PMX_FLAG_PL);
     pmx_toc(c, PMX_T_SCAN);
     if (rc) return rc;
-    const PlOut out = {c->pl[B], c->pl_count[B], c->pl_start[B], c->pl_tile, c->pl_rank, c->flags};
+    const PlOut out = {c->pl[B], c->pl_count[B], c->pl_start[B], c->flags + PMX_FLAG_PL};
     pmx_tic(c, PMX_T_GATHER);
     pl_launch<PL_CAP>(c, A, out, user, K2(s), K1(s + 1), D(s + 1), s);
     pmx_toc(c, PMX_T_GATHER);
     PMX_LAUNCH_CHECK();
-    // a tile overflowed: redo the step exactly (skipped on the device otherwise)
-    if ((rc = pmx_fill_u32(c, c->pl_count[B], nt + 1, 0u, c->flags))) return rc;
+    // a tile overflowed: redo the move exactly, by the counts of the pass
+    // (skipped on the device otherwise)
+    const PlOut redo = {c->pl[B], c->tile_cap, c->pl_start[B], c->flags + PMX_FLAG_PL};
     pmx_tic(c, PMX_T_BIN);
-    pl_launch<PL_COUNT>(c, A, out, user, K2(s), K1(s + 1), D(s + 1), s);
-    PMX_LAUNCH_CHECK();
-    if ((rc = pmx_scan_exclusive(c, c->pl_count[B], c->pl_start[B], nt + 1, c->flags))) return rc;
-    pl_launch<PL_WRITE>(c, A, out, user, K2(s), K1(s + 1), D(s + 1), s);
+    if ((rc = pmx_tile_exact(c, c->pl_count[B], c->pl_start[B], 1, PMX_FLAG_PL))) return rc;
+    pl_launch<PL_WRITE>(c, A, redo, user, K2(s), K1(s + 1), D(s + 1), s);
     pmx_toc(c, PMX_T_BIN);
     PMX_LAUNCH_CHECK();
     A = B;
@@ -533,19 +517,19 @@ __device__ __forceinline__ void al_put(const AState& st, uint32_t slot, float4 s
 // Writes particle i (after the first reverse kick and drift) with its
 // cotangents to slot start[ptile[i]] + prank[i] of st; |vel_cot| maxima per
 // channel to vmax.
-__global__ void __launch_bounds__(PMX_TPB)
+__global__ void __launch_bounds__(KD_ADJ_TPB)
     al_fill_k(const int16_t* __restrict__ pmid, const float* __restrict__ disp,
               const float* __restrict__ vel, const float* __restrict__ disp_cot,
               const float* __restrict__ vel_cot, long long n, MeshGeom g,
               const uint32_t* __restrict__ ptile, const uint32_t* __restrict__ prank,
               const uint32_t* __restrict__ start, AState st, float* __restrict__ vmax) {
-  constexpr int T3 = 3 * PMX_TPB;
+  constexpr int TPB = KD_ADJ_TPB, T3 = 3 * TPB;
   __shared__ __align__(16) float sh[4 * T3];  // disp | vel | disp_cot | vel_cot
   __shared__ __align__(16) int16_t sp[T3];
-  const long long b0 = (long long)blockIdx.x * PMX_TPB;
-  const int cnt = (int)(n - b0 < PMX_TPB ? n - b0 : PMX_TPB);
-  pmx_stage_in3<4, PMX_TPB>(sh, {{disp, vel, disp_cot, vel_cot}}, b0, cnt);
-  pmx_stage_pmid<PMX_TPB>(sp, pmid, b0, cnt);
+  const long long b0 = (long long)blockIdx.x * TPB;
+  const int cnt = (int)(n - b0 < TPB ? n - b0 : TPB);
+  pmx_stage_in3<4, TPB>(sh, {{disp, vel, disp_cot, vel_cot}}, b0, cnt);
+  pmx_stage_pmid<TPB>(sp, pmid, b0, cnt);
   __syncthreads();
   const int q = threadIdx.x;
   float vm[3] = {0.f, 0.f, 0.f};
@@ -577,8 +561,6 @@ struct AlOut {
   AState st;
   uint32_t* count;
   const uint32_t* start;
-  uint32_t* ptile;
-  uint32_t* prank;
   uint32_t* flag;
 };
 
@@ -610,7 +592,7 @@ __global__ void __launch_bounds__(AL_TPB) __attribute__((amdgpu_waves_per_eu(4))
               const float* __restrict__ F2, const float* __restrict__ R, float val, float kp,
               float ka, float dd, const float* __restrict__ snap, AlOut out, AlUser user,
               float* __restrict__ vmax, double* __restrict__ pf, double* __restrict__ pd) {
-  if ((MODE == PL_COUNT || MODE == PL_WRITE) && out.flag[0] == 0u) return;
+  if (MODE == PL_WRITE && out.flag[0] == 0u) return;
   extern __shared__ float sh[];
   __shared__ uint32_t s_cnt[27], s_base[27];
   double fsum = 0, dsum = 0;
@@ -727,21 +709,8 @@ __global__ void __launch_bounds__(AL_TPB) __attribute__((amdgpu_waves_per_eu(4))
 #pragma unroll
         for (int u = 0; u < AL_U; ++u) {
           const uint32_t q = q0 + u * AL_TPB + threadIdx.x;
-          if (q < cnt)
-            al_put(out.st, out.start[out.ptile[start + q]] + out.prank[start + q], n0[u], n1[u],
-                   m0[u], m1[u]);
-        }
-        continue;
-      }
-      if (MODE == PL_COUNT) {
-#pragma unroll
-        for (int u = 0; u < AL_U; ++u) {
-          const uint32_t q = q0 + u * AL_TPB + threadIdx.x;
           const uint32_t r = agg_slot(out.count, nt[u], q < cnt);
-          if (q < cnt) {
-            out.ptile[start + q] = nt[u];
-            out.prank[start + q] = r;
-          }
+          if (q < cnt) al_put(out.st, out.start[nt[u]] + r, n0[u], n1[u], m0[u], m1[u]);
         }
         continue;
       }
@@ -770,7 +739,7 @@ __global__ void __launch_bounds__(AL_TPB) __attribute__((amdgpu_waves_per_eu(4))
       }
     }
   };
-  if (MODE == PL_COUNT || MODE == PL_WRITE) {
+  if (MODE == PL_WRITE) {
     const unsigned ntl = (unsigned)tg.ntx * tg.nty * tg.ntz;
     for (unsigned tb = blockIdx.x; tb < ntl; tb += gridDim.x) {
       tile((int)pmx_xcd_block(tb, ntl));
@@ -793,7 +762,7 @@ static void al_launch(pmx_ctx* c, int src, float val, float kp, float ka, float 
   const MeshGeom g = pmx_geom_padded(c);
   const TileGeom& tg = c->tg;
   const size_t lds = (size_t)4 * (tg.tx + 1) * (tg.ty + 1) * (tg.tz + 1) * sizeof(float);
-  const bool rebin = MODE == PL_COUNT || MODE == PL_WRITE;
+  const bool rebin = MODE == PL_WRITE;
   const unsigned grid = rebin && c->ntiles > PL_REBIN_GRID ? PL_REBIN_GRID : (unsigned)c->ntiles;
 #define AL_LAUNCH(F)                                                                            \
   al_step_k<MODE, F><<<grid, AL_TPB, lds, c->stream>>>(                                          \
@@ -854,7 +823,7 @@ extern "C" int pmx_nbody_steps_adj(pmx_ctx* c, const int16_t* pmid, float* disp,
   if ((rc = pmx_ensure_adj_state(c, nsteps))) return rc;
   PMX_REQUIRE(c->rec_cap < (1LL << 32) - 1, "pmx_nbody_steps_adj: too many particles");
   const long long nt = c->ntiles;
-  const unsigned nb1 = pmx_blocks(n);
+  const unsigned nb1 = pmx_kd_adj_blocks(n);
   if ((rc = pmx_ensure_red(c, nb1 > 2 * nt ? (long long)nb1 : 2 * nt))) return rc;
   if ((rc = pmx_ensure_halo(c, 3))) return rc;
   if ((rc = pmx_ensure_scan(c, nt + 1))) return rc;
@@ -878,7 +847,7 @@ extern "C" int pmx_nbody_steps_adj(pmx_ctx* c, const int16_t* pmid, float* disp,
   if (rc) return rc;
   if ((rc = pmx_fill_u32(c, vmax_u, 3, 0u))) return rc;
   pmx_tic(c, PMX_T_FILL);
-  al_fill_k<<<nb1, PMX_TPB, 0, c->stream>>>(pmid, disp, vel, disp_cot, vel_cot, n, g, c->pkey,
+  al_fill_k<<<nb1, KD_ADJ_TPB, 0, c->stream>>>(pmid, disp, vel, disp_cot, vel_cot, n, g, c->pkey,
                                             c->prank, c->pl_start[A], c->al[A], c->vmax);
   pmx_toc(c, PMX_T_FILL);
   PMX_LAUNCH_CHECK();
@@ -909,14 +878,11 @@ extern "C" int pmx_nbody_steps_adj(pmx_ctx* c, const int16_t* pmid, float* disp,
     }
     const int B = 1 - A;
     pmx_tic(c, PMX_T_SCAN);
-    pl_caps_k<<<pmx_blocks(nt + 1), PMX_TPB, 0, c->stream>>>(c->pl_count[A], c->tile_cap,
-                                                             c->pl_count[B], nt, c->flags);
-    PMX_LAUNCH_CHECK();
-    rc = pmx_scan_exclusive(c, c->tile_cap, c->pl_start[B], nt + 1);
+    rc = pmx_tile_caps(c, c->pl_count[A], c->pl_count[B], c->pl_start[B], 0, PMX_FLAG_PL);
     pmx_toc(c, PMX_T_SCAN);
     if (rc) return rc;
     if ((rc = pmx_fill_u32(c, vmax_u, 3, 0u))) return rc;
-    const AlOut out = {c->al[B], c->pl_count[B], c->pl_start[B], c->pkey, c->prank, c->flags};
+    const AlOut out = {c->al[B], c->pl_count[B], c->pl_start[B], c->flags + PMX_FLAG_PL};
     const float* snap = s + 2 == nsteps ? disp_snap : nullptr;
     pmx_tic(c, PMX_T_GRADG);
     al_launch<PL_CAP>(c, A, val, kb[s], ka[s + 1], d[s + 1], snap, out, user);
@@ -924,13 +890,12 @@ extern "C" int pmx_nbody_steps_adj(pmx_ctx* c, const int16_t* pmid, float* disp,
     PMX_LAUNCH_CHECK();
     if ((rc = pmx_red_reduce_to(c, 0, nt, c->al_dots + 2 * s + 1))) return rc;
     if ((rc = pmx_red_reduce_to(c, nt, nt, c->al_dots + 2 * (s + 1)))) return rc;
-    // a tile overflowed: redo the move exactly (skipped on the device otherwise)
-    if ((rc = pmx_fill_u32(c, c->pl_count[B], nt + 1, 0u, c->flags))) return rc;
+    // a tile overflowed: redo the move exactly, by the counts of the pass
+    // (skipped on the device otherwise)
+    const AlOut redo = {c->al[B], c->tile_cap, c->pl_start[B], c->flags + PMX_FLAG_PL};
     pmx_tic(c, PMX_T_BIN);
-    al_launch<PL_COUNT>(c, A, val, kb[s], ka[s + 1], d[s + 1], snap, out, user);
-    PMX_LAUNCH_CHECK();
-    if ((rc = pmx_scan_exclusive(c, c->pl_count[B], c->pl_start[B], nt + 1, c->flags))) return rc;
-    al_launch<PL_WRITE>(c, A, val, kb[s], ka[s + 1], d[s + 1], snap, out, user);
+    if ((rc = pmx_tile_exact(c, c->pl_count[B], c->pl_start[B], 1, PMX_FLAG_PL))) return rc;
+    al_launch<PL_WRITE>(c, A, val, kb[s], ka[s + 1], d[s + 1], snap, redo, user);
     pmx_toc(c, PMX_T_BIN);
     PMX_LAUNCH_CHECK();
     A = B;

@@ -44,7 +44,7 @@ __device__ __forceinline__ bool load_block(const int16_t* __restrict__ pmid,
 // interleaved.  One particle a thread in the caller's order, whose neighbours
 // read neighbouring cells; an XCD takes a contiguous eighth of the particles,
 // so the rows they share stay in its L2.  Bound by those reads: 16.8 M
-// particles on a 256^3 mesh 1028 -> 149 us against the any-geometry kernel,
+// particles on a 256^3 mesh take 251 us, 1028 in the any-geometry kernel,
 // whose run-time corner loops keep their arrays in scratch memory.
 template <int NC>
 __global__ void __launch_bounds__(PMX_TPB)
@@ -77,8 +77,9 @@ __global__ void __launch_bounds__(PMX_TPB)
 // Position and value cotangents (scatter.py:86-121, gather.py:80-116) of
 // values v (per particle, or vs) against a mesh f: disp_cot = sum_j (f[c_j].v)
 // grad w_j / cell and, when wanted, val_cot = sum_j f[c_j] w_j.  Laid out as
-// the gather; disp_cot leaves through LDS in 16-byte stores.  One channel,
-// 16.8 M particles on a 512^3 mesh: 1543 us in the any-geometry kernel.
+// the gather; disp_cot leaves through LDS in 16-byte stores.  16.8 M
+// particles, one channel on a 512^3 mesh: 415 us (1543 in the any-geometry
+// kernel); three channels with both cotangents on 256^3: 631 us (3263).
 template <int NC>
 __global__ void __launch_bounds__(PMX_TPB)
     cic_adj_k(MeshGeom g, const int16_t* __restrict__ pmid, const float* __restrict__ disp,
@@ -140,7 +141,8 @@ __global__ void __launch_bounds__(PMX_TPB)
 // be of any magnitude, infinite or NaN, and each contribution keeps its
 // float32 rounding.  LDS takes float64 adds about as fast as 64-bit integer
 // ones.  The any-geometry kernel is bound by its global float32 atomics, 24
-// per particle: 16.8 M particles, three channels on a 256^3 mesh, 17.5 ms.
+// per particle: 16.8 M particles, three channels on a 256^3 mesh, 17.5 ms
+// against 1.0 ms here; one channel 0.5 ms.
 // Three channels take 118 KB of LDS, one workgroup of 1024 threads per CU;
 // one channel 39 KB, four of 512.
 template <int NC>
