@@ -13,6 +13,8 @@
 // inverse ends with y (strided) and z c2r (rows).
 #include "pmx_internal.h"
 
+#include <algorithm>
+
 #define FFT_CAP 8192                 // complex values per strided workgroup, fixed lengths
 #define PFFT_CAP 4096                // Poisson x pass (8 columns of 512, three 40 KB workgroups
                                      // per CU; 16 columns measured slower)
@@ -657,9 +659,13 @@ __device__ __forceinline__ unsigned pass_block(unsigned lin, unsigned nb, int re
 // ------------------------------------------------------------ z passes --
 // Up to three meshes of one row pass: block b works on field b / nblk, in the
 // block order of pass_block (rev per field).  fold: the halo shells of field
-// i lie i * hstride floats into the halo.
+// i lie i * hstride floats into the halo.  o: the real side, rows of ors
+// floats that an r2c reads and a c2r writes (f itself when in place; dense
+// caller meshes save the copy into or out of the padded layout).
 struct RowFields {
   float* f[3];
+  float* o[3];
+  int ors;
   int rev[3];
   unsigned nblk;
   long long hstride;
@@ -671,6 +677,7 @@ __device__ __forceinline__ int row_field(unsigned nblk, int rev0, int rev1, int 
 }
 #define PMX_ROW_FIELD(rf, blk) row_field((rf).nblk, (rf).rev[0], (rf).rev[1], (rf).rev[2], blk)
 #define PMX_ROW_DATA(rf, i) ((i) == 0 ? (rf).f[0] : ((i) == 1 ? (rf).f[1] : (rf).f[2]))
+#define PMX_ROW_REAL(rf, i) ((i) == 0 ? (rf).o[0] : ((i) == 1 ? (rf).o[1] : (rf).o[2]))
 
 // In-place r2c of padded rows by a length-n2 complex FFT (odd n2; even ones
 // take z_r2c_half_k): two rows a and b are transformed as z = a + i b, and
@@ -688,6 +695,7 @@ __global__ void __launch_bounds__(GEN_MAXTPB, 4) z_r2c_k(RowFields rf, long long
   unsigned blk;
   const int field = PMX_ROW_FIELD(rf, blk);
   float* data = PMX_ROW_DATA(rf, field);
+  const float* real = PMX_ROW_REAL(rf, field);
   const long long row0 = (long long)blk * 2 * P;
   const int nr = (int)((nrows - row0) < 2 * P ? (nrows - row0) : 2 * P);
   const int np = (nr + 1) / 2;
@@ -697,8 +705,8 @@ __global__ void __launch_bounds__(GEN_MAXTPB, 4) z_r2c_k(RowFields rf, long long
       np * n2,
       [&](int idx) {
         const int p = dn(idx), j = idx - p * n2;
-        const float* r = data + (row0 + 2 * p) * rs + j;
-        float2 v = make_float2(r[0], 2 * p + 1 < nr ? r[rs] : 0.f);
+        const float* r = real + (row0 + 2 * p) * rf.ors + j;
+        float2 v = make_float2(r[0], 2 * p + 1 < nr ? r[rf.ors] : 0.f);
         if (PRE) {
           v.x = v.x - 1.f;
           v.x = v.x * coef;
@@ -740,7 +748,8 @@ __global__ void __launch_bounds__(GEN_MAXTPB, 4) z_c2r_k(RowFields rf, long long
   float2* stw = s + lds_elems(ROWS, n2, P);
   unsigned blk;
   const int field = PMX_ROW_FIELD(rf, blk);
-  float* data = PMX_ROW_DATA(rf, field);
+  const float* data = PMX_ROW_DATA(rf, field);
+  float* real = PMX_ROW_REAL(rf, field);
   const long long row0 = (long long)blk * 2 * P;
   const int nr = (int)((nrows - row0) < 2 * P ? (nrows - row0) : 2 * P);
   const int np = (nr + 1) / 2;
@@ -769,9 +778,9 @@ __global__ void __launch_bounds__(GEN_MAXTPB, 4) z_c2r_k(RowFields rf, long long
   for (int idx = threadIdx.x; idx < np * n2; idx += tpb<GEN_TPB>()) {
     const int p = dn(idx), j = idx - p * n2;
     const float2 v = s[lidx<ROWS>(p, j, n2, P)];
-    float* r = data + (row0 + 2 * p) * rs + j;
+    float* r = real + (row0 + 2 * p) * rf.ors + j;
     r[0] = v.x * scale;
-    if (2 * p + 1 < nr) r[rs] = v.y * scale;
+    if (2 * p + 1 < nr) r[rf.ors] = v.y * scale;
   }
 }
 
@@ -932,6 +941,8 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
   const int np = LH ? PC : (int)((nrows - row0) < P ? (nrows - row0) : P);
   const int rsc = rs / 2;
   float2* blk = reinterpret_cast<float2*>(PMX_ROW_DATA(rf, field)) + row0 * rsc;
+  const int orc = rf.ors / 2;
+  const float2* src = reinterpret_cast<const float2*>(PMX_ROW_REAL(rf, field)) + row0 * orc;
   const int total = np * H;
   if (FOLD) fi.halo += field * rf.hstride;
   stage_twiddles<TPB>(stw, tw, 2 * H);
@@ -952,7 +963,7 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
     for (int it = 0; it < MAXV; ++it) {
       const int idx = threadIdx.x + it * tpb<TPB>();
       const int p = rsp.row(idx);
-      if (idx < total) r[it] = blk[__umul24(p, rsc) + rsp.col(idx, p)];
+      if (idx < total) r[it] = src[__umul24(p, orc) + rsp.col(idx, p)];
     }
     if (FOLD) {
       if ((int)threadIdx.x < PC * (H >> 3)) {
@@ -1019,11 +1030,12 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
   float2* stw = s + lds_elems(ROWS, H, P);
   unsigned bk;
   const int field = PMX_ROW_FIELD(rf, bk);
-  float* data = PMX_ROW_DATA(rf, field);
   const long long row0 = (long long)bk * P;
   const int np = LH ? PC : (int)((nrows - row0) < P ? (nrows - row0) : P);
   const int rsc = rs / 2;
-  float2* blk = reinterpret_cast<float2*>(data) + row0 * rsc;
+  const float2* blk = reinterpret_cast<const float2*>(PMX_ROW_DATA(rf, field)) + row0 * rsc;
+  const int orc = rf.ors / 2;
+  float2* dst = reinterpret_cast<float2*>(PMX_ROW_REAL(rf, field)) + row0 * orc;
   const int total = np * H;
   stage_twiddles<TPB>(stw, tw, 2 * H);
   // X[k] and X[H-k] per thread: both loads of the batch are issued first
@@ -1071,7 +1083,7 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
     const int idx = threadIdx.x + it * tpb<TPB>();
     const int p = rsp.row(idx);
     if (idx < total)
-      blk[__umul24(p, rsc) + rsp.col(idx, p)] = make_float2(r[it].x * scale, r[it].y * scale);
+      dst[__umul24(p, orc) + rsp.col(idx, p)] = make_float2(r[it].x * scale, r[it].y * scale);
   }
 }
 
@@ -1080,6 +1092,12 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
 struct Fields3 {
   float2* f[3];
   int rev;
+};
+// One side of a strided pass: element j of pencil (o, c) of field i at
+// f[i] + o * os + j * es + c.
+struct Side3 {
+  float2* f[3];
+  long long es, os;
 };
 
 // Block coordinates of a (gx, gy, gz) grid after the XCD-contiguous remap
@@ -1110,14 +1128,14 @@ __device__ __forceinline__ ColMap col_map(int lB) {
   return m;
 }
 
-// In-place FFT along a strided axis of a complex (outer, n, ncol) view:
-// element j of pencil (o, c) is at o*ostride + j*es + c.  A workgroup takes
-// B consecutive columns, so each of its loads is B contiguous float2.
+// FFT along a strided axis of complex (outer, n, ncol) views, from one side
+// to the other (the same one in place).  A workgroup takes B consecutive
+// columns, so each of its loads is B contiguous float2.
 // LDS: the n x B block, then the n-entry twiddle table.  LN > 0 fixes
 // n = 2^LN and B = ct_cols(LN, FFT_CAP) at compile time.
 template <int DIR, bool POW2, int LN>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) : GEN_MAXTPB, 4) strided_fft_k(Fields3 fl, int n_, long long es,
-                                                         long long ostride, int ncol, int B_,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) : GEN_MAXTPB, 4) strided_fft_k(Side3 si, Side3 so, int rev,
+                                                         int n_, int ncol, int B_,
                                                          const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, FFT_CAP) : 1;
@@ -1128,14 +1146,14 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) :
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
   float2* stw = s + n * B;
   int bx, by, bz;
-  xcd_block3(bx, by, bz, fl.rev);
+  xcd_block3(bx, by, bz, rev);
   const int c0 = bx * B;
   const int nb = ncol - c0 < B ? ncol - c0 : B;
   const ColMap cm = col_map<TPB>(lB);
   const bool live = cm.b < nb;
-  float2* g = (bz == 0 ? fl.f[0] : (bz == 1 ? fl.f[1] : fl.f[2])) + (long long)by * ostride + c0 +
-              cm.b + (long long)cm.j0 * es;
-  const long long gs = (long long)cm.js * es;
+  const float2* g = (bz == 0 ? si.f[0] : (bz == 1 ? si.f[1] : si.f[2])) + (long long)by * si.os +
+                    c0 + cm.b + (long long)cm.j0 * si.es;
+  const long long gs = (long long)cm.js * si.es;
   stage_twiddles<TPB>(stw, tw, n);
   float2 r[MAXV];
 #pragma unroll
@@ -1151,9 +1169,12 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) :
 #pragma unroll
   for (int it = 0; it < MAXV; ++it)
     if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * tpb<TPB>()];
+  float2* d = (bz == 0 ? so.f[0] : (bz == 1 ? so.f[1] : so.f[2])) + (long long)by * so.os + c0 +
+              cm.b + (long long)cm.j0 * so.es;
+  const long long ds = (long long)cm.js * so.es;
 #pragma unroll
   for (int it = 0; it < MAXV; ++it)
-    if (live && cm.j0 + it * cm.js < n) g[it * gs] = r[it];
+    if (live && cm.j0 + it * cm.js < n) d[it * ds] = r[it];
 }
 
 struct KTab {
@@ -1520,6 +1541,18 @@ __global__ void copy_rows_k(float* __restrict__ dst, int dst_rs, const float* __
   }
 }
 
+// copies n0*n1 rows of ncols floats between row strides (ncols <= 0: n2)
+int pmx_copy_rows(pmx_ctx* c, float* dst, int dst_rs, const float* src, int src_rs, int ncols) {
+  if (ncols <= 0) ncols = c->n[2];
+  long long nrows = (long long)c->n[0] * c->n[1];
+  long long total = nrows * ncols;
+  unsigned nblk = (unsigned)((total + PMX_TPB - 1) / PMX_TPB);
+  if (nblk > 65536u * 4) nblk = 65536u * 4;
+  copy_rows_k<<<nblk, PMX_TPB, 0, c->stream>>>(dst, dst_rs, src, src_rs, nrows, ncols);
+  PMX_LAUNCH_CHECK();
+  return PMX_OK;
+}
+
 // ------------------------------------------------------------ drivers --
 #define PMX_LDS_MAX (160 * 1024)     // LDS a gfx950 workgroup may allocate
 
@@ -1624,29 +1657,39 @@ int pmx_fold_deferrable(const pmx_ctx* c) {
   return r.lh > 0 && c->n[1] % r.P == 0;
 }
 
-static RowFields row_fields(float* const* f, int nf, const int* rev, unsigned nblk, long long hstride) {
+static RowFields row_fields(const pmx_ctx* c, float* const* f, int nf, const int* rev, unsigned nblk,
+                            long long hstride, float* const* real, int ors) {
   RowFields rf;
   for (int i = 0; i < 3; ++i) {
     rf.f[i] = f[i < nf ? i : 0];
+    rf.o[i] = real ? real[i < nf ? i : 0] : rf.f[i];
     rf.rev[i] = rev[i < nf ? i : 0];
   }
+  rf.ors = real ? ors : c->rs;
   rf.nblk = nblk;
   rf.hstride = hstride;
   return rf;
 }
 
-// In-place r2c of nf padded real meshes; pre applies (x - 1) * coef.  With
-// halo (pmx_fold_deferrable must hold; one channel's shells per mesh) the
-// deposit's fold is added on load.
-int pmx_fft_r2c_inplace(pmx_ctx* c, float* const* f, int nf, int pre, float coef, const float* halo,
-                        const int* rev) {
+// Whether a row pass can read or write a dense (n0, n1, n2) mesh in place of
+// the padded layout: even n2 moves the rows as float2.
+static bool dense_rows_ok(const pmx_ctx* c, const void* p) {
+  return (c->n[2] & 1) || (reinterpret_cast<uintptr_t>(p) & 7) == 0;
+}
+
+// r2c of nf padded real meshes in place (real: from meshes of ors floats a
+// row); pre applies (x - 1) * coef.  With halo (pmx_fold_deferrable must
+// hold; one channel's shells per mesh) the deposit's fold is added on load.
+int pmx_fft_r2c_rows(pmx_ctx* c, float* const* f, int nf, int pre, float coef, const float* halo,
+                     const int* rev, const float* const* real, int ors) {
   const long long nrows = (long long)c->n[0] * c->n[1];
   const int n2 = c->n[2];
   const RowPlan r = row_plan(n2, nrows);
   if (int rc = fft_fits("z r2c", n2, r.len * r.P, GEN_CAP, r.lds)) return rc;
   const unsigned nblk = (unsigned)((nrows + r.rows - 1) / r.rows);
   const FoldIn fi = {halo, c->tg.shell, c->tg.ntx, c->tg.nty, c->tg.ntz, c->n[1]};
-  const RowFields rf = row_fields(f, nf, rev, nblk, c->ntiles * c->tg.shell);
+  const RowFields rf = row_fields(c, f, nf, rev, nblk, c->ntiles * c->tg.shell,
+                                  const_cast<float* const*>(real), ors);
   const float* fc = pre ? c->dfac : nullptr;
   PMX_REQUIRE(!halo || pmx_fold_deferrable(c), "z r2c: no fold on load for this mesh");
   pmx_tic(c, PMX_T_ZR2C);
@@ -1687,14 +1730,16 @@ int pmx_fft_r2c_inplace(pmx_ctx* c, float* const* f, int nf, int pre, float coef
   return PMX_OK;
 }
 
-// In-place c2r of nf padded meshes with a final scale.
-int pmx_fft_c2r_inplace(pmx_ctx* c, float* const* f, int nf, float scale, const int* rev) {
+// c2r of nf padded meshes with a final scale, in place (real: to meshes of
+// ors floats a row).
+int pmx_fft_c2r_rows(pmx_ctx* c, float* const* f, int nf, float scale, const int* rev,
+                     float* const* real, int ors) {
   const long long nrows = (long long)c->n[0] * c->n[1];
   const int n2 = c->n[2];
   const RowPlan r = row_plan(n2, nrows);
   if (int rc = fft_fits("z c2r", n2, r.len * r.P, GEN_CAP, r.lds)) return rc;
   const unsigned nblk = (unsigned)((nrows + r.rows - 1) / r.rows);
-  const RowFields rf = row_fields(f, nf, rev, nblk, 0);
+  const RowFields rf = row_fields(c, f, nf, rev, nblk, 0, real, ors);
   const unsigned grid = nblk * (unsigned)nf;
   pmx_tic(c, PMX_T_ZC2R);
 #define C2R(L, SM, P2)                                                                         \
@@ -1722,6 +1767,13 @@ int pmx_fft_c2r_inplace(pmx_ctx* c, float* const* f, int nf, float scale, const 
   return PMX_OK;
 }
 
+int pmx_fft_r2c_inplace(pmx_ctx* c, float* const* f, int nf, int pre, float coef, const float* halo,
+                        const int* rev) {
+  return pmx_fft_r2c_rows(c, f, nf, pre, coef, halo, rev, nullptr, 0);
+}
+int pmx_fft_c2r_inplace(pmx_ctx* c, float* const* f, int nf, float scale, const int* rev) {
+  return pmx_fft_c2r_rows(c, f, nf, scale, rev, nullptr, 0);
+}
 // One mesh.
 int pmx_fft_r2c_inplace(pmx_ctx* c, float* buf, int pre, float coef, const float* halo, int rev) {
   return pmx_fft_r2c_inplace(c, &buf, 1, pre, coef, halo, &rev);
@@ -1729,25 +1781,43 @@ int pmx_fft_r2c_inplace(pmx_ctx* c, float* buf, int pre, float coef, const float
 int pmx_fft_c2r_inplace(pmx_ctx* c, float* buf, float scale, int rev) {
   return pmx_fft_c2r_inplace(c, &buf, 1, scale, &rev);
 }
+// One dense caller mesh to or from padded rows.
+static int r2c_dense(pmx_ctx* c, float2* f, const float* in, int pre = 0, float coef = 0.f, int rev = 0) {
+  float* b = reinterpret_cast<float*>(f);
+  if (!dense_rows_ok(c, in)) {
+    if (int rc = pmx_copy_rows(c, b, c->rs, in, c->n[2])) return rc;
+    return pmx_fft_r2c_inplace(c, b, pre, coef, nullptr, rev);
+  }
+  return pmx_fft_r2c_rows(c, &b, 1, pre, coef, nullptr, &rev, &in, c->n[2]);
+}
+static int c2r_dense(pmx_ctx* c, float* out, float2* f, float scale, int rev = 0) {
+  float* b = reinterpret_cast<float*>(f);
+  if (!dense_rows_ok(c, out)) {
+    if (int rc = pmx_fft_c2r_inplace(c, b, scale, rev)) return rc;
+    return pmx_copy_rows(c, out, c->n[2], b, c->rs);
+  }
+  return pmx_fft_c2r_rows(c, &b, 1, scale, &rev, &out, c->n[2]);
+}
 
-// axis 1 (y) or axis 0 (x) complex FFT of nf fields in place
-int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int rev) {
-  Fields3 fl;
-  for (int i = 0; i < 3; ++i) fl.f[i] = f[i < nf ? i : 0];
-  fl.rev = rev;
+// The axis pencils of spectra whose rows are row complex values long.
+static Side3 strided_side(const pmx_ctx* c, float2* const* f, int nf, int axis, int row) {
+  Side3 s;
+  for (int i = 0; i < 3; ++i) s.f[i] = f[i < nf ? i : 0];
+  const long long plane = (long long)c->n[1] * row;
+  s.es = axis == 1 ? row : plane;
+  s.os = axis == 1 ? plane : row;
+  return s;
+}
+
+// axis 1 (y) or axis 0 (x) complex FFT of nf spectra, from src (rows of
+// srow) to dst (rows of drow)
+static int strided_from_to(pmx_ctx* c, float2* const* src, int srow, float2* const* dst, int drow,
+                           int nf, int axis, int dir, int rev) {
+  const Side3 si = strided_side(c, src, nf, axis, srow);
+  const Side3 so = strided_side(c, dst, nf, axis, drow);
   const int n = c->n[axis];
   const int ncol = c->n2h;
-  long long es, ostride;
-  unsigned nouter;
-  if (axis == 1) {
-    es = c->n2p;
-    ostride = (long long)c->n[1] * c->n2p;
-    nouter = c->n[0];
-  } else {
-    es = (long long)c->n[1] * c->n2p;
-    ostride = c->n2p;
-    nouter = c->n[1];
-  }
+  const unsigned nouter = axis == 1 ? c->n[0] : c->n[1];
   const int ln = ct_log2(n);
   const int B = ln ? ct_cols(ln, FFT_CAP) : gen_cols(n, ncol, (long long)nouter * nf);
   const int tpb = ln ? ct_tpb(ln, B, FFT_V) : gen_tpb(n * B);
@@ -1759,18 +1829,23 @@ int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int
   pmx_tic(c, cls);
 #define STRIDED(L)                                                                                  \
   if (dir < 0 && (L || p2))                                                                         \
-    strided_fft_k<-1, true, L><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]); \
+    strided_fft_k<-1, true, L><<<grid, tpb, lds, c->stream>>>(si, so, rev, n, ncol, B, c->tw[axis]); \
   else if (dir < 0)                                                                                 \
-    strided_fft_k<-1, false, 0><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]); \
+    strided_fft_k<-1, false, 0><<<grid, tpb, lds, c->stream>>>(si, so, rev, n, ncol, B, c->tw[axis]); \
   else if (L || p2)                                                                                 \
-    strided_fft_k<1, true, L><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis]);  \
+    strided_fft_k<1, true, L><<<grid, tpb, lds, c->stream>>>(si, so, rev, n, ncol, B, c->tw[axis]);  \
   else                                                                                              \
-    strided_fft_k<1, false, 0><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, c->tw[axis])
+    strided_fft_k<1, false, 0><<<grid, tpb, lds, c->stream>>>(si, so, rev, n, ncol, B, c->tw[axis])
   PMX_CT_SWITCH(ln, STRIDED);
 #undef STRIDED
   pmx_toc(c, cls);
   PMX_LAUNCH_CHECK();
   return PMX_OK;
+}
+
+// the same in place on spectra of the padded layout
+int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int rev) {
+  return strided_from_to(c, f, c->n2p, f, c->n2p, nf, axis, dir, rev);
 }
 
 static KTab ktab(const pmx_ctx* c) {
@@ -1897,26 +1972,22 @@ int pmx_poisson_adj_bufs(pmx_ctx* c, float2* const* f, float scale_out, int defe
   return PMX_OK;
 }
 
-// copies n0*n1 rows of ncols floats between row strides (ncols <= 0: n2)
-int pmx_copy_rows(pmx_ctx* c, float* dst, int dst_rs, const float* src, int src_rs, int ncols) {
-  if (ncols <= 0) ncols = c->n[2];
-  long long nrows = (long long)c->n[0] * c->n[1];
-  long long total = nrows * ncols;
-  unsigned nblk = (unsigned)((total + PMX_TPB - 1) / PMX_TPB);
-  if (nblk > 65536u * 4) nblk = 65536u * 4;
-  copy_rows_k<<<nblk, PMX_TPB, 0, c->stream>>>(dst, dst_rs, src, src_rs, nrows, ncols);
-  PMX_LAUNCH_CHECK();
-  return PMX_OK;
-}
+// Dense complex meshes are rows of n2h float2.
+static bool dense_spec_ok(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; }
 
+// The dense caller meshes are the first pass's source and the last pass's
+// destination, which saves two copies (the one r2c in white noise to 2LPT at
+// 256^3: 2475 -> 2403 us for the whole).  Pointers that the passes' float2
+// accesses cannot take still go through the copies.
 extern "C" int pmx_rfftn(pmx_ctx* c, const float* in, float* out_c) {
   PMX_ENTRY(c);
   PMX_REQUIRE(c && in && out_c, "pmx_rfftn: NULL argument");
   int rc;
-  float2* f[3] = {c->cbuf[0], c->cbuf[1], c->cbuf[2]};
-  if ((rc = pmx_copy_rows(c, (float*)f[0], c->rs, in, c->n[2]))) return rc;
-  if ((rc = pmx_fft_r2c_inplace(c, (float*)f[0], 0, 0.f))) return rc;
+  float2* f[1] = {c->cbuf[0]};
+  float2* o[1] = {reinterpret_cast<float2*>(out_c)};
+  if ((rc = r2c_dense(c, f[0], in))) return rc;
   if ((rc = pmx_fft_strided(c, f, 1, 1, -1))) return rc;
+  if (dense_spec_ok(out_c)) return strided_from_to(c, f, c->n2p, o, c->n2h, 1, 0, -1, 0);
   if ((rc = pmx_fft_strided(c, f, 1, 0, -1))) return rc;
   return pmx_copy_rows(c, out_c, 2 * c->n2h, (const float*)f[0], c->rs, 2 * c->n2h);
 }
@@ -1925,12 +1996,16 @@ extern "C" int pmx_irfftn(pmx_ctx* c, const float* in_c, float* out) {
   PMX_ENTRY(c);
   PMX_REQUIRE(c && in_c && out, "pmx_irfftn: NULL argument");
   int rc;
-  float2* f[3] = {c->cbuf[0], c->cbuf[1], c->cbuf[2]};
-  if ((rc = pmx_copy_rows(c, (float*)f[0], c->rs, in_c, 2 * c->n2h, 2 * c->n2h))) return rc;
-  if ((rc = pmx_fft_strided(c, f, 1, 0, 1))) return rc;
+  float2* f[1] = {c->cbuf[0]};
+  float2* in[1] = {reinterpret_cast<float2*>(const_cast<float*>(in_c))};
+  if (dense_spec_ok(in_c)) {
+    if ((rc = strided_from_to(c, in, c->n2h, f, c->n2p, 1, 0, 1, 0))) return rc;
+  } else {
+    if ((rc = pmx_copy_rows(c, (float*)f[0], c->rs, in_c, 2 * c->n2h, 2 * c->n2h))) return rc;
+    if ((rc = pmx_fft_strided(c, f, 1, 0, 1))) return rc;
+  }
   if ((rc = pmx_fft_strided(c, f, 1, 1, 1))) return rc;
-  if ((rc = pmx_fft_c2r_inplace(c, (float*)f[0], (float)(1.0 / (double)c->M)))) return rc;
-  return pmx_copy_rows(c, out, c->n[2], (const float*)f[0], c->rs);
+  return c2r_dense(c, out, f[0], (float)(1.0 / (double)c->M));
 }
 
 extern "C" int pmx_poisson_grad(pmx_ctx* c, const float* dens, float coef, float* grad) {
@@ -1964,17 +2039,25 @@ extern "C" int pmx_poisson_grad_adj(pmx_ctx* c, const float* grad_cot, float coe
 // F conj(G) in float32 (optionally deconvolved by sinc^-deconv per axis),
 // the weight N = 2 (1 on the kz = 0 and, for an even n2, Nyquist planes),
 // and the bin of |k| among the float64 edges (right: edge < k counts; else
-// edge <= k).  Each workgroup sums k N, Re P N, Im P N and N per bin in
-// float64 in LDS (atomic adds: their order within a workgroup is not
-// fixed) and writes its partials; a second kernel adds the partials in
-// workgroup order.
+// edge <= k).
+//
+// |k| and the bin are the same for the cells (+-kx, +-ky) of a kz, so a
+// thread takes such a group (1, 2 or 4 cells) at once, and L groups of
+// consecutive |ky| one after the other: their sums of k N, Re P N, Im P N and
+// N stay in registers (float64) until the bin changes and then go to the
+// workgroup's bins in LDS (float64 atomic adds: their order within a
+// workgroup is not fixed).  Lanes run along kz, so the loads are whole lines.
+// A second kernel adds the workgroups' partials, 32 threads to a sum.
+// 512^3, 28 bins: 168 us, 3.2 TB/s of spectrum read (more loads in flight, copies
+// of the bins in LDS and fewer edge searches changed nothing); one cell a
+// thread with three LDS atomics each took 1190 us, and the sums of the 1024
+// partials by one thread each 236 us (now 12).
 #define PS_TPB 256
 #define PS_BLOCKS 1024
+#define PS_RED 32
 
-__device__ __forceinline__ float ps_freq(int j, int n, bool rfft) {
-  const int jj = (!rfft && j >= (n + 1) / 2) ? j - n : j;
-  return (float)((double)jj / (double)n);
-}
+// |fftfreq| of the index of least magnitude j <= n/2
+__device__ __forceinline__ float ps_freq(int j, int n) { return (float)((double)j / (double)n); }
 
 __device__ __forceinline__ float ps_sinc(float x) {
   if (x == 0.f) return 1.f;
@@ -1982,78 +2065,136 @@ __device__ __forceinline__ float ps_sinc(float x) {
   return sinf(px) / px;
 }
 
+// F and, with CROSS, G: (n0, n1, n2p) spectra, n2h columns used.  nc1: chunks
+// of L |ky| values.
+template <bool CROSS>
 __global__ void __launch_bounds__(PS_TPB)
     powspec_bin_k(const float2* __restrict__ F, const float2* __restrict__ G, int n0, int n1,
                   int n2, int n2h, int n2p, const double* __restrict__ edges, int nedges, int right,
-                  int deconv, double* __restrict__ part) {
+                  int deconv, int L, int nc1, double* __restrict__ part) {
   extern __shared__ double ps_sh[];
   double* acc = ps_sh;                 // 4 * nedges
   double* e = ps_sh + 4 * nedges;      // nedges
+  const int h0 = n0 / 2 + 1, h1 = n1 / 2 + 1;
+  float* tfy = reinterpret_cast<float*>(e + nedges);  // |fy|, then sinc^-deconv
+  float* tsy = tfy + h1;
   for (int i = threadIdx.x; i < 4 * nedges; i += PS_TPB) acc[i] = 0.0;
   for (int i = threadIdx.x; i < nedges; i += PS_TPB) e[i] = edges[i];
+  for (int i = threadIdx.x; i < h1; i += PS_TPB) {
+    const float fy = ps_freq(i, n1);
+    tfy[i] = fy;
+    if (deconv) tsy[i] = powf(ps_sinc(fy), (float)-deconv);
+  }
   __syncthreads();
-  const long long total = (long long)n0 * n1 * n2h;
-  for (long long idx = (long long)blockIdx.x * PS_TPB + threadIdx.x; idx < total;
-       idx += (long long)gridDim.x * PS_TPB) {
-    const int kz = (int)(idx % n2h);
-    const long long r = idx / n2h;
-    const int ky = (int)(r % n1);
-    const int kx = (int)(r / n1);
-    const float2 f = F[((long long)kx * n1 + ky) * n2p + kz];
-    float pr, pi = 0.f;
-    if (G) {
-      const float2 gg = G[((long long)kx * n1 + ky) * n2p + kz];
-      pr = f.x * gg.x + f.y * gg.y;
-      pi = f.y * gg.x - f.x * gg.y;
-    } else {
-      pr = f.x * f.x + f.y * f.y;
-    }
-    const float fx = ps_freq(kx, n0, false), fy = ps_freq(ky, n1, false),
-                fz = ps_freq(kz, n2, true);
-    const float k = sqrtf((fx * fx + fy * fy) + fz * fz);
+  const unsigned total = (unsigned)h0 * nc1 * n2h;
+  for (unsigned u = blockIdx.x * PS_TPB + threadIdx.x; u < total; u += gridDim.x * PS_TPB) {
+    const unsigned r = u / (unsigned)n2h;
+    const int kz = (int)(u - r * n2h);
+    const int kx = (int)(r / (unsigned)nc1);
+    const int y0 = (int)(r - (unsigned)kx * nc1) * L;
+    const int y1 = y0 + L < h1 ? y0 + L : h1;
+    const bool x2 = kx != 0 && 2 * kx != n0;  // -kx is another cell
+    const float fx = ps_freq(kx, n0), fz = ps_freq(kz, n2);
+    float sx = 1.f, sz = 1.f;
     if (deconv) {
-      const float sx = powf(ps_sinc(fx), (float)-deconv);
-      const float sy = powf(ps_sinc(fy), (float)-deconv);
-      const float sz = powf(ps_sinc(fz), (float)-deconv);
-      pr = ((pr * sx) * sy) * sz;
-      pi = ((pi * sx) * sy) * sz;
+      sx = powf(ps_sinc(fx), (float)-deconv);
+      sz = powf(ps_sinc(fz), (float)-deconv);
     }
-    // number of edges below k (right) or at most k (left-inclusive bins)
-    const double kd = (double)k;
-    int lo = 0, hi = nedges;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      const bool below = right ? (e[mid] < kd) : (e[mid] <= kd);
-      if (below) lo = mid + 1;
-      else hi = mid;
-    }
-    if (lo >= nedges) continue;
     const float w = (kz == 0 || ((n2 & 1) == 0 && kz == n2 / 2)) ? 1.f : 2.f;
-    atomicAdd(&acc[lo], (double)(k * w));
-    atomicAdd(&acc[nedges + lo], (double)(pr * w));
-    if (G) atomicAdd(&acc[2 * nedges + lo], (double)(pi * w));
-    atomicAdd(&acc[3 * nedges + lo], (double)w);
+    const long long pa = (long long)kx * n1 * n2p + kz;
+    const long long pb = (long long)(x2 ? n0 - kx : kx) * n1 * n2p + kz;
+    int bin = nedges;
+    double ak = 0.0, ar = 0.0, ai = 0.0, an = 0.0;
+    auto flush = [&]() {
+      if (bin >= nedges) return;
+      atomicAdd(&acc[bin], ak);
+      atomicAdd(&acc[nedges + bin], ar);
+      if (CROSS) atomicAdd(&acc[2 * nedges + bin], ai);
+      atomicAdd(&acc[3 * nedges + bin], an);
+    };
+#pragma unroll 2
+    for (int ky = y0; ky < y1; ++ky) {
+      const bool y2 = ky != 0 && 2 * ky != n1;
+      const long long ra = (long long)ky * n2p, rb = (long long)(y2 ? n1 - ky : ky) * n2p;
+      const long long at[4] = {pa + ra, pa + rb, pb + ra, pb + rb};
+      float2 f[4], g[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bool on = ((q & 1) == 0 || y2) && ((q & 2) == 0 || x2);
+        f[q] = g[q] = make_float2(0.f, 0.f);
+        if (on) {
+          f[q] = F[at[q]];
+          if (CROSS) g[q] = G[at[q]];
+        }
+      }
+      const float fy = tfy[ky];
+      const float k = sqrtf((fx * fx + fy * fy) + fz * fz);
+      // number of edges below k (right) or at most k (left-inclusive bins)
+      const double kd = (double)k;
+      int lo = 0, hi = nedges;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        const bool below = right ? (e[mid] < kd) : (e[mid] <= kd);
+        if (below) lo = mid + 1;
+        else hi = mid;
+      }
+      if (lo != bin) {
+        flush();
+        bin = lo;
+        ak = ar = ai = an = 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (((q & 1) && !y2) || ((q & 2) && !x2)) continue;
+        float pr, pi = 0.f;
+        if (CROSS) {
+          pr = f[q].x * g[q].x + f[q].y * g[q].y;
+          pi = f[q].y * g[q].x - f[q].x * g[q].y;
+        } else {
+          pr = f[q].x * f[q].x + f[q].y * f[q].y;
+        }
+        if (deconv) {
+          const float sy = tsy[ky];
+          pr = ((pr * sx) * sy) * sz;
+          pi = ((pi * sx) * sy) * sz;
+        }
+        ar += (double)(pr * w);
+        if (CROSS) ai += (double)(pi * w);
+      }
+      const double mult = (double)((x2 ? 2 : 1) * (y2 ? 2 : 1));
+      ak += mult * (double)(k * w);
+      an += mult * (double)w;
+    }
+    flush();
   }
   __syncthreads();
   for (int i = threadIdx.x; i < 4 * nedges; i += PS_TPB)
     part[(long long)blockIdx.x * 4 * nedges + i] = acc[i];
 }
 
-__global__ void powspec_reduce_k(const double* __restrict__ part, int nblocks, int m,
-                                 double* __restrict__ out) {
-  const int i = blockIdx.x * PS_TPB + threadIdx.x;
-  if (i >= m) return;
+// out[i] = the sum over blocks of part[b * m + i]: PS_RED threads to an i,
+// each over every PS_RED-th block in order, then their sums in order.
+__global__ void __launch_bounds__(PS_TPB)
+    powspec_reduce_k(const double* __restrict__ part, int nblocks, int m, double* __restrict__ out) {
+  constexpr int W = PS_TPB / PS_RED;
+  __shared__ double sh[PS_TPB];
+  const int col = threadIdx.x % W, row = threadIdx.x / W;
+  const int i = blockIdx.x * W + col;
   double s = 0.0;
-  for (int b = 0; b < nblocks; ++b) s += part[(long long)b * m + i];
+  if (i < m)
+    for (int b = row; b < nblocks; b += PS_RED) s += part[(long long)b * m + i];
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (row || i >= m) return;
+  for (int r = 1; r < PS_RED; ++r) s += sh[r * W + col];
   out[i] = s;
 }
 
 // r2c of a caller mesh into context buffer cb (padded layout, all axes)
 static int ps_r2c(pmx_ctx* c, const float* in, int cb) {
   int rc;
-  float2* f[3] = {c->cbuf[cb], c->cbuf[0], c->cbuf[0]};
-  if ((rc = pmx_copy_rows(c, (float*)f[0], c->rs, in, c->n[2]))) return rc;
-  if ((rc = pmx_fft_r2c_inplace(c, (float*)f[0], 0, 0.f))) return rc;
+  float2* f[1] = {c->cbuf[cb]};
+  if ((rc = r2c_dense(c, f[0], in))) return rc;
   if ((rc = pmx_fft_strided(c, f, 1, 1, -1))) return rc;
   return pmx_fft_strided(c, f, 1, 0, -1);
 }
@@ -2078,12 +2219,25 @@ extern "C" int pmx_powspec(pmx_ctx* c, const float* f, const float* g, int nedge
                                hipMemcpyHostToDevice, c->stream));
   if ((rc = ps_r2c(c, f, 1))) return rc;
   if (g && (rc = ps_r2c(c, g, 2))) return rc;
-  const size_t lds = (size_t)(m + nedges) * sizeof(double);
-  powspec_bin_k<<<PS_BLOCKS, PS_TPB, lds, c->stream>>>(
-      c->cbuf[1], g ? c->cbuf[2] : nullptr, c->n[0], c->n[1], c->n[2], c->n2h, c->n2p, dedges,
-      nedges, right, deconv, part);
+  // Groups of |ky| per thread: 8 let a sum stay in registers over a run; a
+  // small mesh takes fewer, down to one, before it leaves threads without work.
+  const int h0 = c->n[0] / 2 + 1, h1 = c->n[1] / 2 + 1;
+  int L = 8;
+  while (L > 1 && (long long)h0 * ((h1 + L - 1) / L) * c->n2h < PS_BLOCKS * PS_TPB) L /= 2;
+  const int nc1 = (h1 + L - 1) / L;
+  const long long units = (long long)h0 * nc1 * c->n2h;
+  const int nblk = (int)std::min<long long>((units + PS_TPB - 1) / PS_TPB, PS_BLOCKS);
+  const size_t lds = (size_t)(m + nedges) * sizeof(double) + 2 * (size_t)h1 * sizeof(float);
+#define PS_BIN(CROSS)                                                                              \
+  powspec_bin_k<CROSS><<<nblk, PS_TPB, lds, c->stream>>>(                                          \
+      c->cbuf[1], c->cbuf[2], c->n[0], c->n[1], c->n[2], c->n2h, c->n2p, dedges, nedges, right,    \
+      deconv, L, nc1, part)
+  if (g) PS_BIN(true);
+  else PS_BIN(false);
+#undef PS_BIN
   PMX_LAUNCH_CHECK();
-  powspec_reduce_k<<<(m + PS_TPB - 1) / PS_TPB, PS_TPB, 0, c->stream>>>(part, PS_BLOCKS, m, sums);
+  constexpr int W = PS_TPB / PS_RED;
+  powspec_reduce_k<<<(m + W - 1) / W, PS_TPB, 0, c->stream>>>(part, nblk, m, sums);
   PMX_LAUNCH_CHECK();
   PMX_CHECK_HIP(hipMemcpyAsync(out, sums, (size_t)m * sizeof(double), hipMemcpyDeviceToHost,
                                c->stream));

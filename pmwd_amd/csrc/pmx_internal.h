@@ -1082,6 +1082,10 @@ int pmx_fft_c2r_inplace(pmx_ctx* c, float* buf, float scale, int rev = 0);
 int pmx_fft_r2c_inplace(pmx_ctx* c, float* const* f, int nf, int pre, float coef, const float* halo,
                         const int* rev);
 int pmx_fft_c2r_inplace(pmx_ctx* c, float* const* f, int nf, float scale, const int* rev);
+int pmx_fft_r2c_rows(pmx_ctx* c, float* const* f, int nf, int pre, float coef, const float* halo,
+                     const int* rev, const float* const* real, int ors);
+int pmx_fft_c2r_rows(pmx_ctx* c, float* const* f, int nf, float scale, const int* rev,
+                     float* const* real, int ors);
 int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int rev = 0);
 int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev = 0);
 int pmx_poisson_x(pmx_ctx* c, float2* const* f, int adjoint, int kin = 0, int rev = 0);
