@@ -121,6 +121,22 @@ int pmx_random_bits(pmx_ctx* ctx, unsigned long long seed, long long nblocks, ui
  * source of lpt.py:40-76.  Order 2 holds one more mesh in the context.     */
 int pmx_lpt(pmx_ctx* ctx, const float* modes, float cell_vol, int order,
             const float* fac, float* disp, float* vel);
+/* The same from the Lagrangian grid (order 1 or 2): disp and vel are written
+ * and not read, disp's base being the grid's displacements dtab (device, n0 +
+ * n1 + n2 per-axis values; pmwd/particles.py:109-144), vel's zero.           */
+int pmx_lpt_grid(pmx_ctx* ctx, const float* modes, float cell_vol, int order,
+                 const float* fac, const float* dtab, float* disp, float* vel);
+/* Adjoint of pmx_lpt with respect to the modes: modes_cot (n0,n1,n2/2+1)
+ * complex64 is written, the conjugate gradient of a real loss (interior
+ * columns of the last axis count twice).                                    */
+int pmx_lpt_vjp(pmx_ctx* ctx, const float* modes, float cell_vol, int order,
+                const float* fac, const float* disp_cot, const float* vel_cot,
+                float* modes_cot);
+/* pmwd/particles.py:109-144 (gen_grid) from device tables of n0 + n1 + n2
+ * per-axis values: pmid and disp (N,3), N = n0 n1 n2, either may be NULL;
+ * 16-byte aligned.  No context.                                             */
+int pmx_grid(const int16_t* ptab, const float* dtab, int n0, int n1, int n2,
+             int16_t* pmid, float* disp, void* stream);
 /* pmwd/modes.py:67-117 (linear_modes) on an r2c spectrum (n0,n1,n2/2+1)
  * complex64 in place, on a context of the particle grid: modes *= scale
  * (float32; the 'ortho' normalisation of the white-noise transform), then
@@ -131,6 +147,11 @@ int pmx_lpt(pmx_ctx* ctx, const float* modes, float cell_vol, int order,
  * k_pivot, k_pivot, n_s, q = pi (c/H_0)^2 / Omega_m, V, d2 = D(a)^2 or 1}. */
 int pmx_linear_modes(pmx_ctx* ctx, float* modes, float scale, const double* tk,
                      const double* tT, int ntab, const double* par);
+/* Adjoint of the r2c of real white noise followed by pmx_linear_modes: cot is
+ * the modes' conjugate gradient (as pmx_lpt_vjp writes it), white_cot
+ * (n0,n1,n2) that of the noise.                                             */
+int pmx_linear_modes_vjp(pmx_ctx* ctx, const float* cot, float scale, const double* tk,
+                         const double* tT, int ntab, const double* par, float* white_cot);
 
 /* ----------------------------------------------------------- scatter ---
  * Default-argument CIC mass assignment (pmwd/scatter.py:33-83 with

@@ -1088,7 +1088,6 @@ int pmx_fft_c2r_rows(pmx_ctx* c, float* const* f, int nf, float scale, const int
                      float* const* real, int ors);
 int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int rev = 0);
 int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev = 0);
-int pmx_poisson_x(pmx_ctx* c, float2* const* f, int adjoint, int kin = 0, int rev = 0);
 // copies n0*n1 rows of ncols floats between row strides (ncols <= 0: n2)
 int pmx_copy_rows(pmx_ctx* c, float* dst, int dst_rs, const float* src, int src_rs, int ncols = 0);
 int pmx_poisson_adj_ctx(pmx_ctx* c, float scale_out, int deferred = 0);

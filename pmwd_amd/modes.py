@@ -12,6 +12,7 @@ import math
 
 import numpy as np
 import torch
+from torch.autograd.function import once_differentiable
 
 from .boltzmann import growth
 from .cosmo_param import check_theta, host_value, modes_factor_derivs
@@ -71,27 +72,81 @@ def _needs_graph(modes, theta):
     return theta is not None and any(t.requires_grad for t in theta.values())
 
 
-def _linear_modes_fused(modes, cosmo, conf, a, real):
-    """linear_modes without gradients: the r2c of real white noise, then one
-    library pass (pmx_linear_modes) for the 'ortho' scale and sqrt(V P)."""
+class _Power:
+    """The host side of pmx_linear_modes: transfer table and constants."""
+
+    def __init__(self, cosmo, conf, a):
+        self.tk = np.ascontiguousarray(conf.transfer_k, dtype=np.float64)
+        self.tT = np.ascontiguousarray(cosmo.transfer, dtype=np.float64)
+        self.par = np.array([0.32 * cosmo.A_s * cosmo.k_pivot, cosmo.k_pivot, cosmo.n_s,
+                             math.pi * (conf.c / conf.H_0)**2 / cosmo.Omega_m, conf.box_vol,
+                             float(growth(a, cosmo, conf))**2 if a is not None else 1.0],
+                            dtype=np.float64)
+
+    def args(self):
+        P = lambda x: x.ctypes.data_as(ctypes.c_void_p)
+        return P(self.tk), P(self.tT), len(self.tk), P(self.par)
+
+
+def _apply_power(modes, conf, power):
+    """sqrt(V P) times the modes of real or complex white noise: the r2c of
+    real noise, then one library pass for its 'ortho' scale and the factor."""
     from . import _lib
-    dev = modes.device
-    c = _lib.context(conf.ptcl_grid_shape, conf.ptcl_spacing, dev)
+    c = _lib.context(conf.ptcl_grid_shape, conf.ptcl_spacing, modes.device)
     if torch.is_complex(modes):
-        out = modes.detach().to(torch.complex64).clone().contiguous()
+        out = modes.detach().to(torch.complex64).resolve_conj().resolve_neg()
+        out = out.clone(memory_format=torch.contiguous_format)
         scale = 1.0
     else:
         out = fftfwd(modes.detach().to(conf.float_dtype))
         scale = 1 / math.sqrt(math.prod(conf.ptcl_grid_shape))
-    tk = np.ascontiguousarray(conf.transfer_k, dtype=np.float64)
-    tT = np.ascontiguousarray(cosmo.transfer, dtype=np.float64)
-    par = np.array([0.32 * cosmo.A_s * cosmo.k_pivot, cosmo.k_pivot, cosmo.n_s,
-                    math.pi * (conf.c / conf.H_0)**2 / cosmo.Omega_m, conf.box_vol,
-                    float(growth(a, cosmo, conf))**2 if a is not None else 1.0],
-                   dtype=np.float64)
-    P = lambda x: x.ctypes.data_as(ctypes.c_void_p)
-    _lib.check(_lib.lib().pmx_linear_modes(c.bind(), _lib.ptr(out), float(scale), P(tk), P(tT),
-                                           len(tk), P(par)))
+    _lib.check(_lib.lib().pmx_linear_modes(c.bind(), _lib.ptr(out), float(scale), *power.args()))
+    return out, scale, c
+
+
+class _LinearModesFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, modes, conf, power):
+        out, ctx.scale, ctx.pmx = _apply_power(modes, conf, power)
+        ctx.power, ctx.real, ctx.shape = power, not torch.is_complex(modes), tuple(modes.shape)
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, cot):
+        from . import _lib
+        g = cot.resolve_conj().resolve_neg().contiguous()
+        # the forward's context: autograd may run this on another thread
+        if ctx.real:
+            out = torch.empty(ctx.shape, dtype=torch.float32, device=g.device)
+            _lib.check(_lib.lib().pmx_linear_modes_vjp(ctx.pmx.bind(), _lib.ptr(g),
+                                                       float(ctx.scale), *ctx.power.args(),
+                                                       _lib.ptr(out)))
+        else:
+            out = g.clone()   # a real factor is its own adjoint
+            _lib.check(_lib.lib().pmx_linear_modes(ctx.pmx.bind(), _lib.ptr(out), 1.0,
+                                                   *ctx.power.args()))
+        return out, None, None
+
+
+def _fused_graph(modes, theta, conf):
+    """Whether gradients go through the library's adjoint: those of float32 or
+    complex64 noise of the particle grid.  Cosmological parameters with
+    gradients keep the tensor path."""
+    n0, n1, n2 = conf.ptcl_grid_shape
+    shape = (n0, n1, n2 // 2 + 1) if torch.is_complex(modes) else (n0, n1, n2)
+    return (modes.is_cuda and conf.float_dtype == torch.float32
+            and modes.dtype in (torch.float32, torch.complex64) and tuple(modes.shape) == shape
+            and (theta is None or not any(t.requires_grad for t in theta.values())))
+
+
+def _linear_modes_fused(modes, cosmo, conf, a, real):
+    """linear_modes in the library, and its gradient with respect to the noise."""
+    power = _Power(cosmo, conf, a)
+    if _needs_graph(modes, None):
+        out = _LinearModesFn.apply(modes, conf, power)
+    else:
+        out, _, _ = _apply_power(modes, conf, power)
     if real:
         out = fftinv(out, shape=conf.ptcl_grid_shape, norm=conf.ptcl_spacing)
     return out
@@ -107,7 +162,7 @@ def linear_modes(modes, cosmo, conf, a=None, real=False, theta=None):
     if cosmo.transfer is None:
         raise ValueError('Transfer table is empty. Call transfer_integ or boltzmann first.')
     theta = check_theta(theta, cosmo)
-    if not _needs_graph(modes, theta):
+    if not _needs_graph(modes, theta) or _fused_graph(modes, theta, conf):
         return _linear_modes_fused(modes, cosmo, conf, a, real)
     if not torch.is_complex(modes):
         modes = fftfwd(modes.to(conf.float_dtype), norm='ortho')

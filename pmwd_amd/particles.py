@@ -18,6 +18,41 @@ def default_device():
     return torch.device('cuda') if torch.cuda.is_available() else torch.device('cpu')
 
 
+def _grid_axes(conf):
+    """Per axis the Lagrangian grid's int16 mesh indices and float32 displacements."""
+    axes = []
+    for sp, sm in zip(conf.ptcl_grid_shape, conf.mesh_shape):
+        p1 = np.rint(np.linspace(0, sm, num=sp, endpoint=False)).astype(np.int16)
+        d1 = (np.arange(sp) * sm - p1.astype(np.int64) * sp) * (conf.cell_size / sp)
+        axes.append((p1, d1.astype(np.float32)))
+    return axes
+
+
+def _grid_on_device(conf, device):
+    """Whether the library writes the grid: 3D, int16 and float32, on a GPU."""
+    return (device.type == 'cuda' and conf.dim == 3 and conf.pmid_dtype == torch.int16
+            and conf.float_dtype == torch.float32)
+
+
+def _grid_tables(axes, device):
+    return tuple(torch.as_tensor(np.concatenate(t), device=device) for t in zip(*axes))
+
+
+def _gen_grid_dev(conf, tables, disp):
+    """pmid and, with ``disp``, the displacements of the grid (``pmx_grid``)."""
+    from . import _lib
+    dev = tables[0].device
+    shape = (int(conf.ptcl_num), 3)
+    with torch.cuda.device(dev):
+        pmid = torch.empty(shape, dtype=torch.int16, device=dev)
+        d = torch.empty(shape, dtype=torch.float32, device=dev) if disp else None
+        stream = torch.cuda.current_stream(dev).cuda_stream
+        _lib.check(_lib.lib().pmx_grid(_lib.ptr(tables[0]), _lib.ptr(tables[1]),
+                                       *(int(s) for s in conf.ptcl_grid_shape), _lib.ptr(pmid),
+                                       _lib.ptr(d), ctypes.c_void_p(stream)))
+    return pmid, d
+
+
 @dataclass(frozen=True)
 class Particles:
     """Particle state: ``pmid``, ``disp``, optional ``vel``, ``acc``, ``attr``.
@@ -82,12 +117,14 @@ class Particles:
     def gen_grid(cls, conf, vel=False, acc=False, device=None):
         """Particles on the Lagrangian grid (particles.py:109-144)."""
         device = torch.device(device) if device is not None else default_device()
-        pmid, disp = [], []
-        for sp, sm in zip(conf.ptcl_grid_shape, conf.mesh_shape):
-            p1 = np.rint(np.linspace(0, sm, num=sp, endpoint=False)).astype(np.int16)
-            d1 = (np.arange(sp) * sm - p1.astype(np.int64) * sp) * (conf.cell_size / sp)
-            pmid.append(torch.as_tensor(p1, device=device).to(conf.pmid_dtype))
-            disp.append(torch.as_tensor(d1.astype(np.float32), device=device).to(conf.float_dtype))
+        axes = _grid_axes(conf)
+        if _grid_on_device(conf, device):
+            pmid, disp = _gen_grid_dev(conf, _grid_tables(axes, device), True)
+            v = torch.zeros_like(disp) if vel else None
+            a = torch.zeros_like(disp) if acc else None
+            return cls(conf, pmid, disp, vel=v, acc=a)
+        pmid = [torch.as_tensor(p, device=device).to(conf.pmid_dtype) for p, _ in axes]
+        disp = [torch.as_tensor(d, device=device).to(conf.float_dtype) for _, d in axes]
         pmid = torch.stack(torch.meshgrid(*pmid, indexing='ij'), dim=-1).reshape(-1, conf.dim)
         disp = torch.stack(torch.meshgrid(*disp, indexing='ij'), dim=-1).reshape(-1, conf.dim)
         v = torch.zeros_like(disp) if vel else None
