@@ -24,7 +24,7 @@
 #define PL_TPB 512
 #endif
 #ifndef PL_U
-#define PL_U 4
+#define PL_U 2
 #endif
 #ifndef PL_MINB
 #define PL_MINB 1
@@ -50,6 +50,16 @@ struct PlUser {
   float* vel;
   float* acc;
 };
+
+// Three consecutive floats of particle i in one 12-byte store (the compiler
+// joins them; interleaved stores to arrays that may alias it leaves as nine).
+// The last step: 64^3 particles 16.1 -> 11.9 us, 512^3 4302 -> 4164, the
+// reverse one at 128^3 160 -> 150.
+__device__ __forceinline__ void put3(float* o, long long i, const float v[3]) {
+  o[3 * i] = v[0];
+  o[3 * i + 1] = v[1];
+  o[3 * i + 2] = v[2];
+}
 
 __device__ __forceinline__ void pl_put(const PState& st, uint32_t slot, float4 s0, float4 s1) {
   st.s0[slot] = s0;
@@ -134,22 +144,35 @@ __global__ void __launch_bounds__(PL_TPB, PL_MINB)
     const int ltot = (s[0] + 1) * LY * LZ;
     const float* F[3] = {F0, F1, F2};
     if (MODE == PL_CAP && threadIdx.x < 27) s_cnt[threadIdx.x] = 0u;
-    pmx_stage_tile<3, PL_TPB>(sh, o, LY, LZ, ltot, g, F);
-    __syncthreads();
     const uint32_t start = in_start[t];
     const uint32_t cnt = in_count[t];
+    // a round's particles are loaded ahead, the first with the tile's meshes,
+    // so no load's latency stands alone (128^3 mesh, 512 tiles: 13.5 -> 12.8
+    // us; 512^3: 2237 -> 2207)
+    float4 p0[PL_U], p1[PL_U];
+    auto fetch = [&](uint32_t q0) {
+  #pragma unroll
+      for (int u = 0; u < PL_U; ++u) {
+        const uint32_t q = q0 + u * PL_TPB + threadIdx.x;
+        if (q < cnt) {
+          p0[u] = in.s0[start + q];
+          p1[u] = in.s1[start + q];
+        }
+      }
+    };
+    fetch(0);
+    pmx_stage_tile<3, PL_TPB>(sh, o, LY, LZ, ltot, g, F);
+    __syncthreads();
     for (uint32_t q0 = 0; q0 < cnt; q0 += PL_TPB * PL_U) {
       float4 a0[PL_U], a1[PL_U], n0[PL_U], n1[PL_U];
       uint32_t nt[PL_U];
       int code[PL_U];
   #pragma unroll
       for (int u = 0; u < PL_U; ++u) {
-        const uint32_t q = q0 + u * PL_TPB + threadIdx.x;
-        if (q < cnt) {
-          a0[u] = in.s0[start + q];
-          a1[u] = in.s1[start + q];
-        }
+        a0[u] = p0[u];
+        a1[u] = p1[u];
       }
+      fetch(q0 + PL_TPB * PL_U);
   #pragma unroll
       for (int u = 0; u < PL_U; ++u) {
         const uint32_t q = q0 + u * PL_TPB + threadIdx.x;
@@ -170,12 +193,9 @@ __global__ void __launch_bounds__(PL_TPB, PL_MINB)
           for (int a = 0; a < 3; ++a) v[a] = v[a] + acc[a] * k2;
           if (MODE == PL_LAST) {
             const long long i = __float_as_uint(a1[u].w);
-  #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-              user.acc[3 * i + a] = acc[a];
-              user.vel[3 * i + a] = v[a];
-              user.disp[3 * i + a] = x[a];
-            }
+            put3(user.acc, i, acc);
+            put3(user.vel, i, v);
+            put3(user.disp, i, x);
           } else {
   #pragma unroll
             for (int a = 0; a < 3; ++a) {
@@ -605,8 +625,6 @@ __global__ void __launch_bounds__(AL_TPB) __attribute__((amdgpu_waves_per_eu(4))
     const int ltot = (s[0] + 1) * LY * LZ;
     const float* F[4] = {F0, F1, F2, R};
     if (MODE == PL_CAP && threadIdx.x < 27) s_cnt[threadIdx.x] = 0u;
-    pmx_stage_tile<4, AL_TPB>(sh, o, LY, LZ, ltot, g, F);
-    __syncthreads();
     const uint32_t start = in_start[t];
     const uint32_t cnt = in_count[t];
     // the next round's particles are loaded before this round's arithmetic,
@@ -627,6 +645,8 @@ __global__ void __launch_bounds__(AL_TPB) __attribute__((amdgpu_waves_per_eu(4))
       }
     };
     fetch(0, pa0, pa1, pc0, pc1);
+    pmx_stage_tile<4, AL_TPB>(sh, o, LY, LZ, ltot, g, F);
+    __syncthreads();
     for (uint32_t q0 = 0; q0 < cnt; q0 += AL_TPB * AL_U) {
       float4 a0[AL_U], a1[AL_U], c0[AL_U];
       float2 c1[AL_U];
@@ -664,15 +684,12 @@ __global__ void __launch_bounds__(AL_TPB) __attribute__((amdgpu_waves_per_eu(4))
         for (int a = 0; a < 3; ++a) at[a] = at[a] + gr[a];
         if (MODE == PL_LAST) {
           const long long i = __float_as_uint(a1[u].w);
-#pragma unroll
-          for (int a = 0; a < 3; ++a) {
-            user.disp[3 * i + a] = x[a];
-            user.vel[3 * i + a] = v[a];
-            user.disp_cot[3 * i + a] = dc[a];
-            user.vel_cot[3 * i + a] = vc[a];
-            user.acc[3 * i + a] = ac[a];
-            user.acc_cot[3 * i + a] = at[a];
-          }
+          put3(user.disp, i, x);
+          put3(user.vel, i, v);
+          put3(user.disp_cot, i, dc);
+          put3(user.vel_cot, i, vc);
+          put3(user.acc, i, ac);
+          put3(user.acc_cot, i, at);
           continue;
         }
 #pragma unroll
