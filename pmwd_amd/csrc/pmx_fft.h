@@ -233,25 +233,44 @@ __host__ __device__ constexpr int lds_elems(int lay, int n, int P) {
 
 __host__ __device__ constexpr int ilog2c(int n) { return n <= 1 ? 0 : 1 + ilog2c(n >> 1); }
 
-// Columns per workgroup of a strided pass of fixed length 2^ln: 16 (128-byte
+// Lengths with compile-time kernels, by the code LN: 2^LN for 6..10, and
+// 3 2^(LN - 32) for 37..40 (96, 192, 384, 768: the meshes of 1.5 cells a
+// particle).  With run-time stages, divisions and addresses the passes of
+// 192^3 took: Poisson x 90 us (now 28), the inverse y pair 67 (22), y 31 (13),
+// c2r 39 (29).
+__host__ __device__ constexpr bool ct_three(int ln) { return ln >= 32; }
+__host__ __device__ constexpr int ct_n(int ln) { return ct_three(ln) ? 3 << (ln - 32) : 1 << ln; }
+__host__ __device__ constexpr int pow2_floor(int n) { return n < 2 ? 1 : 2 * pow2_floor(n / 2); }
+
+// Columns per workgroup of a strided pass of fixed length: 16 (128-byte
 // segments of a row), fewer when they exceed cap values; and its threads, of
 // v values each.  A 64^3 or 128^3 mesh has 33 or 65 columns, which blocks
 // filled to cap (128 and 64 columns) left half empty and too few.
 __host__ __device__ constexpr int ct_cols(int ln, int cap) {
-  return (cap >> ln) >= 16 ? 16 : (cap >> ln);
+  return cap / ct_n(ln) >= 16 ? 16 : pow2_floor(cap / ct_n(ln));
 }
-__host__ __device__ constexpr int ct_tpb(int ln, int cols, int v) { return (cols << ln) / v; }
-#define FFT_V 16   // y and plain x passes
-#define PFFT_V 8   // Poisson x pass
+__host__ __device__ constexpr int ct_tpb(int ln, int cols, int v) { return cols * ct_n(ln) / v; }
+// Values per thread of the y and plain x passes: 16, and 8 where more
+// wavefronts on the few blocks of a small mesh count (inverse of 128^3: 9.6
+// -> 8.5 us, the pair of components 10.8 -> 9.7; 256^3 25.0 -> 24.4 and 42.7
+// -> 41.1; but 512^3 251 -> 256 and 413 -> 433).  The forward passes keep 16:
+// with 8 the compiler contracts other products into FMAs, and results would
+// move by a rounding.
+// Lengths 3 2^k take 12, which their first (4) and last (6) radix divide.
+__host__ __device__ constexpr int fft_v(int dir, int ln) {
+  return ct_three(ln) ? 12 : (dir > 0 && ln <= 8 ? 8 : 16);
+}
+// Poisson x pass
+__host__ __device__ constexpr int pfft_v(int ln) { return ct_three(ln) ? 12 : 8; }
 
-// Rows per workgroup of a row pass of fixed length 2^lh: RFFT_CAP values, or
-// a quarter of that for meshes whose row blocks would leave CUs idle.  The
-// workgroup has eight values per thread.
+// Rows per workgroup of a row pass of fixed length: RFFT_CAP values, or
+// a quarter of that (3/8 for 3 2^k: whole wavefronts) for meshes whose row
+// blocks would leave CUs idle.  The workgroup has eight values per thread.
 __host__ __device__ constexpr int ct_rows(int lh, bool small) {
-  return (small ? RFFT_CAP / 4 : RFFT_CAP) >> lh ? ((small ? RFFT_CAP / 4 : RFFT_CAP) >> lh) : 1;
+  return pow2_floor((small ? (ct_three(lh) ? RFFT_CAP * 3 / 8 : RFFT_CAP / 4) : RFFT_CAP) / ct_n(lh));
 }
 __host__ __device__ constexpr int ct_row_tpb(int lh, bool small) {
-  return (ct_rows(lh, small) << lh) / 8;
+  return ct_rows(lh, small) * ct_n(lh) / 8;
 }
 
 // One Stockham stage of radix R (n a power of two, Ns the size of the
@@ -508,18 +527,27 @@ __device__ __forceinline__ void lds_fft(float2* s, int n, int P, const float2* _
 // element x of pencil p sits at lidx(p, x); the R inputs of a butterfly are
 // a fixed stride apart, and so are its R outputs except for ROWS stages
 // with 1 < NS < 8, which compute each address.
-template <int R, int DIR, int LAY, int N, int P, int NS, int TPB, int TWS>
-__device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ tw) {
+//
+// REG (COLS): the first (REG & 1) stage takes its inputs from reg, the last
+// (REG & 2) leaves its outputs there, both in the order of ColMap (element e
+// of a thread is row j0 + e js): a butterfly's inputs j + r N/R of the first
+// stage and outputs of the last are the rows that its thread loads and
+// stores, so half of a transform's LDS traffic and three of its barriers go.
+// Poisson x pass, same bits: 128^3 15.0 -> 13.2 us, 256^3 53 -> 45, 512^3 470
+// -> 455 (there bound by memory).
+template <int R, int DIR, int LAY, int N, int P, int NS, int TPB, int TWS, int REG = 0>
+__device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ tw,
+                                         float2* reg = nullptr) {
   constexpr int NB = N / R, TOTAL = P * NB;
   constexpr int NG = (TOTAL + TPB - 1) / TPB;
   constexpr bool FULL = TOTAL % TPB == 0;
-  constexpr int LP = ilog2c(P), LNB = ilog2c(NB);
+  constexpr int LP = ilog2c(P);
   constexpr int STEP = N / (NS * R) * TWS;
   constexpr bool SEP_IN = LAY == COLS || NB % 8 == 0;
   constexpr bool SEP_OUT = LAY == COLS || NS % 8 == 0 || NS == 1;
   constexpr int SIN = LAY == ROWS ? NB + (NB >> 3) : NB * P;
   constexpr int SOUT = LAY == ROWS ? NS + (NS >> 3) : NS * P;
-  constexpr bool ALLTW = LAY == COLS;
+  constexpr bool ALLTW = LAY == COLS || R == 6;
   float2 v[NG * R];
   float2 w[NG][R > 1 ? R - 1 : 1];
   int ob[NG];
@@ -527,14 +555,16 @@ __device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ t
   for (int it = 0; it < NG; ++it) {
     const int idx = threadIdx.x + it * tpb<TPB>();
     if (FULL || idx < TOTAL) {
-      const int p = LAY == ROWS ? idx >> LNB : idx & (P - 1);
-      const int j = LAY == ROWS ? idx & (NB - 1) : idx >> LP;
+      const int p = LAY == ROWS ? (unsigned)idx / NB : idx & (P - 1);
+      const int j = LAY == ROWS ? (unsigned)idx % NB : idx >> LP;
       const int k = j & (NS - 1);
       ob[it] = lidx<LAY>(p, (j - k) * R + k, N, P);
       const int ib = lidx<LAY>(p, j, N, P);
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        v[it * R + r] = SEP_IN ? s[ib + r * SIN] : s[lidx<LAY>(p, j + r * NB, N, P)];
+      for (int r = 0; r < R; ++r) {
+        if constexpr (REG & 1) v[it * R + r] = reg[it + r * NG];
+        else v[it * R + r] = SEP_IN ? s[ib + r * SIN] : s[lidx<LAY>(p, j + r * NB, N, P)];
+      }
       if (NS > 1) {
         const int m = k * STEP;
         if (ALLTW) {
@@ -568,7 +598,14 @@ __device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ t
       dftR<R, DIR>(u);
     }
   }
-  __syncthreads();
+  if constexpr (REG & 2) {
+#pragma unroll
+    for (int it = 0; it < NG; ++it)
+#pragma unroll
+      for (int r = 0; r < R; ++r) reg[it + r * NG] = v[it * R + r];
+    return;
+  }
+  if constexpr (!(REG & 1)) __syncthreads();
 #pragma unroll
   for (int it = 0; it < NG; ++it) {
     const int idx = threadIdx.x + it * tpb<TPB>();
@@ -577,7 +614,7 @@ __device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ t
 #pragma unroll
         for (int r = 0; r < R; ++r) s[ob[it] + r * SOUT] = v[it * R + r];
       } else {
-        const int p = idx >> LNB, j = idx & (NB - 1);
+        const int p = (unsigned)idx / NB, j = (unsigned)idx % NB;
         const int k = j & (NS - 1), o = (j - k) * R + k;
 #pragma unroll
         for (int r = 0; r < R; ++r) s[lidx<LAY>(p, o + r * NS, N, P)] = v[it * R + r];
@@ -587,22 +624,40 @@ __device__ __forceinline__ void ct_stage(float2* s, const float2* __restrict__ t
   __syncthreads();
 }
 
+// Radix of the stage after NS: 8 (then 4 or 2) for powers of two; 4, then 8
+// or 4, and 6 last for 3 2^k, so that every NS is a power of two.
+__host__ __device__ constexpr int ct_radix(int n, int ns) {
+  return n % 3      ? (n / ns % 8 == 0 ? 8 : (n / ns % 4 == 0 ? 4 : 2))
+         : ns == 1  ? 4
+         : n / ns == 6 ? 6
+                    : (n / ns / 6 % 8 == 0 && n / ns != 96 ? 8 : (n / ns / 6 % 4 == 0 ? 4 : 2));
+}
+
 template <int DIR, int LAY, int N, int P, int NS, int TPB, int TWS>
 __device__ __forceinline__ void ct_fft(float2* s, const float2* __restrict__ tw) {
   if constexpr (NS < N) {
-    constexpr int REM = N / NS;
-    constexpr int R = REM % 8 == 0 ? 8 : (REM % 4 == 0 ? 4 : 2);
+    constexpr int R = ct_radix(N, NS);
     ct_stage<R, DIR, LAY, N, P, NS, TPB, TWS>(s, tw);
     ct_fft<DIR, LAY, N, P, NS * R, TPB, TWS>(s, tw);
   }
 }
 
+// The same from and to registers (N >= 64: at least two stages).
+template <int DIR, int N, int P, int NS, int TPB>
+__device__ __forceinline__ void ct_fft_reg(float2* reg, float2* s, const float2* __restrict__ tw) {
+  if constexpr (NS < N) {
+    constexpr int R = ct_radix(N, NS);
+    ct_stage<R, DIR, COLS, N, P, NS, TPB, 1, (NS == 1 ? 1 : 0) | (NS * R == N ? 2 : 0)>(s, tw, reg);
+    ct_fft_reg<DIR, N, P, NS * R, TPB>(reg, s, tw);
+  }
+}
+
 // FFT of P pencils of length n: the compile-time path when LN > 0
-// (n = 2^LN, P = 2^LP), else lds_fft.
+// (n = ct_n(LN), P = 2^LP), else lds_fft.
 template <int DIR, int LAY, bool POW2, int LN, int LP, int MAXV, int TPB, int TWS = 1>
 __device__ __forceinline__ void fft_run(float2* s, int n, int P, const float2* __restrict__ tw) {
   if constexpr (LN > 0)
-    ct_fft<DIR, LAY, 1 << LN, 1 << LP, 1, TPB, TWS>(s, tw);
+    ct_fft<DIR, LAY, ct_n(LN), 1 << LP, 1, TPB, TWS>(s, tw);
   else
     lds_fft<DIR, LAY, POW2, MAXV, TPB>(s, n, P, tw, TWS);
 }
@@ -658,15 +713,15 @@ __device__ __forceinline__ float2 r2c_half_x(const float2* s, const float2* stw,
   return cadd(e, cmul(stw[k], o));
 }
 
-// Splits a block's value index into row and position (shifts when H = 2^LH).
+// Splits a block's value index into row and position (by a constant when LH).
 template <int LH>
 struct RowSplit {
   int H;
   FastDiv d;
   __device__ __forceinline__ explicit RowSplit(int H_) : H(H_), d(LH ? 1 : H_) {}
-  __device__ __forceinline__ int row(int idx) const { return LH ? idx >> LH : d(idx); }
+  __device__ __forceinline__ int row(int idx) const { return LH ? (unsigned)idx / ct_n(LH) : d(idx); }
   __device__ __forceinline__ int col(int idx, int p) const {
-    return LH ? idx & ((1 << LH) - 1) : idx - p * H;
+    return LH ? (unsigned)idx % ct_n(LH) : idx - p * H;
   }
 };
 
@@ -787,6 +842,26 @@ __device__ __forceinline__ ColMap col_map(int lB) {
   return m;
 }
 
+// FFT of a block of columns held in registers in the order of cm, through
+// the LDS block s, which no thread may still be reading on entry (and some
+// may on return).  The staging of the twiddles need not be waited for.
+template <int DIR, bool POW2, int LN, int LP, int MAXV, int TPB>
+__device__ __forceinline__ void fft_cols(float2 (&r)[MAXV], float2* s, int n, int P,
+                                         const float2* __restrict__ tw, const ColMap& cm) {
+  if constexpr (LN > 0) {
+    ct_fft_reg<DIR, ct_n(LN), 1 << LP, 1, TPB>(r, s, tw);
+  } else {
+#pragma unroll
+    for (int it = 0; it < MAXV; ++it)
+      if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * tpb<TPB>()] = r[it];
+    __syncthreads();
+    fft_run<DIR, COLS, POW2, LN, LP, MAXV, TPB>(s, n, P, tw);
+#pragma unroll
+    for (int it = 0; it < MAXV; ++it)
+      if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * tpb<TPB>()];
+  }
+}
+
 // Source of a Poisson x pass other than its own buffer (poisson_x_k).
 struct SpecSrc {
   const float2* modes;
@@ -818,12 +893,13 @@ static inline size_t lds_bytes(int n, int P, int lay = COLS) {
 static inline size_t tw_bytes(int n) { return (size_t)n * sizeof(float2); }
 
 
-// log2 of a length that has compile-time kernel variants (64..1024), else 0
-static inline int ct_log2(int n) {
-  if (!is_pow2(n) || n < 64 || n > 1024) return 0;
-  int l = 0;
-  while ((1 << l) < n) ++l;
-  return l;
+// Code of a length that has compile-time kernels, else 0.
+static inline int ct_code(int n) {
+  for (int l = 6; l <= 10; ++l)
+    if (n == ct_n(l)) return l;
+  for (int l = 37; l <= 40; ++l)
+    if (n == ct_n(l)) return l;
+  return 0;
 }
 
 // Threads of a run-time-length workgroup of `total` values.
@@ -836,7 +912,7 @@ static inline int gen_tpb(int total) {
 #define FFT_MIN_WGS 1024
 
 // The z pass of n2 over nrows rows: even n2 as half-length transforms, of
-// compile-time length 2^lh when that is 64..1024 and the row blocks come out
+// compile-time length (code lh) when there are kernels and the row blocks come out
 // even, else (and for odd n2, two rows a pencil) at run time.  rows: rows per
 // workgroup.  Meshes of few rows take smaller blocks (sm): a 128^3 mesh has
 // 256 row blocks of 4096 values, one per CU, and their load, barrier and
@@ -851,7 +927,7 @@ static inline RowPlan row_plan(int n2, long long nrows) {
   RowPlan r;
   r.half = n2 >= 4 && (n2 & 1) == 0;
   r.len = r.half ? n2 / 2 : n2;
-  r.lh = r.half ? ct_log2(r.len) : 0;
+  r.lh = r.half ? ct_code(r.len) : 0;
   r.sm = false;
   if (r.lh) {
     r.sm = nrows / ct_rows(r.lh, false) < FFT_MIN_WGS;
@@ -881,7 +957,7 @@ static inline int gen_cols(int n, int ncol, long long nouter) {
   return B;
 }
 
-// CALL(L) with L the compile-time constant for ln (0: generic kernels)
+// CALL(L) with L the compile-time code ln (0: generic kernels)
 #define PMX_CT_SWITCH(ln, CALL) \
   do {                          \
     switch (ln) {               \
@@ -890,6 +966,10 @@ static inline int gen_cols(int n, int ncol, long long nouter) {
       case 8: CALL(8); break;   \
       case 9: CALL(9); break;   \
       case 10: CALL(10); break; \
+      case 37: CALL(37); break; \
+      case 38: CALL(38); break; \
+      case 39: CALL(39); break; \
+      case 40: CALL(40); break; \
       default: CALL(0);         \
     }                           \
   } while (0)

@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(GEN_MAXTPB, 4) z_c2r_k(RowFields rf, long long
 // Half-length r2c for even n2, H = n2/2: the row is read as H complex values z[m] = x[2m] + i x[2m+1],
 // Z = FFT_H(z), and for k = 0..H:  X[k] = E + w^k O,  E = (Z[k] + conj Z[H-k])/2,
 // O = -i (Z[k] - conj Z[H-k])/2,  w = exp(-2 pi i/n2)  (Z[H] = Z[0]).
-// PRE applies (x - 1) * coef on load.  LH > 0 fixes H = 2^LH and
+// PRE applies (x - 1) * coef on load.  LH > 0 fixes H = ct_n(LH) and
 // P = ct_rows(LH, SM) at compile time (the launch then holds whole blocks);
 // LH = 0 takes any H, POW2 telling whether it is a power of two.
 // The deposit's halo shells of one channel for a row pass that folds them
@@ -255,7 +255,7 @@ __device__ __forceinline__ void fold_rows(float2 (&r)[NV], const FoldIn& fi, int
   }
 }
 
-// FOLD (with LH > 0, 16^3 tiles, P | n1): the density is the deposit's tile
+// FOLD (with H = 2^LH, 16^3 tiles, P | n1): the density is the deposit's tile
 // interiors plus the fold of fi.halo, added here on load.
 template <int PRE, int LH, bool SM, bool FOLD, bool POW2>
 __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
@@ -266,8 +266,8 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
   if (PRE && fcoef) coef = fcoef[0];
   constexpr int PC = LH ? ct_rows(LH, SM) : 1;
   constexpr int TPB = LH ? ct_row_tpb(LH, SM) : GEN_TPB;
-  constexpr int MAXV = LH ? (PC << LH) / TPB : GEN_MAXV;
-  const int H = LH ? 1 << LH : n2 >> 1;
+  constexpr int MAXV = LH ? PC * ct_n(LH) / TPB : GEN_MAXV;
+  const int H = LH ? ct_n(LH) : n2 >> 1;
   const int P = LH ? PC : P_;
   const RowSplit<LH> rsp(H);
   float2* stw = s + lds_elems(ROWS, H, P);
@@ -342,8 +342,8 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
   extern __shared__ float2 s[];
   constexpr int PC = LH ? ct_rows(LH, SM) : 1;
   constexpr int TPB = LH ? ct_row_tpb(LH, SM) : GEN_TPB;
-  constexpr int MAXV = LH ? (PC << LH) / TPB : GEN_MAXV;
-  const int H = LH ? 1 << LH : n2 >> 1;
+  constexpr int MAXV = LH ? PC * ct_n(LH) / TPB : GEN_MAXV;
+  const int H = LH ? ct_n(LH) : n2 >> 1;
   const int P = LH ? PC : P_;
   const RowSplit<LH> rsp(H);
   float2* stw = s + lds_elems(ROWS, H, P);
@@ -373,16 +373,16 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
 // to the other (the same one in place).  A workgroup takes B consecutive
 // columns, so each of its loads is B contiguous float2.
 // LDS: the n x B block, then the n-entry twiddle table.  LN > 0 fixes
-// n = 2^LN and B = ct_cols(LN, FFT_CAP) at compile time.
+// n = ct_n(LN) and B = ct_cols(LN, FFT_CAP) at compile time.
 template <int DIR, bool POW2, int LN>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) : GEN_MAXTPB, 4) strided_fft_k(Side3 si, Side3 so, int rev,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(DIR, LN)) : GEN_MAXTPB, 4) strided_fft_k(Side3 si, Side3 so, int rev,
                                                          int n_, int ncol, int B_,
                                                          const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, FFT_CAP) : 1;
-  constexpr int TPB = LN ? ct_tpb(LN, BC, FFT_V) : GEN_TPB;
-  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
-  const int n = LN ? 1 << LN : n_;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, fft_v(DIR, LN)) : GEN_TPB;
+  constexpr int MAXV = LN ? BC * ct_n(LN) / TPB : GEN_MAXV;
+  const int n = LN ? ct_n(LN) : n_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
   float2* stw = s + n * B;
@@ -402,14 +402,7 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) :
     r[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n) r[it] = g[it * gs];
   }
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * tpb<TPB>()] = r[it];
-  __syncthreads();
-  fft_run<DIR, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * tpb<TPB>()];
+  fft_cols<DIR, POW2, LN, ilog2c(BC), MAXV, TPB>(r, s, n, B, stw, cm);
   float2* d = (bz == 0 ? so.f[0] : (bz == 1 ? so.f[1] : so.f[2])) + (long long)by * so.os + c0 +
               cm.b + (long long)cm.j0 * so.es;
   const long long ds = (long long)cm.js * so.es;
@@ -428,19 +421,20 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) :
 // other in the same LDS block, h kept in registers meanwhile.  Pencils along
 // axis 0 of (n0,n1,n2h); blockIdx.y = y index, blockIdx.x = block of B kz
 // columns.  LDS: the n0 x B block, the n0-entry twiddle table, then the k_0
-// and km_0 tables.
+// and km_0 tables.  The run-time kernels are held to 128 VGPRs, two blocks a
+// CU: at 179 x 181 x 173 that spills a few and takes 69 us instead of 85.
 // KIN: the source.  0: rows of n2p of f[0] after the y pass; 1: the full
 // spectrum sp.modes (rows of n2h) over sp.vol; 2: sp.ca times that plus sp.cb
 // times the x transform of sp.f (rows of n2p).
 template <bool POW2, int LN, int KIN = 0>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V) : GEN_MAXTPB) poisson_x_k(Fields3 fl, int n0_, int n1, int n2h, int n2p,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), pfft_v(LN)) : GEN_MAXTPB, LN ? 1 : 4) poisson_x_k(Fields3 fl, int n0_, int n1, int n2h, int n2p,
                                                        int B_, KTab kt, const float2* __restrict__ tw,
                                                        SpecSrc sp) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, PFFT_CAP) : 1;
-  constexpr int TPB = LN ? ct_tpb(LN, BC, PFFT_V) : GEN_TPB;
-  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
-  const int n0 = LN ? 1 << LN : n0_;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, pfft_v(LN)) : GEN_TPB;
+  constexpr int MAXV = LN ? BC * ct_n(LN) / TPB : GEN_MAXV;
+  const int n0 = LN ? ct_n(LN) : n0_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
   float2* stw = s + n0 * B;
@@ -475,16 +469,14 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
       if constexpr (KIN == 2) r[it] = sp.f[off + cm.b + (long long)cm.j0 * es + it * gs];
     }
   }
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = r[it];
+  float2 m[MAXV];
   if constexpr (KIN == 2) {
 #pragma unroll
     for (int it = 0; it < MAXV; ++it)
-      if (live && cm.j0 + it * cm.js < n0) r[it] = gm[it * ms];
+      if (live && cm.j0 + it * cm.js < n0) m[it] = gm[it * ms];
   }
-  __syncthreads();
-  if constexpr (KIN != 1) fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
+  if constexpr (KIN != 1) fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB>(r, s, n0, B, stw, cm);
+  else __syncthreads();  // the tables are read below
   const float ky = kt.k[1][y];
   const float kz = live ? kt.k[2][c0 + cm.b] : 0.f;
   float2 h[MAXV];
@@ -493,10 +485,10 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
     const int j = cm.j0 + it * cm.js;
     h[it] = make_float2(0.f, 0.f);
     if (live && j < n0) {
-      float2 v = s[threadIdx.x + it * tpb<TPB>()];
+      float2 v = r[it];
       if constexpr (KIN == 1) v = make_float2(v.x / sp.vol, v.y / sp.vol);
       if constexpr (KIN == 2)
-        v = make_float2(sp.ca * (r[it].x / sp.vol) + sp.cb * v.x, sp.ca * (r[it].y / sp.vol) + sp.cb * v.y);
+        v = make_float2(sp.ca * (m[it].x / sp.vol) + sp.cb * v.x, sp.ca * (m[it].y / sp.vol) + sp.cb * v.y);
       float kx = sk[j];
       float k2 = kx * kx;
       k2 = k2 + ky * ky;
@@ -508,37 +500,26 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
       }
     }
   }
-  __syncthreads();
   // x component: IFFT_x(km_0 h) to c_0
 #pragma unroll
   for (int it = 0; it < MAXV; ++it) {
     const int j = cm.j0 + it * cm.js;
     if (j < n0) {
       const float kmx = skm[j];
-      s[threadIdx.x + it * tpb<TPB>()] = make_float2(kmx * h[it].x, kmx * h[it].y);
+      r[it] = make_float2(kmx * h[it].x, kmx * h[it].y);
     }
   }
   __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) r[it] = s[threadIdx.x + it * tpb<TPB>()];
-  __syncthreads();
-  // h to c_1
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = h[it];
+  fft_cols<1, POW2, LN, ilog2c(BC), MAXV, TPB>(r, s, n0, B, stw, cm);
 #pragma unroll
   for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n0) g0[it * gs] = r[it];
   __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
+  // h to c_1
+  fft_cols<1, POW2, LN, ilog2c(BC), MAXV, TPB>(h, s, n0, B, stw, cm);
 #pragma unroll
   for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) r[it] = s[threadIdx.x + it * tpb<TPB>()];
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (live && cm.j0 + it * cm.js < n0) g1[it * gs] = r[it];
+    if (live && cm.j0 + it * cm.js < n0) g1[it * gs] = h[it];
 }
 
 // Adjoint x pass: acc = sum_d (-i km_d) laplace(FFT_x c_d); inverse FFT
@@ -549,13 +530,13 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
 // LDS block (the first result kept in registers), then the inverse of the
 // sum.  LDS as poisson_x_k.
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V) : GEN_MAXTPB) poisson_x_adj_k(Fields3 fl, int n0_, int n1, int n2h, int n2p,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), pfft_v(LN)) : GEN_MAXTPB, LN ? 1 : 4) poisson_x_adj_k(Fields3 fl, int n0_, int n1, int n2h, int n2p,
                                                            int B_, KTab kt, const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, PFFT_CAP) : 1;
-  constexpr int TPB = LN ? ct_tpb(LN, BC, PFFT_V) : GEN_TPB;
-  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
-  const int n0 = LN ? 1 << LN : n0_;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, pfft_v(LN)) : GEN_TPB;
+  constexpr int MAXV = LN ? BC * ct_n(LN) / TPB : GEN_MAXV;
+  const int n0 = LN ? ct_n(LN) : n0_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
   float2* stw = s + n0 * B;
@@ -583,28 +564,15 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
     x0[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n0) x0[it] = g0[it * gs];
   }
+  float2 yz[MAXV];
 #pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = x0[it];
-  __syncthreads();
-  fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
-  {
-    float2 yz[MAXV];
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it) {
-      yz[it] = make_float2(0.f, 0.f);
-      if (live && cm.j0 + it * cm.js < n0) yz[it] = g1[it * gs];
-    }
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it)
-      if (cm.j0 + it * cm.js < n0) x0[it] = s[threadIdx.x + it * tpb<TPB>()];
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it)
-      if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = yz[it];
+  for (int it = 0; it < MAXV; ++it) {
+    yz[it] = make_float2(0.f, 0.f);
+    if (live && cm.j0 + it * cm.js < n0) yz[it] = g1[it * gs];
   }
+  fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB>(x0, s, n0, B, stw, cm);
   __syncthreads();
-  fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
+  fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB>(yz, s, n0, B, stw, cm);
   const float ky = kt.k[1][y];
   const float kz = live ? kt.k[2][c0 + cm.b] : 0.f;
   float2 acc[MAXV];
@@ -619,7 +587,7 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
       k2 = k2 + kz * kz;
       if (k2 != 0.f) {
         const float kmx = skm[j];
-        const float2 w = s[threadIdx.x + it * tpb<TPB>()];
+        const float2 w = yz[it];
         float sx = kmx * x0[it].x + w.x, sy = kmx * x0[it].y + w.y;
         // pot = -sum / k^2, acc = -i pot = (pot.y, -pot.x)
         const float q = 1.f / k2;
@@ -628,14 +596,7 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
     }
   }
   __syncthreads();
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = acc[it];
-  __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n0) acc[it] = s[threadIdx.x + it * tpb<TPB>()];
+  fft_cols<1, POW2, LN, ilog2c(BC), MAXV, TPB>(acc, s, n0, B, stw, cm);
 #pragma unroll
   for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n0) g0[it * gs] = acc[it];
@@ -656,14 +617,14 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
 // of c_2, then their combination km_1 FFT_y(c_1) + km_2 FFT_y(c_2) to c_1
 // for poisson_x_adj_k.
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) : GEN_MAXTPB, 2) y_inv_seq_k(Fields3 fl, int n_, long long es,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(1, LN)) : GEN_MAXTPB, LN ? 2 : 4) y_inv_seq_k(Fields3 fl, int n_, long long es,
                                                         long long ostride, int ncol, int B_,
                                                         KTab kt, const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, FFT_CAP) : 1;
-  constexpr int TPB = LN ? ct_tpb(LN, BC, FFT_V) : GEN_TPB;
-  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
-  const int n = LN ? 1 << LN : n_;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, fft_v(1, LN)) : GEN_TPB;
+  constexpr int MAXV = LN ? BC * ct_n(LN) / TPB : GEN_MAXV;
+  const int n = LN ? ct_n(LN) : n_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
   float2* stw = s + n * B;
@@ -690,41 +651,31 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) :
     const int j = cm.j0 + it * cm.js;
     if (j < n) {
       const float kmy = kt.km[1][j];
-      s[threadIdx.x + it * tpb<TPB>()] = make_float2(kmy * h[it].x, kmy * h[it].y);
+      r[it] = make_float2(kmy * h[it].x, kmy * h[it].y);
     }
   }
-  __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * tpb<TPB>()];
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n)
-      s[threadIdx.x + it * tpb<TPB>()] = make_float2(kmz * h[it].x, kmz * h[it].y);
+  fft_cols<1, POW2, LN, ilog2c(BC), MAXV, TPB>(r, s, n, B, stw, cm);
 #pragma unroll
   for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n) g1[it * gs] = r[it];
+#pragma unroll
+  for (int it = 0; it < MAXV; ++it) h[it] = make_float2(kmz * h[it].x, kmz * h[it].y);
   __syncthreads();
-  fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
+  fft_cols<1, POW2, LN, ilog2c(BC), MAXV, TPB>(h, s, n, B, stw, cm);
 #pragma unroll
   for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) r[it] = s[threadIdx.x + it * tpb<TPB>()];
-#pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (live && cm.j0 + it * cm.js < n) g2[it * gs] = r[it];
+    if (live && cm.j0 + it * cm.js < n) g2[it * gs] = h[it];
 }
 
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) : GEN_MAXTPB, 2) y_fwd_seq_k(Fields3 fl, int n_, long long es,
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(-1, LN)) : GEN_MAXTPB, LN ? 2 : 4) y_fwd_seq_k(Fields3 fl, int n_, long long es,
                                                         long long ostride, int ncol, int B_,
                                                         KTab kt, const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, FFT_CAP) : 1;
-  constexpr int TPB = LN ? ct_tpb(LN, BC, FFT_V) : GEN_TPB;
-  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
-  const int n = LN ? 1 << LN : n_;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, fft_v(-1, LN)) : GEN_TPB;
+  constexpr int MAXV = LN ? BC * ct_n(LN) / TPB : GEN_MAXV;
+  const int n = LN ? ct_n(LN) : n_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
   float2* stw = s + n * B;
@@ -746,35 +697,21 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), FFT_V) :
     a[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n) a[it] = g1[it * gs];
   }
+  float2 c[MAXV];
 #pragma unroll
-  for (int it = 0; it < MAXV; ++it)
-    if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * tpb<TPB>()] = a[it];
-  __syncthreads();
-  fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
-  {
-    float2 c[MAXV];
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it) {
-      c[it] = make_float2(0.f, 0.f);
-      if (live && cm.j0 + it * cm.js < n) c[it] = g2[it * gs];
-    }
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it)
-      if (cm.j0 + it * cm.js < n) a[it] = s[threadIdx.x + it * tpb<TPB>()];
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it)
-      if (cm.j0 + it * cm.js < n) s[threadIdx.x + it * tpb<TPB>()] = c[it];
+  for (int it = 0; it < MAXV; ++it) {
+    c[it] = make_float2(0.f, 0.f);
+    if (live && cm.j0 + it * cm.js < n) c[it] = g2[it * gs];
   }
+  fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB>(a, s, n, B, stw, cm);
   __syncthreads();
-  fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n, B, stw);
+  fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB>(c, s, n, B, stw, cm);
 #pragma unroll
   for (int it = 0; it < MAXV; ++it) {
     const int j = cm.j0 + it * cm.js;
     if (j < n) {
-      const float2 c = s[threadIdx.x + it * tpb<TPB>()];
       const float kmy = kt.km[1][j];
-      a[it] = make_float2(kmy * a[it].x + kmz * c.x, kmy * a[it].y + kmz * c.y);
+      a[it] = make_float2(kmy * a[it].x + kmz * c[it].x, kmy * a[it].y + kmz * c[it].y);
     }
   }
 #pragma unroll
@@ -814,7 +751,7 @@ int pmx_fold_deferrable(const pmx_ctx* c) {
   if (t.tx != 16 || t.ty != 16 || t.tz != 16) return 0;
   if (c->n[0] % 16 || c->n[1] % 16 || c->n[2] % 16) return 0;
   const RowPlan r = row_plan(c->n[2], (long long)c->n[0] * c->n[1]);
-  return r.lh > 0 && c->n[1] % r.P == 0;
+  return r.lh > 0 && !ct_three(r.lh) && c->n[1] % r.P == 0;
 }
 
 static RowFields row_fields(const pmx_ctx* c, float* const* f, int nf, const int* rev, unsigned nblk,
@@ -859,8 +796,8 @@ int pmx_fft_r2c_rows(pmx_ctx* c, float* const* f, int nf, int pre, float coef, c
       rf, nrows, n2, c->rs, r.P, coef, c->tw[2], fi, fc)
 #define R2C_SM(L, SM)                                   \
   do {                                                  \
-    if (halo && pre) R2C(1, L, SM, (L > 0), true);      \
-    else if (halo) R2C(0, L, SM, (L > 0), true);        \
+    if (halo && pre) R2C(1, L, SM, (L > 0 && L < 32), true);      \
+    else if (halo) R2C(0, L, SM, (L > 0 && L < 32), true);        \
     else if (pre) R2C(1, L, SM, false, true);           \
     else R2C(0, L, SM, false, true);                    \
   } while (0)
@@ -869,7 +806,7 @@ int pmx_fft_r2c_rows(pmx_ctx* c, float* const* f, int nf, int pre, float coef, c
   else R2C_SM(L, false)
 #define R2C_FULL(PRE, P2)                                                              \
   z_r2c_k<PRE, P2><<<grid, r.tpb, r.lds, c->stream>>>(rf, nrows, n2, c->rs, r.P, coef, c->tw[2], fc)
-  if (r.half && is_pow2(r.len)) {
+  if (r.lh || (r.half && is_pow2(r.len))) {
     PMX_CT_SWITCH(r.lh, R2C_HALF);
   } else if (r.half) {
     if (pre) R2C(1, 0, false, false, false);
@@ -910,7 +847,7 @@ int pmx_fft_c2r_rows(pmx_ctx* c, float* const* f, int nf, float scale, const int
   else C2R(L, false, true)
 #define C2R_FULL(P2) \
   z_c2r_k<P2><<<grid, r.tpb, r.lds, c->stream>>>(rf, nrows, n2, c->rs, r.P, scale, c->tw[2])
-  if (r.half && is_pow2(r.len)) {
+  if (r.lh || (r.half && is_pow2(r.len))) {
     PMX_CT_SWITCH(r.lh, C2R_HALF);
   } else if (r.half) {
     C2R(0, false, false);
@@ -976,9 +913,9 @@ int pmx_strided_from_to(pmx_ctx* c, float2* const* src, int srow, float2* const*
   const int n = c->n[axis];
   const int ncol = c->n2h;
   const unsigned nouter = axis == 1 ? c->n[0] : c->n[1];
-  const int ln = ct_log2(n);
+  const int ln = ct_code(n);
   const int B = ln ? ct_cols(ln, FFT_CAP) : gen_cols(n, ncol, (long long)nouter * nf);
-  const int tpb = ln ? ct_tpb(ln, B, FFT_V) : gen_tpb(n * B);
+  const int tpb = ln ? ct_tpb(ln, B, fft_v(dir, ln)) : gen_tpb(n * B);
   dim3 grid((ncol + B - 1) / B, nouter, nf);
   size_t lds = lds_bytes(n, B) + tw_bytes(n);
   if (int rc = fft_fits("strided FFT", n, n * B, ln ? FFT_CAP : GEN_CAP, lds)) return rc;
@@ -1014,9 +951,9 @@ int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev) {
   Fields3 fl = {{f[0], f[1], f[2]}, rev};
   const int n = c->n[1];
   const int ncol = c->n2h;
-  const int ln = ct_log2(n);
+  const int ln = ct_code(n);
   const int B = ln ? ct_cols(ln, FFT_CAP) : gen_cols(n, ncol, c->n[0]);
-  const int tpb = ln ? ct_tpb(ln, B, FFT_V) : gen_tpb(n * B);
+  const int tpb = ln ? ct_tpb(ln, B, fft_v(dir, ln)) : gen_tpb(n * B);
   const long long es = c->n2p, ostride = (long long)n * c->n2p;
   dim3 grid((ncol + B - 1) / B, c->n[0], 1);
   const size_t lds = lds_bytes(n, B) + tw_bytes(n);
@@ -1044,9 +981,9 @@ int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev) {
 int pmx_poisson_x(pmx_ctx* c, float2* const* f, int adjoint, const SpecSrc* src, int rev) {
   Fields3 fl = {{f[0], f[1], f[2]}, rev};
   const int n0 = c->n[0];
-  const int ln = ct_log2(n0);
+  const int ln = ct_code(n0);
   const int B = ln ? ct_cols(ln, PFFT_CAP) : gen_cols(n0, c->n2h, c->n[1]);
-  const int tpb = ln ? ct_tpb(ln, B, PFFT_V) : gen_tpb(n0 * B);
+  const int tpb = ln ? ct_tpb(ln, B, pfft_v(ln)) : gen_tpb(n0 * B);
   dim3 grid((c->n2h + B - 1) / B, c->n[1], 1);
   // the data block, the twiddles, then the k_0 and km_0 tables
   size_t lds = lds_bytes(n0, B) + tw_bytes(n0) + 2 * (size_t)n0 * sizeof(float);

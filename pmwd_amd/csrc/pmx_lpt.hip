@@ -35,14 +35,14 @@ __device__ __forceinline__ float strain_f(int set, int o, float kx, float ky, fl
 // along x.  One read of the modes serves the three: pot stays in registers.
 // 8 values a thread, as poisson_x_k.
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V) : GEN_MAXTPB)
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), pfft_v(LN)) : GEN_MAXTPB)
     lpt_x_k(Fields3 fl, const float2* __restrict__ modes, int n0_, int n1, int n2h, int n2p, int B_,
             KTab kt, const float2* __restrict__ tw, float cell_vol, int set) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, PFFT_CAP) : 1;
-  constexpr int TPB = LN ? ct_tpb(LN, BC, PFFT_V) : GEN_TPB;
-  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
-  const int n0 = LN ? 1 << LN : n0_;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, pfft_v(LN)) : GEN_TPB;
+  constexpr int MAXV = LN ? BC * ct_n(LN) / TPB : GEN_MAXV;
+  const int n0 = LN ? ct_n(LN) : n0_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
   float2* stw = s + n0 * B;
@@ -84,21 +84,17 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
   const long long es = (long long)n1 * n2p;
   const long long o0 = (long long)y * n2p + c0 + cm.b + (long long)cm.j0 * es;
   for (int o = 0; o < 3; ++o) {
+    float2 r[MAXV];
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
       const int j = cm.j0 + it * cm.js;
       if (j >= n0) continue;
       const float f = strain_f(set, o, sk[j], ky, kz, skm[j], my, mz);
-      s[threadIdx.x + it * tpb<TPB>()] = make_float2(f * pot[it].x, f * pot[it].y);
+      r[it] = make_float2(f * pot[it].x, f * pot[it].y);
     }
-    __syncthreads();
-    fft_run<1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
+    if (o) __syncthreads();
+    fft_cols<1, POW2, LN, ilog2c(BC), MAXV, TPB>(r, s, n0, B, stw, cm);
     float2* d = (o == 0 ? fl.f[0] : (o == 1 ? fl.f[1] : fl.f[2])) + o0;
-    float2 r[MAXV];
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it)
-      if (cm.j0 + it * cm.js < n0) r[it] = s[threadIdx.x + it * tpb<TPB>()];
-    __syncthreads();
 #pragma unroll
     for (int it = 0; it < MAXV; ++it)
       if (live && cm.j0 + it * cm.js < n0) d[(long long)it * cm.js * es] = r[it];
@@ -110,14 +106,14 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
 // times -w scale / k^2, w = 2 on the last axis' interior columns (those that
 // stand for two of the full spectrum), 0 at k = 0.
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V) : GEN_MAXTPB)
+__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), pfft_v(LN)) : GEN_MAXTPB)
     lpt_x_adj_k(Fields3 fl, float2* __restrict__ out, int n0_, int n1, int n2, int n2h, int n2p,
                 int B_, KTab kt, const float2* __restrict__ tw, float scale, int set, int first) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, PFFT_CAP) : 1;
-  constexpr int TPB = LN ? ct_tpb(LN, BC, PFFT_V) : GEN_TPB;
-  constexpr int MAXV = LN ? (BC << LN) / TPB : GEN_MAXV;
-  const int n0 = LN ? 1 << LN : n0_;
+  constexpr int TPB = LN ? ct_tpb(LN, BC, pfft_v(LN)) : GEN_TPB;
+  constexpr int MAXV = LN ? BC * ct_n(LN) / TPB : GEN_MAXV;
+  const int n0 = LN ? ct_n(LN) : n0_;
   const int B = LN ? BC : B_;
   const int lB = LN ? ilog2c(BC) : __ffs(B_) - 1;
   float2* stw = s + n0 * B;
@@ -149,17 +145,13 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), PFFT_V)
       r[it] = make_float2(0.f, 0.f);
       if (live && cm.j0 + it * cm.js < n0) r[it] = g[(long long)it * cm.js * es];
     }
-    __syncthreads();  // the last transform's results are read
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it)
-      if (cm.j0 + it * cm.js < n0) s[threadIdx.x + it * tpb<TPB>()] = r[it];
-    __syncthreads();
-    fft_run<-1, COLS, POW2, LN, ilog2c(BC), MAXV, TPB>(s, n0, B, stw);
+    if (o) __syncthreads();
+    fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB>(r, s, n0, B, stw, cm);
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
       const int j = cm.j0 + it * cm.js;
       if (j >= n0) continue;
-      const float2 v = s[threadIdx.x + it * tpb<TPB>()];
+      const float2 v = r[it];
       if (set == 2) {
         const float km = o == 0 ? skm[j] : (o == 1 ? my : mz);
         t[it].x -= km * v.y;
@@ -233,8 +225,8 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
   extern __shared__ float2 s[];
   constexpr int PC = LH ? ct_rows(LH, SM) : 1;
   constexpr int TPB = LH ? ct_row_tpb(LH, SM) : GEN_TPB;
-  constexpr int MAXV = LH ? (PC << LH) / TPB : GEN_MAXV;
-  const int H = LH ? 1 << LH : n2 >> 1;
+  constexpr int MAXV = LH ? PC * ct_n(LH) / TPB : GEN_MAXV;
+  const int H = LH ? ct_n(LH) : n2 >> 1;
   const int P = LH ? PC : P_;
   const RowSplit<LH> rsp(H);
   float2* stw = s + lds_elems(ROWS, H, P);
@@ -447,9 +439,9 @@ static int lpt_x(pmx_ctx* c, float2* const* f, int set, const float* in, float c
                  float scale, int first) {
   const Fields3 fl = {{f[0], f[1], f[2]}, 0};
   const int n0 = c->n[0];
-  const int ln = ct_log2(n0);
+  const int ln = ct_code(n0);
   const int B = ln ? ct_cols(ln, PFFT_CAP) : gen_cols(n0, c->n2h, c->n[1]);
-  const int tpb = ln ? ct_tpb(ln, B, PFFT_V) : gen_tpb(n0 * B);
+  const int tpb = ln ? ct_tpb(ln, B, pfft_v(ln)) : gen_tpb(n0 * B);
   const dim3 grid((c->n2h + B - 1) / B, c->n[1], 1);
   const size_t lds = lds_bytes(n0, B) + tw_bytes(n0) + 2 * (size_t)n0 * sizeof(float);
   if (int rc = fft_fits("2LPT x pass", n0, n0 * B, PFFT_CAP, lds)) return rc;
@@ -486,7 +478,7 @@ static int lpt_rows_fused(pmx_ctx* c, const LptRows& q, const RowPlan& r) {
   lpt_rows_k<OP, L, SM, P2><<<nblk, r.tpb, r.lds, c->stream>>>(q, nrows, c->n[0], c->n[1],      \
                                                                c->n[2], c->rs, r.P, c->tw[2])
 #define LROWS_P2(L) LROWS(L, (L > 0), true)
-  if (is_pow2(r.len)) {
+  if (r.lh || is_pow2(r.len)) {
     PMX_CT_SWITCH(r.lh, LROWS_P2);
   } else {
     LROWS(0, false, false);

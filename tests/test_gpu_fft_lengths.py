@@ -13,7 +13,10 @@ pytestmark = pytest.mark.gpu
 # fixed lengths 32 and up in small and large row blocks; a single row pair
 SHAPES = [(6, 9, 10), (14, 15, 18), (11, 26, 13), (17, 34, 51), (19, 62, 127), (49, 121, 25),
           (24, 96, 48), (150, 45, 30), (20, 180, 210), (32, 32, 64), (33, 32, 64), (3, 5, 64),
-          (8, 512, 128), (96, 192, 66), (1, 3, 375), (1, 1, 9), (5, 1, 2), (2, 2, 4095)]
+          (8, 512, 128), (96, 192, 66), (1, 3, 375), (1, 1, 9), (5, 1, 2), (2, 2, 4095),
+          # 3 2^k of fixed length in each axis, small, large and left-over row blocks
+          (96, 192, 384), (384, 96, 192), (8, 768, 66), (768, 6, 768), (40, 24, 1536),
+          (192, 192, 192), (5, 7, 192)]
 
 
 def _rel(a, b):

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 # fixed and run-time lengths on each axis, small and large row blocks, odd
 # rows, an axis of one
 SHAPES = [(16, 16, 16), (64, 128, 256), (12, 10, 8), (9, 8, 10), (8, 9, 15), (20, 33, 66),
-          (64, 64, 128), (1, 24, 6), (130, 128, 128)]
+          (64, 64, 128), (1, 24, 6), (130, 128, 128), (96, 96, 192)]
 
 
 def rel(a, b):
