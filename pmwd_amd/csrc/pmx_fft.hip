@@ -422,7 +422,7 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(DI
 // axis 0 of (n0,n1,n2h); blockIdx.y = y index, blockIdx.x = block of B kz
 // columns.  LDS: the n0 x B block, the n0-entry twiddle table, then the k_0
 // and km_0 tables.  The run-time kernels are held to 128 VGPRs, two blocks a
-// CU: at 179 x 181 x 173 that spills a few and takes 69 us instead of 85.
+// CU: at 150 x 180 x 210 that spills a few and takes 69 us instead of 85.
 // KIN: the source.  0: rows of n2p of f[0] after the y pass; 1: the full
 // spectrum sp.modes (rows of n2h) over sp.vol; 2: sp.ca times that plus sp.cb
 // times the x transform of sp.f (rows of n2p).
@@ -611,12 +611,13 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, PFFT_CAP), pfft_v(
 // Inverse: from h = IFFT_x(-i pot) in c_1, the y and z force components
 // IFFT_y(km_1 h) to c_1 and IFFT_y(km_2 h) to c_2 -- the products and
 // transforms of a separate y pass over km_1 h and km_2 h, with h read once
-// and kept in registers.
+// and kept in registers.  BOTH: the x
+// component's inverse (c_0 in place) runs in the same launch (pmx_fft_yinv).
 //
 // Forward (adjoint path, y_fwd_seq_k): FFT_y of c_1 (kept in registers) and
 // of c_2, then their combination km_1 FFT_y(c_1) + km_2 FFT_y(c_2) to c_1
 // for poisson_x_adj_k.
-template <bool POW2, int LN>
+template <bool POW2, int LN, int BOTH>
 __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(1, LN)) : GEN_MAXTPB, LN ? 2 : 4) y_inv_seq_k(Fields3 fl, int n_, long long es,
                                                         long long ostride, int ncol, int B_,
                                                         KTab kt, const float2* __restrict__ tw) {
@@ -630,6 +631,10 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(1,
   float2* stw = s + n * B;
   int bx, by, bz;
   xcd_block3(bx, by, bz, fl.rev);
+  // BOTH: odd rows of the grid are the x component's (alternating, so that
+  // every XCD's share of the blocks holds as many pairs)
+  const bool xc = BOTH && (by & 1);
+  by >>= BOTH;
   const int c0 = bx * B;
   const int nb = ncol - c0 < B ? ncol - c0 : B;
   const long long off = (long long)by * ostride + c0;
@@ -637,7 +642,7 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(1,
   const ColMap cm = col_map<TPB>(lB);
   const bool live = cm.b < nb;
   const float kmz = live ? kt.km[2][c0 + cm.b] : 0.f;
-  float2* g1 = fl.f[1] + off + cm.b + (long long)cm.j0 * es;
+  float2* g1 = (xc ? fl.f[0] : fl.f[1]) + off + cm.b + (long long)cm.j0 * es;
   float2* g2 = fl.f[2] + off + cm.b + (long long)cm.j0 * es;
   const long long gs = (long long)cm.js * es;
   float2 h[MAXV], r[MAXV];
@@ -651,13 +656,14 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(1,
     const int j = cm.j0 + it * cm.js;
     if (j < n) {
       const float kmy = kt.km[1][j];
-      r[it] = make_float2(kmy * h[it].x, kmy * h[it].y);
+      r[it] = xc ? h[it] : make_float2(kmy * h[it].x, kmy * h[it].y);
     }
   }
   fft_cols<1, POW2, LN, ilog2c(BC), MAXV, TPB>(r, s, n, B, stw, cm);
 #pragma unroll
   for (int it = 0; it < MAXV; ++it)
     if (live && cm.j0 + it * cm.js < n) g1[it * gs] = r[it];
+  if (xc) return;
 #pragma unroll
   for (int it = 0; it < MAXV; ++it) h[it] = make_float2(kmz * h[it].x, kmz * h[it].y);
   __syncthreads();
@@ -944,10 +950,10 @@ int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int
 }
 
 // Paired y pass of the gradient's y and z components: dir > 0 turns h in
-// f[1] into the two force components in f[1] and f[2] (y_inv_seq_k);
-// dir < 0 turns the cotangents in f[1] and f[2] into km_1 FFT_y(f[1]) +
-// km_2 FFT_y(f[2]) in f[1] (y_fwd_seq_k).
-int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev) {
+// f[1] into the two force components in f[1] and f[2] (y_inv_seq_k; both:
+// and inverts f[0]); dir < 0 turns the cotangents in f[1] and f[2] into km_1
+// FFT_y(f[1]) + km_2 FFT_y(f[2]) in f[1] (y_fwd_seq_k).
+static int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev, int both = 0) {
   Fields3 fl = {{f[0], f[1], f[2]}, rev};
   const int n = c->n[1];
   const int ncol = c->n2h;
@@ -955,27 +961,50 @@ int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev) {
   const int B = ln ? ct_cols(ln, FFT_CAP) : gen_cols(n, ncol, c->n[0]);
   const int tpb = ln ? ct_tpb(ln, B, fft_v(dir, ln)) : gen_tpb(n * B);
   const long long es = c->n2p, ostride = (long long)n * c->n2p;
-  dim3 grid((ncol + B - 1) / B, c->n[0], 1);
+  dim3 grid((ncol + B - 1) / B, c->n[0] << both, 1);
   const size_t lds = lds_bytes(n, B) + tw_bytes(n);
   if (int rc = fft_fits("paired y FFT", n, n * B, ln ? FFT_CAP : GEN_CAP, lds)) return rc;
   const KTab kt = ktab(c);
   const bool p2 = is_pow2(n);
   const int cls = dir < 0 ? PMX_T_YFWD : PMX_T_YINV;
   pmx_tic(c, cls);
+#define YINV1(P2, L, BOTH) \
+  y_inv_seq_k<P2, L, BOTH><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1])
+#define YINV(P2, L)        \
+  do {                     \
+    if (both) YINV1(P2, L, 1); \
+    else YINV1(P2, L, 0);  \
+  } while (0)
 #define YPAIR(L)                                                                                  \
   if (dir < 0 && (L || p2))                                                                       \
     y_fwd_seq_k<true, L><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
   else if (dir < 0)                                                                               \
     y_fwd_seq_k<false, 0><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
   else if (L || p2)                                                                               \
-    y_inv_seq_k<true, L><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1]); \
+    YINV(true, L); \
   else                                                                                            \
-    y_inv_seq_k<false, 0><<<grid, tpb, lds, c->stream>>>(fl, n, es, ostride, ncol, B, kt, c->tw[1])
+    YINV(false, 0)
   PMX_CT_SWITCH(ln, YPAIR);
 #undef YPAIR
+#undef YINV
+#undef YINV1
   pmx_toc(c, cls);
   PMX_LAUNCH_CHECK();
   return PMX_OK;
+}
+
+// The inverse y passes of the three components after poisson_x_k.  Meshes of
+// few blocks take them in one launch (128^3, 640 blocks: 18.4 -> 12.3 us);
+// larger ones keep one mesh's and the pair's streams apart (256^3, 2304
+// blocks: 63 against 67; 512^3: 664 against 687, and their z pass 679 against
+// 730, as the pair's meshes are then the last ones written).
+int pmx_fft_yinv(pmx_ctx* c, float2* const* f, int rev) {
+  const int ln = ct_code(c->n[1]);
+  const int B = ln ? ct_cols(ln, FFT_CAP) : gen_cols(c->n[1], c->n2h, c->n[0]);
+  if ((long long)((c->n2h + B - 1) / B) * c->n[0] < 2 * FFT_MIN_WGS)
+    return pmx_fft_ypair(c, f, 1, rev, 1);
+  if (int rc = pmx_fft_strided(c, f, 1, 1, 1, rev)) return rc;
+  return pmx_fft_ypair(c, f, 1, 1 - rev);
 }
 
 int pmx_poisson_x(pmx_ctx* c, float2* const* f, int adjoint, const SpecSrc* src, int rev) {
@@ -1028,8 +1057,7 @@ int pmx_poisson_ctx(pmx_ctx* c, float coef, int deferred) {
   if ((rc = pmx_fft_r2c_inplace(c, (float*)f[0], 1, coef, halo, 1))) return rc;
   if ((rc = pmx_fft_strided(c, f, 1, 1, -1, 0))) return rc;
   if ((rc = pmx_poisson_x(c, f, 0, nullptr, 1))) return rc;
-  if ((rc = pmx_fft_strided(c, f, 1, 1, 1, 0))) return rc;
-  if ((rc = pmx_fft_ypair(c, f, 1, 1))) return rc;
+  if ((rc = pmx_fft_yinv(c, f, 0))) return rc;
   float scale = (float)(1.0 / (double)c->M);
   float* z[3] = {(float*)f[1], (float*)f[2], (float*)f[0]};
   const int rev[3] = {0, 1, 1};

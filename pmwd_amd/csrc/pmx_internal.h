@@ -1087,7 +1087,7 @@ int pmx_fft_r2c_rows(pmx_ctx* c, float* const* f, int nf, int pre, float coef, c
 int pmx_fft_c2r_rows(pmx_ctx* c, float* const* f, int nf, float scale, const int* rev,
                      float* const* real, int ors);
 int pmx_fft_strided(pmx_ctx* c, float2* const* f, int nf, int axis, int dir, int rev = 0);
-int pmx_fft_ypair(pmx_ctx* c, float2* const* f, int dir, int rev = 0);
+int pmx_fft_yinv(pmx_ctx* c, float2* const* f, int rev);
 // copies n0*n1 rows of ncols floats between row strides (ncols <= 0: n2)
 int pmx_copy_rows(pmx_ctx* c, float* dst, int dst_rs, const float* src, int src_rs, int ncols = 0);
 int pmx_poisson_adj_ctx(pmx_ctx* c, float scale_out, int deferred = 0);

@@ -540,8 +540,7 @@ static int strains(pmx_ctx* c, float2* const* f, int set, const float* modes, fl
 static int lpt_move(pmx_ctx* c, float2* const* f, const SpecSrc& src, const LptOut& out) {
   int rc;
   if ((rc = pmx_poisson_x(c, f, 0, &src))) return rc;
-  if ((rc = pmx_fft_strided(c, f, 1, 1, 1))) return rc;
-  if ((rc = pmx_fft_ypair(c, f, 1))) return rc;
+  if ((rc = pmx_fft_yinv(c, f, 0))) return rc;
   return lpt_rows(c, LPT_MOVE, {{f[0], f[1], f[2]}, nullptr, 0.f, out});
 }
 
