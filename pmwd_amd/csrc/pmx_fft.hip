@@ -4,8 +4,8 @@
 // r2c/c2r row passes run in place; the complex mesh is (n0, n1, n2h) float2 in rows of n2p >= n2h.
 // Each kernel stages P pencils of length n in LDS (pencil-major for the
 // contiguous row passes, interleaved for the strided passes) and runs a
-// Stockham autosort FFT with radix 8/4/2 stages, or a direct DFT for lengths
-// that are not powers of two.
+// Stockham autosort FFT: radix 8/4/2 stages for powers of two, mixed radices
+// for other lengths (pmx_fft.h).
 //
 // Pass order (forward): z r2c (rows, contiguous) -> y (strided) -> x
 // (strided).  The x pass of the Poisson solve does forward x FFT, Green's
@@ -182,9 +182,9 @@ __device__ __forceinline__ float2 fold_pair(float2 v, const FoldIn& fi, int x, i
 // S = 4 term and Z1[p + P tz] the S = 5 or S = 6 term of cell (p, 16 tz),
 // one each per thread (P * H / 8 <= TPB of them).  All of it is issued before
 // the row loads, so no wait falls between two of them.
-template <int P, int TPB>
-__device__ __forceinline__ void fold_tables(const FoldIn& fi, int x, int y0, int lH, int H, float* T,
-                                            float& z0, float& z1) {
+template <int P, int TPB, int H>
+__device__ __forceinline__ void fold_tables(const FoldIn& fi, int x, int y0, float* T, float& z0,
+                                            float& z1) {
   typedef __attribute__((address_space(1))) const void gptr;
   typedef __attribute__((address_space(3))) void lptr;
   constexpr int lP = ilog2c(P);
@@ -205,13 +205,15 @@ __device__ __forceinline__ void fold_tables(const FoldIn& fi, int x, int y0, int
         z1 = tile(tx, tym, tzm)[289 + lx * 17 + 16];
     }
   }
-  // a wave's 64 entries lie in one row (2H >= 128), so the face-row test is
-  // wave-uniform; lane l of a wave writes the LDS word at its base plus l
-  const int n2 = 2 * H, wave0 = j & ~63;
+  // a wave's 64 entries lie in one row (2H a multiple of 64), so the face-row
+  // test is wave-uniform; lane l of a wave writes the LDS word at its base plus l
+  static_assert(2 * H % 64 == 0 && TPB % 64 == 0 && P * (H >> 3) <= TPB, "fold tables");
+  constexpr int n2 = 2 * H;
+  const int wave0 = j & ~63;
   for (int e0 = 0; e0 < P * n2; e0 += TPB) {
     const int e = e0 + j;
     if (e >= P * n2) break;
-    const int p = e >> (lH + 1), z = e & (n2 - 1);
+    const int p = (unsigned)e / n2, z = (unsigned)e % n2;
     const int y = y0 + p, ly = y & 15, ty = y >> 4;
     if ((lx == 0) == (ly == 0)) continue;
     const float* src = lx == 0 ? tile(txm, ty, z >> 4) + ly * 17 + (z & 15)
@@ -221,22 +223,21 @@ __device__ __forceinline__ void fold_tables(const FoldIn& fi, int x, int y0, int
 }
 
 // Adds the fold (fold_tables' terms, in pmx_fold_sum16's order) to a block's
-// NV values per thread (row p = idx >> lH, pair m = idx & (H - 1)).
-template <int NV, int TPB, int P>
-__device__ __forceinline__ void fold_rows(float2 (&r)[NV], const FoldIn& fi, int x, int y0, int lH,
-                                          int H, int total, const float* T, const float* Z0,
-                                          const float* Z1) {
+// NV values per thread (row p = idx / H, pair m = idx % H).
+template <int NV, int TPB, int P, int H>
+__device__ __forceinline__ void fold_rows(float2 (&r)[NV], const FoldIn& fi, int x, int y0, int total,
+                                          const float* T, const float* Z0, const float* Z1) {
   const int lx = x & 15;
 #pragma unroll
   for (int it = 0; it < NV; ++it) {
     const int idx = threadIdx.x + it * tpb<TPB>();
     if (idx >= total) continue;
-    const int p = idx >> lH, y = y0 + p, m = idx & (H - 1);
+    const int p = (unsigned)idx / H, y = y0 + p, m = (unsigned)idx % H;
     const int ly = y & 15, z = 2 * m, lz = z & 15, k = (m >> 3) * P + p;
     if (lx == 0 && ly == 0) {
       r[it] = fold_pair(r[it], fi, x, y, m);
     } else if (lx == 0 || ly == 0) {
-      const float* t = T + (p << (lH + 1)) + z;
+      const float* t = T + p * 2 * H + z;
       float sx = 0.f;
       sx += t[0];
       if (lz == 0) {
@@ -255,8 +256,9 @@ __device__ __forceinline__ void fold_rows(float2 (&r)[NV], const FoldIn& fi, int
   }
 }
 
-// FOLD (with H = 2^LH, 16^3 tiles, P | n1): the density is the deposit's tile
-// interiors plus the fold of fi.halo, added here on load.
+// FOLD (with LH > 0, 16^3 tiles, P | n1): the density is the deposit's tile
+// interiors plus the fold of fi.halo, added here on load (192^3: 27 us, where
+// the pass and a fold pass took 18 + 33; 512^3: 243).
 template <int PRE, int LH, bool SM, bool FOLD, bool POW2>
 __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
     z_r2c_half_k(RowFields rf, long long nrows, int n2, int rs, int P_, float coef,
@@ -293,7 +295,7 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
     float* Z0 = T + PC * 2 * H;
     float* Z1 = Z0 + PC * (H >> 3);
     float z0 = 0.f, z1 = 0.f;
-    if (FOLD) fold_tables<PC, TPB>(fi, fx, fy0, LH, H, T, z0, z1);
+    if constexpr (FOLD) fold_tables<PC, TPB, ct_n(LH)>(fi, fx, fy0, T, z0, z1);
     float2 r[MAXV];
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
@@ -301,14 +303,14 @@ __global__ void __launch_bounds__(LH ? ct_row_tpb(LH, SM) : GEN_MAXTPB, 4)
       const int p = rsp.row(idx);
       if (idx < total) r[it] = src[__umul24(p, orc) + rsp.col(idx, p)];
     }
-    if (FOLD) {
+    if constexpr (FOLD) {
       if ((int)threadIdx.x < PC * (H >> 3)) {
         Z0[threadIdx.x] = z0;
         Z1[threadIdx.x] = z1;
       }
       __builtin_amdgcn_s_waitcnt(0);  // T's loads into LDS have landed
       __syncthreads();
-      fold_rows<MAXV, TPB, PC>(r, fi, fx, fy0, LH, H, total, T, Z0, Z1);
+      fold_rows<MAXV, TPB, PC, ct_n(LH)>(r, fi, fx, fy0, total, T, Z0, Z1);
       __syncthreads();  // T is read before the rows take its place
     }
     if (PRE) {
@@ -757,7 +759,7 @@ int pmx_fold_deferrable(const pmx_ctx* c) {
   if (t.tx != 16 || t.ty != 16 || t.tz != 16) return 0;
   if (c->n[0] % 16 || c->n[1] % 16 || c->n[2] % 16) return 0;
   const RowPlan r = row_plan(c->n[2], (long long)c->n[0] * c->n[1]);
-  return r.lh > 0 && !ct_three(r.lh) && c->n[1] % r.P == 0;
+  return r.lh > 0 && c->n[1] % r.P == 0;
 }
 
 static RowFields row_fields(const pmx_ctx* c, float* const* f, int nf, const int* rev, unsigned nblk,
@@ -802,8 +804,8 @@ int pmx_fft_r2c_rows(pmx_ctx* c, float* const* f, int nf, int pre, float coef, c
       rf, nrows, n2, c->rs, r.P, coef, c->tw[2], fi, fc)
 #define R2C_SM(L, SM)                                   \
   do {                                                  \
-    if (halo && pre) R2C(1, L, SM, (L > 0 && L < 32), true);      \
-    else if (halo) R2C(0, L, SM, (L > 0 && L < 32), true);        \
+    if (halo && pre) R2C(1, L, SM, (L > 0), true);      \
+    else if (halo) R2C(0, L, SM, (L > 0), true);        \
     else if (pre) R2C(1, L, SM, false, true);           \
     else R2C(0, L, SM, false, true);                    \
   } while (0)
