@@ -380,7 +380,8 @@ extern "C" int pmx_gather_cic_adj(pmx_ctx* c, const pmx_cic_geom* g, const int16
   if (rc) return rc;
   if (n == 0) return PMX_OK;
   PMX_REQUIRE(pmid && disp && mesh && val_cot, "pmx_gather_cic_adj: NULL pointer");
-  if (pmx_values_fit(c, g, nchan)) {
+  // few particles with a mesh cotangent: both in the one launch below
+  if (pmx_values_fit(c, g, nchan) && (!mesh_cot || n >= c->values_min)) {
     if (disp_cot && (rc = pmx_values_adj(c, pmid, disp, n, mesh, nchan, val_cot, 0.f, disp_cot, nullptr)))
       return rc;
     disp_cot = nullptr;

@@ -193,6 +193,8 @@ struct pmx_ctx {
   int halo_nch;        // channels the halo buffer holds
   int fold_on_load;    // the Poisson row pass may take the deposit's fold
                        // (environment PMX_FOLD_ON_LOAD=0 at creation: never)
+  long long values_min;  // particles from which values are scattered in tiles
+                         // (environment PMX_VALUES_MIN at creation)
   int deposit_split;   // several-channel deposits: a workgroup per tile and
                        // channel (environment PMX_DEPOSIT_SPLIT=0 at
                        // creation: the channels in turn in one workgroup)

@@ -14,6 +14,14 @@ pytestmark = pytest.mark.gpu
 CASES = [((16, 16, 32), 2), ((20, 12, 35), 1), ((5, 7, 9), 1), ((1, 17, 33), 1), ((24, 24, 24), 1.5)]
 
 
+@pytest.fixture(autouse=True)
+def in_tiles(monkeypatch):
+    """Contexts that scatter values in tiles at any particle count."""
+    from pmwd_amd import _lib
+    monkeypatch.setenv('PMX_VALUES_MIN', '0')
+    monkeypatch.setattr(_lib, '_ctx_cache', {})
+
+
 def _setup(dev, shape, ratio, std=2.0, seed=0):
     import pmwd_amd as pa
     conf = pa.Configuration(1.7, shape, mesh_shape=ratio)
@@ -115,3 +123,17 @@ def test_value_scatter_under_capture_without_scratch(dev):
         np.testing.assert_allclose(again.cpu().numpy(), want.cpu().numpy(), rtol=1e-5, atol=1e-5)
     del graph
     fresh.close()
+
+
+@pytest.mark.parametrize('n', [131071, 131072])
+def test_value_scatter_either_side_of_the_tile_rule(dev, n, monkeypatch):
+    """Few particles are scattered with atomics, more in tiles: the same
+    numbers to the scatter's tolerance."""
+    import pmwd_amd as pa
+    monkeypatch.delenv('PMX_VALUES_MIN')
+    conf, ptcl, pmid, disp, rng = _setup(dev, (64, 32, 65), 1, seed=3)
+    val = rng.standard_normal((n, 3)).astype(np.float32)
+    got = pa.scatter(ptcl[:n], conf, val=torch.as_tensor(val, device=dev)).cpu().numpy()
+    want = opm.scatter(pmid[:n], disp[:n], conf.cell_size, conf.mesh_shape, val=val.astype(np.float64),
+                       mesh=np.zeros(conf.mesh_shape + (3,)), dtype=np.float64)
+    assert np.linalg.norm(got - want) < 1e-6 * np.linalg.norm(want)
