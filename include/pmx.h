@@ -187,8 +187,13 @@ typedef struct {
 } pmx_cic_geom;
 
 /* pmwd/scatter.py:33-83 (any arguments): mesh (out_shape + (nchan,)) +=
- * val * w.  val is (n,nchan) or NULL for the scalar val_scalar.  Uses
- * global float atomics (not the hot path).                                  */
+ * val * w.  val is (n,nchan) or NULL for the scalar val_scalar.  Global float
+ * atomics; but many particles of up to three channels on the context's own
+ * mesh at the default geometry are binned by tile and accumulated in LDS.
+ * That takes 20 bytes of device memory per record slot, which the context
+ * keeps for these calls alone (until pmx_ctx_trim): no other call and no
+ * captured graph uses it.  Under graph capture, and where it cannot be
+ * allocated, they take the atomics.                                         */
 int pmx_scatter_cic(pmx_ctx* ctx, const pmx_cic_geom* g, const int16_t* pmid,
                     const float* disp, long long n, const float* val,
                     float val_scalar, int nchan, float* mesh);
@@ -207,7 +212,8 @@ int pmx_scatter_cic_adj(pmx_ctx* ctx, const pmx_cic_geom* g,
                         float* val_cot);
 /* pmwd/gather.py:80-142 (_gather_chunk_adj/_gather_bwd):
  * disp_cot (n,3) = sum_j (val_cot.mesh[c_j]) grad w_j / cell and
- * mesh_cot += scatter(val_cot * w) (either output may be NULL).            */
+ * mesh_cot += scatter(val_cot * w) as pmx_scatter_cic (either output may be
+ * NULL).                                                                    */
 int pmx_gather_cic_adj(pmx_ctx* ctx, const pmx_cic_geom* g,
                        const int16_t* pmid, const float* disp, long long n,
                        const float* mesh, const float* val_cot, int nchan,

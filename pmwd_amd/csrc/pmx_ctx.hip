@@ -110,18 +110,9 @@ static int dev_alloc(pmx_ctx* c, void** p, size_t bytes) {
   return PMX_OK;
 }
 
-static void dev_free(pmx_ctx* c, void** p, size_t bytes) {
+// Gives back memory that no captured graph addresses.
+static void dev_release(pmx_ctx* c, void** p, size_t bytes) {
   if (*p) {
-    // a captured graph addresses the context's scratch: it goes with it
-    if (c->gexec) {
-      (void)hipStreamSynchronize(c->stream);
-      (void)hipGraphExecDestroy(c->gexec);
-      c->gexec = nullptr;
-    }
-    if (c->graph) {
-      (void)hipGraphDestroy(c->graph);
-      c->graph = nullptr;
-    }
     if (c->dfree) {
       (void)hipStreamSynchronize(c->stream);
       c->dfree(*p, bytes, c->device, (void*)c->stream, c->dalloc_user);
@@ -131,6 +122,20 @@ static void dev_free(pmx_ctx* c, void** p, size_t bytes) {
     c->bytes -= bytes;
   }
   *p = nullptr;
+}
+
+static void dev_free(pmx_ctx* c, void** p, size_t bytes) {
+  // a captured graph addresses the context's scratch: it goes with it
+  if (*p && c->gexec) {
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipGraphExecDestroy(c->gexec);
+    c->gexec = nullptr;
+  }
+  if (*p && c->graph) {
+    (void)hipGraphDestroy(c->graph);
+    c->graph = nullptr;
+  }
+  dev_release(c, p, bytes);
 }
 
 int pmx_dev_alloc(pmx_ctx* c, void** p, size_t bytes) { return dev_alloc(c, p, bytes); }
@@ -337,6 +342,9 @@ extern "C" int pmx_ctx_destroy(pmx_ctx* c) {
                 c->red_out, c->sort_k[0], c->sort_k[1], c->sort_v[0], c->sort_v[1], c->sort_hist,
                 c->scan_tmp};
   for (void* p : ps) rel(p);
+  const BinScratch& vb = c->vbin;
+  void* vs[] = {vb.rec, vb.pidx, vb.tile_count, vb.tile_start, vb.tile_cap, vb.flags, vb.scan_tmp};
+  for (void* p : vs) rel(p);
   // pl[1] and al[1] alias the scratch freed above
   void* qs[] = {c->pl[0].s0, c->pl[0].s1, c->pl_count[0], c->pl_start[0], c->pl_count[1],
                 c->pl_start[1], c->al[0].p.s0, c->al[0].p.s1, c->al[0].c0, c->al[0].c1,
@@ -395,6 +403,7 @@ extern "C" int pmx_ctx_trim(pmx_ctx* c, int what) {
     return PMX_OK;
   }
   free_adj_state(c);
+  pmx_free_vbin(c);
   dev_free(c, (void**)&c->lbuf, (size_t)c->Mc * sizeof(float2));
   dev_free(c, (void**)&c->rec, c->rec_cap * 16);
   dev_free(c, (void**)&c->pidx, c->rec_cap * 4);
@@ -452,6 +461,43 @@ int pmx_ensure_ptcl(pmx_ctx* c, long long n) {
   c->ptcl_cap = cap;
   c->rec_cap = rcap;
   return PMX_OK;
+}
+
+void pmx_free_vbin(pmx_ctx* c) {
+  BinScratch& b = c->vbin;
+  const size_t tb = (size_t)(c->ntiles + 1) * 4;
+  dev_release(c, (void**)&b.rec, b.rec_cap * 16);
+  dev_release(c, (void**)&b.pidx, b.rec_cap * 4);
+  dev_release(c, (void**)&b.tile_count, tb);
+  dev_release(c, (void**)&b.tile_start, tb);
+  dev_release(c, (void**)&b.tile_cap, tb);
+  dev_release(c, (void**)&b.flags, 4 * sizeof(uint32_t));
+  dev_release(c, (void**)&b.scan_tmp, b.scan_tmp_cap * 4);
+  b = BinScratch{};
+}
+
+int pmx_ensure_vbin(pmx_ctx* c, long long n) {
+  BinScratch& b = c->vbin;
+  if (n <= b.ptcl_cap) return PMX_OK;
+  if (int rc = pmx_no_capture(c, "value scatter scratch")) return rc;
+  pmx_free_vbin(c);
+  const size_t tb = (size_t)(c->ntiles + 1) * 4;
+  b.ptcl_cap = n + n / 16 + 1024;
+  b.rec_cap = pmx_record_cap(c, b.ptcl_cap);
+  b.scan_tmp_cap = pmx_scan_blocks(c->ntiles + 1);
+  int rc = PMX_OK;
+  auto get = [&](void** p, size_t bytes) {
+    if (rc == PMX_OK) rc = dev_alloc(c, p, bytes);
+  };
+  get((void**)&b.rec, b.rec_cap * 16);
+  get((void**)&b.pidx, b.rec_cap * 4);
+  get((void**)&b.tile_count, tb);
+  get((void**)&b.tile_start, tb);
+  get((void**)&b.tile_cap, tb);
+  get((void**)&b.flags, 4 * sizeof(uint32_t));
+  get((void**)&b.scan_tmp, b.scan_tmp_cap * 4);
+  if (rc) pmx_free_vbin(c);
+  return rc;
 }
 
 int pmx_ensure_halo(pmx_ctx* c, int nch) {

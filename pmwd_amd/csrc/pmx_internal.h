@@ -126,6 +126,15 @@ void pmx_tic(pmx_ctx* c, int cls);
 void pmx_toc(pmx_ctx* c, int cls);
 
 // ------------------------------------------------------------- context --
+// What a binning pass (pmx_bin_particles) writes; the fields of pmx_ctx with
+// these names are described there.
+struct BinScratch {
+  long long ptcl_cap, rec_cap, caps_n, scan_tmp_cap;
+  int caps_valid;
+  float4* rec;
+  uint32_t *pidx, *tile_count, *tile_start, *tile_cap, *flags, *scan_tmp;
+};
+
 struct pmx_ctx {
   PmxTimer* timer;     // NULL unless timing is enabled
   int n[3];
@@ -221,6 +230,8 @@ struct pmx_ctx {
   long long sort_hist_cap;
   uint32_t* scan_tmp;
   long long scan_tmp_cap;
+  // the value scatters' own binning scratch (pmx_values_scatter)
+  BinScratch vbin;
 
   size_t bytes;        // device bytes held
   int no_alloc;        // 1: scratch carved from static device memory; never allocate
@@ -271,6 +282,9 @@ long long pmx_scan_blocks(long long n);
 // hipMalloc), counted in pmx_ctx_bytes; the free takes the allocated size.
 int pmx_dev_alloc(pmx_ctx* c, void** p, size_t bytes);
 void pmx_dev_free(pmx_ctx* c, void** p, size_t bytes);
+// the value scatters' binning scratch for n particles; and its release
+int pmx_ensure_vbin(pmx_ctx* c, long long n);
+void pmx_free_vbin(pmx_ctx* c);
 int pmx_scan_exclusive(pmx_ctx* c, const uint32_t* in, uint32_t* out, long long n,
                        const uint32_t* cond = nullptr);
 // The capacity layout of the next binning: cap = count_in + slack per tile,

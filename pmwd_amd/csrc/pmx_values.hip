@@ -5,6 +5,8 @@
 // kernels of pmx_generic.hip, whose float operations these repeat.
 #include "pmx_internal.h"
 
+#include <utility>
+
 // Lower and upper cell indices per axis and the flat index of corner j.
 struct CicCorners {
   int row[4];  // flat index of (x, y) corner (jx + 2 jy) at z = 0
@@ -270,9 +272,10 @@ int pmx_values_adj(pmx_ctx* c, const int16_t* pmid, const float* disp, long long
   return PMX_OK;
 }
 
-// The binned scatter needs the context's particle scratch.  Where that would
-// have to grow under graph capture or under a graph the context keeps (which
-// growing drops), or has no room to, the caller scatters without it.
+// The binned scatter runs on scratch of its own (c->vbin), so that a graph
+// captured over any call of the context neither loses what it addresses when
+// that scratch grows nor meets it while it replays; under capture, and where
+// there is no room for the scratch, the caller scatters without it.
 // Nor is it taken for few particles (c->values_min, 131072): its binning is
 // five launches more than one of float atomics, which are over before them.
 // Scatter and gradient of 16^3 to 48^3 particles, three channels: 158-162 us
@@ -280,15 +283,36 @@ int pmx_values_adj(pmx_ctx* c, const int16_t* pmid, const float* disp, long long
 // 21.0 and 6.2 ms against 2.0 and 1.4.
 bool pmx_values_scatter_ready(pmx_ctx* c, long long n) {
   if (n < c->values_min || n >= (1LL << 32) - 2048) return false;
-  const bool grow = n > c->ptcl_cap || pmx_scan_blocks(c->ntiles + 1) > c->scan_tmp_cap;
-  if (grow && (c->gexec || c->graph || pmx_capturing(c))) return false;
-  return pmx_ensure_ptcl(c, n) == PMX_OK && pmx_ensure_scan(c, c->ntiles + 1) == PMX_OK;
+  return !pmx_capturing(c) && pmx_ensure_vbin(c, n) == PMX_OK;
 }
+
+// Puts c->vbin in the place of the context's binning scratch for one pass.
+struct UseVbin {
+  pmx_ctx* c;
+  explicit UseVbin(pmx_ctx* c_) : c(c_) { exchange(); }
+  ~UseVbin() { exchange(); }
+  void exchange() {
+    BinScratch& b = c->vbin;
+    std::swap(c->ptcl_cap, b.ptcl_cap);
+    std::swap(c->rec_cap, b.rec_cap);
+    std::swap(c->caps_n, b.caps_n);
+    std::swap(c->scan_tmp_cap, b.scan_tmp_cap);
+    std::swap(c->caps_valid, b.caps_valid);
+    std::swap(c->rec, b.rec);
+    std::swap(c->pidx, b.pidx);
+    std::swap(c->tile_count, b.tile_count);
+    std::swap(c->tile_start, b.tile_start);
+    std::swap(c->tile_cap, b.tile_cap);
+    std::swap(c->flags, b.flags);
+    std::swap(c->scan_tmp, b.scan_tmp);
+  }
+};
 
 int pmx_values_scatter(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
                        const float* val, float vs, int nchan, float* mesh) {
   const MeshGeom g = plain_geom(c);
   const TileGeom& tg = c->tg;
+  const UseVbin use(c);
   int rc;
   if ((rc = pmx_bin_particles(c, pmid, disp, n))) return rc;
   const size_t lds =
