@@ -138,7 +138,8 @@ __global__ void __launch_bounds__(PMX_TPB)
 // binned records (values read at the particle's index) to float64 sums in LDS
 // over the tile and its +1 shell, then to the interleaved mesh: cells that no
 // other tile reaches by a plain read and write, the low faces and the shell
-// (which the tiles share) by float32 atomics, 1538 of a tile's 4913 cells.
+// (which the tiles share) by float32 atomics, 1538 of a tile's 4913 cells
+// (atomicAdd, as the any-geometry kernel: the mesh is the caller's memory).
 // Float64 sums rather than the density deposit's fixed-point ones: values may
 // be of any magnitude, infinite or NaN, and each contribution keeps its
 // float32 rounding.  LDS takes float64 adds about as fast as 64-bit integer
@@ -216,7 +217,7 @@ __global__ void __launch_bounds__(ValTpb<NC>::v)
     const bool shared = qx == 0 || qy == 0 || qz == 0 || qx == s[0] || qy == s[1] || qz == s[2];
     if (a != 0.0) {
       if (shared)
-        unsafeAtomicAdd(m, (float)a);
+        atomicAdd(m, (float)a);
       else
         *m = *m + (float)a;
     }
