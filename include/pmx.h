@@ -128,7 +128,8 @@ int pmx_lpt_grid(pmx_ctx* ctx, const float* modes, float cell_vol, int order,
                  const float* fac, const float* dtab, float* disp, float* vel);
 /* Adjoint of pmx_lpt with respect to the modes: modes_cot (n0,n1,n2/2+1)
  * complex64 is written, the conjugate gradient of a real loss (interior
- * columns of the last axis count twice).                                    */
+ * columns of the last axis count twice).  Order 1 does not read modes, which
+ * may then be NULL.                                                         */
 int pmx_lpt_vjp(pmx_ctx* ctx, const float* modes, float cell_vol, int order,
                 const float* fac, const float* disp_cot, const float* vel_cot,
                 float* modes_cot);

@@ -598,7 +598,8 @@ extern "C" int pmx_lpt_vjp(pmx_ctx* c, const float* modes, float cell_vol, int o
                            float* modes_cot) {
   PMX_ENTRY(c);
   PMX_REQUIRE(c && order >= 1 && order <= 2, "pmx_lpt_vjp: bad argument (order %d)", order);
-  PMX_REQUIRE(modes && fac && disp_cot && vel_cot && modes_cot, "pmx_lpt_vjp: NULL pointer");
+  PMX_REQUIRE((modes || order == 1) && fac && disp_cot && vel_cot && modes_cot,
+              "pmx_lpt_vjp: NULL pointer");
   PMX_REQUIRE(cell_vol > 0.f, "pmx_lpt_vjp: cell volume must be positive");
   int rc;
   if (order > 1 && (rc = ensure_lbuf(c))) return rc;

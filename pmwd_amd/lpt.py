@@ -90,7 +90,10 @@ class _LptFn(torch.autograd.Function):
     def forward(ctx, modes, conf, fac, dtab):
         m = _plain(modes.detach())
         disp, vel, ctx.pmx = _lpt_call(m, conf, fac, dtab)
-        ctx.save_for_backward(m)
+        # the second order's strains come from the modes again; the caller may
+        # write to its own between the passes
+        if conf.lpt_order > 1:
+            ctx.save_for_backward(m.clone() if m.data_ptr() == modes.data_ptr() else m)
         ctx.conf, ctx.fac = conf, fac
         return disp, vel
 
@@ -98,10 +101,11 @@ class _LptFn(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, disp_cot, vel_cot):
         from . import _lib
-        (m,) = ctx.saved_tensors
         conf = ctx.conf
-        out = torch.empty_like(m)
+        m = ctx.saved_tensors[0] if conf.lpt_order > 1 else None
         gd, gv = _plain(disp_cot), _plain(vel_cot)
+        n0, n1, n2 = conf.ptcl_grid_shape
+        out = torch.empty((n0, n1, n2 // 2 + 1), dtype=torch.complex64, device=gd.device)
         # the forward's context: autograd may run this on another thread
         _lib.check(_lib.lib().pmx_lpt_vjp(
             ctx.pmx.bind(), _lib.ptr(m), float(conf.ptcl_cell_vol), int(conf.lpt_order),
