@@ -252,7 +252,7 @@ extern "C" int pmx_ctx_create(int n0, int n1, int n2, double cell_size, void* st
   const char* fol = getenv("PMX_FOLD_ON_LOAD");
   c->fold_on_load = !(fol && strcmp(fol, "0") == 0);
   const char* vmin = getenv("PMX_VALUES_MIN");
-  c->values_min = vmin ? atoll(vmin) : 131072;
+  c->values_min = vmin ? atoll(vmin) : -1;
   const char* dsp = getenv("PMX_DEPOSIT_SPLIT");
   c->deposit_split = !(dsp && strcmp(dsp, "0") == 0);
   c->ntiles = (long long)c->tg.ntx * c->tg.nty * c->tg.ntz;

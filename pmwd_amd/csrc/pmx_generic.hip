@@ -324,7 +324,7 @@ extern "C" int pmx_scatter_cic(pmx_ctx* c, const pmx_cic_geom* g, const int16_t*
   if (rc) return rc;
   if (n == 0) return PMX_OK;
   PMX_REQUIRE(pmid && disp, "pmx_scatter_cic: NULL particle arrays");
-  if (pmx_values_fit(c, g, nchan) && pmx_values_scatter_ready(c, n))
+  if (pmx_values_fit(c, g, nchan) && pmx_values_scatter_ready(c, n, nchan))
     return pmx_values_scatter(c, pmid, disp, n, val, val_scalar, nchan, mesh);
   gen_scatter_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(G, pmid, disp, n, val, val_scalar, nchan,
                                                           mesh);
@@ -380,13 +380,17 @@ extern "C" int pmx_gather_cic_adj(pmx_ctx* c, const pmx_cic_geom* g, const int16
   if (rc) return rc;
   if (n == 0) return PMX_OK;
   PMX_REQUIRE(pmid && disp && mesh && val_cot, "pmx_gather_cic_adj: NULL pointer");
-  // few particles with a mesh cotangent: both in the one launch below
-  if (pmx_values_fit(c, g, nchan) && (!mesh_cot || n >= c->values_min)) {
+  // few particles with a mesh cotangent: both in the one launch below.  Its
+  // time is the host's up to twice the scatter's rule for one and two channels
+  // (131072 in cell order on 64^3: 168 us for the readout and its gradients,
+  // 183 in the tiles' seven launches; three channels 192 and 183).
+  const long long split = c->values_min >= 0 ? c->values_min : (nchan > 2 ? 1 : 2) * PMX_VALUES_MIN;
+  if (pmx_values_fit(c, g, nchan) && (!mesh_cot || n >= split)) {
     if (disp_cot && (rc = pmx_values_adj(c, pmid, disp, n, mesh, nchan, val_cot, 0.f, disp_cot, nullptr)))
       return rc;
     disp_cot = nullptr;
     if (!mesh_cot) return PMX_OK;
-    if (pmx_values_scatter_ready(c, n))
+    if (pmx_values_scatter_ready(c, n, nchan))
       return pmx_values_scatter(c, pmid, disp, n, val_cot, 0.f, nchan, mesh_cot);
   }
   gen_gather_adj_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(G, pmid, disp, n, mesh, val_cot, nchan,

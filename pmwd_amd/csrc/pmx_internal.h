@@ -203,7 +203,8 @@ struct pmx_ctx {
   int fold_on_load;    // the Poisson row pass may take the deposit's fold
                        // (environment PMX_FOLD_ON_LOAD=0 at creation: never)
   long long values_min;  // particles from which values are scattered in tiles
-                         // (environment PMX_VALUES_MIN at creation)
+                         // (environment PMX_VALUES_MIN at creation; -1: the
+                         // rule of pmx_values.hip)
   int deposit_split;   // several-channel deposits: a workgroup per tile and
                        // channel (environment PMX_DEPOSIT_SPLIT=0 at
                        // creation: the channels in turn in one workgroup)
@@ -1078,7 +1079,8 @@ int pmx_deposit_binned3(pmx_ctx* c, long long n, float* const* mesh, int mrs, in
 int pmx_ensure_halo(pmx_ctx* c, int nch);
 // default-geometry CIC of one to three value channels (pmx_values.hip)
 bool pmx_values_fit(const pmx_ctx* c, const pmx_cic_geom* g, int nchan);
-bool pmx_values_scatter_ready(pmx_ctx* c, long long n);
+#define PMX_VALUES_MIN 131072
+bool pmx_values_scatter_ready(pmx_ctx* c, long long n, int nchan);
 int pmx_values_gather(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
                       const float* mesh, int nchan, const float* val, float vs, float* out);
 int pmx_values_adj(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n, const float* f,

@@ -166,8 +166,9 @@ __global__ void __launch_bounds__(ValTpb<NC>::v)
   tile_origin(t, tg, g, o, s, ti);
   const int LY = s[1] + 1, LZ = s[2] + 1, sxy = LY * LZ;
   const int ltot = (s[0] + 1) * sxy;
-  for (int i = threadIdx.x; i < NC * ltot; i += TPB) acc[i] = 0.0;
   const uint32_t start = tile_start[t], cnt = tile_count[t];
+  if (cnt == 0u) return;
+  for (int i = threadIdx.x; i < NC * ltot; i += TPB) acc[i] = 0.0;
   __syncthreads();
   // the next round's record and values are loaded before this round's sums
   float4 rn;
@@ -273,17 +274,34 @@ int pmx_values_adj(pmx_ctx* c, const int16_t* pmid, const float* disp, long long
   return PMX_OK;
 }
 
+// Whether n particles' values go by tiles.  Binning is five launches more than
+// one of float atomics and costs what it costs however few the channels; then
+// one workgroup takes a tile, whether it holds few particles or many.  So the
+// atomics win for few particles, for few tiles (idle CUs) and for sparse ones
+// (a sum cleared and flushed for little).  Timed over meshes of 16^3 to 512^3
+// and 32768 to 16 M particles in random and in cell order, 1 and 3 channels,
+// atomics against tiles, us:
+//   131072 on 64^3 (64 tiles)  46-68 / 45-49 (1), 135-172 / 57-64 (3);
+//   131072 on 48^3 (27 tiles)  40-68 / 48 (1), 122-170 / 67-69 (3);
+//   131072 on 32^3 (8 tiles)   45-78 / 61-81 (1), 110-170 / 110-170 (3);
+//   1e6 on 16^3 (1 tile)  696-1557 / 1414-3660 (1), 1504-2251 / 3968-10795 (3);
+//   131072 on 192^3 (76 a tile)  66-68 / 69-82 (1), 175-177 / 131-140 (3);
+//   300000 on 256^3 (73 a tile)  132-141 / 116-132 (1), 387-392 / 253-268 (3);
+//   1e6 on 512^3 (31 a tile)  487-517 / 639-695 (1), 1410-1438 / 1674-1735 (3);
+//   16 M on 256^3  2988-6134 / 708-1326 (1), 13596-18552 / 1271-1714 (3).
+// PMX_VALUES_MIN (c->values_min >= 0) puts a particle count in the rule's place.
+static bool values_tiled(const pmx_ctx* c, long long n, int nchan) {
+  if (c->values_min >= 0) return n >= c->values_min;
+  const long long tiles = nchan > 1 ? 27 : 64, per = nchan > 1 ? 64 : 96;
+  return n >= PMX_VALUES_MIN && c->ntiles >= tiles && n >= per * c->ntiles;
+}
+
 // The binned scatter runs on scratch of its own (c->vbin), so that a graph
 // captured over any call of the context neither loses what it addresses when
 // that scratch grows nor meets it while it replays; under capture, and where
 // there is no room for the scratch, the caller scatters without it.
-// Nor is it taken for few particles (c->values_min, 131072): its binning is
-// five launches more than one of float atomics, which are over before them.
-// Scatter and gradient of 16^3 to 48^3 particles, three channels: 158-162 us
-// with atomics, 166 binned; readout and gradients 145-148 against 160; of 256^3
-// 21.0 and 6.2 ms against 2.0 and 1.4.
-bool pmx_values_scatter_ready(pmx_ctx* c, long long n) {
-  if (n < c->values_min || n >= (1LL << 32) - 2048) return false;
+bool pmx_values_scatter_ready(pmx_ctx* c, long long n, int nchan) {
+  if (!values_tiled(c, n, nchan) || n >= (1LL << 32) - 2048) return false;
   return !pmx_capturing(c) && pmx_ensure_vbin(c, n) == PMX_OK;
 }
 
