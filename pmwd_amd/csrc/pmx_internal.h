@@ -1069,7 +1069,7 @@ int pmx_ensure_adj_state(pmx_ctx* c, int nsteps);
 // reverse kick(s) and drift of the caller's arrays (pending closing kick kp
 // first when nonzero), binned into count/o; per-block partials of the drift
 // dot product at part[0, pmx_kd_adj_blocks(n))
-#define KD_ADJ_TPB 512
+#define KD_ADJ_TPB 256
 inline unsigned pmx_kd_adj_blocks(long long n) { return pmx_blocks(n, KD_ADJ_TPB); }
 int pmx_kd_adj_bin(pmx_ctx* c, const int16_t* pmid, float* disp, float* vel, const float* acc,
                    float* disp_cot, float* vel_cot, const float* acc_cot, const float* disp_snap,
