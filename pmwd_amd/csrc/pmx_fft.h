@@ -845,10 +845,12 @@ __device__ __forceinline__ ColMap col_map(int lB) {
 // FFT of a block of columns held in registers in the order of cm, through
 // the LDS block s, which no thread may still be reading on entry (and some
 // may on return).  The staging of the twiddles need not be waited for.
-template <int DIR, bool POW2, int LN, int LP, int MAXV, int TPB>
+// REGS false: the first and last stage go through LDS as well (fewer
+// registers at once).
+template <int DIR, bool POW2, int LN, int LP, int MAXV, int TPB, bool REGS = true>
 __device__ __forceinline__ void fft_cols(float2 (&r)[MAXV], float2* s, int n, int P,
                                          const float2* __restrict__ tw, const ColMap& cm) {
-  if constexpr (LN > 0) {
+  if constexpr (LN > 0 && REGS) {
     ct_fft_reg<DIR, ct_n(LN), 1 << LP, 1, TPB>(r, s, tw);
   } else {
 #pragma unroll

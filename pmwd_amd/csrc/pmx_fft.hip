@@ -675,13 +675,22 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(1,
     if (live && cm.j0 + it * cm.js < n) g2[it * gs] = h[it];
 }
 
+//
+// Workgroups of 512 threads keep to 128 registers, so that two share a CU; of
+// the 512-long axis the transforms then go through LDS at both ends, which
+// fits without spilling (the cap alone spills 14).  The axis' forward passes
+// in a force and its gradient, from registers without the cap, with it, and
+// now: 512^3 1090, 1080, 1054 us; 128 x 1024 x 128 195, 186, 186; 128 x 768 x
+// 128 155, 146, 146.
+constexpr int yfwd_tpb(int ln) { return ln ? ct_tpb(ln, ct_cols(ln, FFT_CAP), fft_v(-1, ln)) : GEN_MAXTPB; }
 template <bool POW2, int LN>
-__global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(-1, LN)) : GEN_MAXTPB, LN ? 2 : 4) y_fwd_seq_k(Fields3 fl, int n_, long long es,
+__global__ void __launch_bounds__(yfwd_tpb(LN), yfwd_tpb(LN) == 512 ? 4 : 2) y_fwd_seq_k(Fields3 fl, int n_, long long es,
                                                         long long ostride, int ncol, int B_,
                                                         KTab kt, const float2* __restrict__ tw) {
   extern __shared__ float2 s[];
   constexpr int BC = LN ? ct_cols(LN, FFT_CAP) : 1;
   constexpr int TPB = LN ? ct_tpb(LN, BC, fft_v(-1, LN)) : GEN_TPB;
+  constexpr bool REGS = LN != 9;
   constexpr int MAXV = LN ? BC * ct_n(LN) / TPB : GEN_MAXV;
   const int n = LN ? ct_n(LN) : n_;
   const int B = LN ? BC : B_;
@@ -711,9 +720,9 @@ __global__ void __launch_bounds__(LN ? ct_tpb(LN, ct_cols(LN, FFT_CAP), fft_v(-1
     c[it] = make_float2(0.f, 0.f);
     if (live && cm.j0 + it * cm.js < n) c[it] = g2[it * gs];
   }
-  fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB>(a, s, n, B, stw, cm);
+  fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB, REGS>(a, s, n, B, stw, cm);
   __syncthreads();
-  fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB>(c, s, n, B, stw, cm);
+  fft_cols<-1, POW2, LN, ilog2c(BC), MAXV, TPB, REGS>(c, s, n, B, stw, cm);
 #pragma unroll
   for (int it = 0; it < MAXV; ++it) {
     const int j = cm.j0 + it * cm.js;
