@@ -216,6 +216,7 @@ extern "C" int pmx_ctx_create(int n0, int n1, int n2, double cell_size, void* st
     pmx_set_error("pmx_ctx_create: out of host memory");
     return PMX_ENOMEM;
   }
+  pthread_mutex_init(&c->vbin_lock, nullptr);
   pmx_ctx_geometry(c, n0, n1, n2, cell_size, (hipStream_t)stream);
   c->dalloc = g_dalloc;
   c->dfree = g_dfree;
@@ -352,6 +353,7 @@ extern "C" int pmx_ctx_destroy(pmx_ctx* c) {
   for (void* p : qs) rel(p);
   if (c->red_host) hipHostFree(c->red_host);
   if (c->moved) hipEventDestroy(c->moved);
+  pthread_mutex_destroy(&c->vbin_lock);
   free(c);
   return PMX_OK;
 }
@@ -403,7 +405,10 @@ extern "C" int pmx_ctx_trim(pmx_ctx* c, int what) {
     return PMX_OK;
   }
   free_adj_state(c);
-  pmx_free_vbin(c);
+  {
+    const VbinTurn turn(c);
+    pmx_free_vbin(c);
+  }
   dev_free(c, (void**)&c->lbuf, (size_t)c->Mc * sizeof(float2));
   dev_free(c, (void**)&c->rec, c->rec_cap * 16);
   dev_free(c, (void**)&c->pidx, c->rec_cap * 4);

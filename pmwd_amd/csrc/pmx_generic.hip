@@ -324,8 +324,9 @@ extern "C" int pmx_scatter_cic(pmx_ctx* c, const pmx_cic_geom* g, const int16_t*
   if (rc) return rc;
   if (n == 0) return PMX_OK;
   PMX_REQUIRE(pmid && disp, "pmx_scatter_cic: NULL particle arrays");
-  if (pmx_values_fit(c, g, nchan) && pmx_values_scatter_ready(c, n, nchan))
-    return pmx_values_scatter(c, pmid, disp, n, val, val_scalar, nchan, mesh);
+  if (pmx_values_fit(c, g, nchan) &&
+      pmx_values_scatter(c, pmid, disp, n, val, val_scalar, nchan, mesh, &rc))
+    return rc;
   gen_scatter_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(G, pmid, disp, n, val, val_scalar, nchan,
                                                           mesh);
   PMX_LAUNCH_CHECK();
@@ -390,8 +391,7 @@ extern "C" int pmx_gather_cic_adj(pmx_ctx* c, const pmx_cic_geom* g, const int16
       return rc;
     disp_cot = nullptr;
     if (!mesh_cot) return PMX_OK;
-    if (pmx_values_scatter_ready(c, n, nchan))
-      return pmx_values_scatter(c, pmid, disp, n, val_cot, 0.f, nchan, mesh_cot);
+    if (pmx_values_scatter(c, pmid, disp, n, val_cot, 0.f, nchan, mesh_cot, &rc)) return rc;
   }
   gen_gather_adj_k<<<pmx_blocks(n), PMX_TPB, 0, c->stream>>>(G, pmid, disp, n, mesh, val_cot, nchan,
                                                              disp_cot, mesh_cot);

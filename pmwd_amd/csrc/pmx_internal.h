@@ -1,6 +1,7 @@
 // Internal definitions shared by the pmx HIP translation units (gfx950 only).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <pthread.h>
 #include <stdint.h>
 #include <stddef.h>
 #include <string>
@@ -231,8 +232,9 @@ struct pmx_ctx {
   long long sort_hist_cap;
   uint32_t* scan_tmp;
   long long scan_tmp_cap;
-  // the value scatters' own binning scratch (pmx_values_scatter)
+  // the value scatters' own binning scratch (pmx_values_scatter), and who uses it
   BinScratch vbin;
+  pthread_mutex_t vbin_lock;
 
   size_t bytes;        // device bytes held
   int no_alloc;        // 1: scratch carved from static device memory; never allocate
@@ -283,9 +285,15 @@ long long pmx_scan_blocks(long long n);
 // hipMalloc), counted in pmx_ctx_bytes; the free takes the allocated size.
 int pmx_dev_alloc(pmx_ctx* c, void** p, size_t bytes);
 void pmx_dev_free(pmx_ctx* c, void** p, size_t bytes);
-// the value scatters' binning scratch for n particles; and its release
+// the value scatters' binning scratch for n particles, its release, and the
+// turn to do either or to use it
 int pmx_ensure_vbin(pmx_ctx* c, long long n);
 void pmx_free_vbin(pmx_ctx* c);
+struct VbinTurn {
+  pmx_ctx* c;
+  explicit VbinTurn(pmx_ctx* c_) : c(c_) { pthread_mutex_lock(&c->vbin_lock); }
+  ~VbinTurn() { pthread_mutex_unlock(&c->vbin_lock); }
+};
 int pmx_scan_exclusive(pmx_ctx* c, const uint32_t* in, uint32_t* out, long long n,
                        const uint32_t* cond = nullptr);
 // The capacity layout of the next binning: cap = count_in + slack per tile,
@@ -1080,13 +1088,12 @@ int pmx_ensure_halo(pmx_ctx* c, int nch);
 // default-geometry CIC of one to three value channels (pmx_values.hip)
 bool pmx_values_fit(const pmx_ctx* c, const pmx_cic_geom* g, int nchan);
 #define PMX_VALUES_MIN 131072
-bool pmx_values_scatter_ready(pmx_ctx* c, long long n, int nchan);
 int pmx_values_gather(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
                       const float* mesh, int nchan, const float* val, float vs, float* out);
 int pmx_values_adj(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n, const float* f,
                    int nchan, const float* val, float vs, float* disp_cot, float* val_cot);
-int pmx_values_scatter(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
-                       const float* val, float vs, int nchan, float* mesh);
+bool pmx_values_scatter(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
+                        const float* val, float vs, int nchan, float* mesh, int* rc);
 int pmx_poisson_ctx(pmx_ctx* c, float coef, int deferred = 0);
 // FFT passes on meshes in the context's padded layout (pmx_fft.hip):
 // in-place z r2c (pre: (x - 1) * coef on load; halo: the deposit's fold

@@ -5,8 +5,6 @@
 // kernels of pmx_generic.hip, whose float operations these repeat.
 #include "pmx_internal.h"
 
-#include <utility>
-
 // Lower and upper cell indices per axis and the flat index of corner j.
 struct CicCorners {
   int row[4];  // flat index of (x, y) corner (jx + 2 jy) at z = 0
@@ -274,6 +272,22 @@ int pmx_values_adj(pmx_ctx* c, const int16_t* pmid, const float* disp, long long
   return PMX_OK;
 }
 
+static int deposit_vals(pmx_ctx* c, const float* val, float vs, int nchan, float* mesh) {
+  const MeshGeom g = plain_geom(c);
+  const TileGeom& tg = c->tg;
+  const size_t lds =
+      (size_t)(tg.tx + 1) * (tg.ty + 1) * (tg.tz + 1) * sizeof(double) * (size_t)nchan;
+#define CALL(NC)                                                                               \
+  deposit_vals_k<NC><<<(unsigned)c->ntiles, ValTpb<NC>::v, lds, c->stream>>>(                  \
+      c->rec, c->pidx, c->tile_start, c->tile_count, g, tg, val, vs, mesh)
+  pmx_tic(c, PMX_T_DEPOSIT);
+  VAL_SWITCH(nchan, CALL);
+  pmx_toc(c, PMX_T_DEPOSIT);
+#undef CALL
+  PMX_LAUNCH_CHECK();
+  return PMX_OK;
+}
+
 // Whether n particles' values go by tiles.  Binning is five launches more than
 // one of float atomics and costs what it costs however few the channels; then
 // one workgroup takes a tile, whether it holds few particles or many.  So the
@@ -296,53 +310,39 @@ static bool values_tiled(const pmx_ctx* c, long long n, int nchan) {
   return n >= PMX_VALUES_MIN && c->ntiles >= tiles && n >= per * c->ntiles;
 }
 
-// The binned scatter runs on scratch of its own (c->vbin), so that a graph
-// captured over any call of the context neither loses what it addresses when
-// that scratch grows nor meets it while it replays; under capture, and where
-// there is no room for the scratch, the caller scatters without it.
-bool pmx_values_scatter_ready(pmx_ctx* c, long long n, int nchan) {
-  if (!values_tiled(c, n, nchan) || n >= (1LL << 32) - 2048) return false;
-  return !pmx_capturing(c) && pmx_ensure_vbin(c, n) == PMX_OK;
+// The context with c->vbin for its binning scratch (c itself is left alone).
+static pmx_ctx with_vbin(const pmx_ctx* c) {
+  const BinScratch& b = c->vbin;
+  pmx_ctx v = *c;
+  v.ptcl_cap = b.ptcl_cap;
+  v.rec_cap = b.rec_cap;
+  v.caps_n = b.caps_n;
+  v.scan_tmp_cap = b.scan_tmp_cap;
+  v.caps_valid = b.caps_valid;
+  v.rec = b.rec;
+  v.pidx = b.pidx;
+  v.tile_count = b.tile_count;
+  v.tile_start = b.tile_start;
+  v.tile_cap = b.tile_cap;
+  v.flags = b.flags;
+  v.scan_tmp = b.scan_tmp;
+  return v;
 }
 
-// Puts c->vbin in the place of the context's binning scratch for one pass.
-struct UseVbin {
-  pmx_ctx* c;
-  explicit UseVbin(pmx_ctx* c_) : c(c_) { exchange(); }
-  ~UseVbin() { exchange(); }
-  void exchange() {
-    BinScratch& b = c->vbin;
-    std::swap(c->ptcl_cap, b.ptcl_cap);
-    std::swap(c->rec_cap, b.rec_cap);
-    std::swap(c->caps_n, b.caps_n);
-    std::swap(c->scan_tmp_cap, b.scan_tmp_cap);
-    std::swap(c->caps_valid, b.caps_valid);
-    std::swap(c->rec, b.rec);
-    std::swap(c->pidx, b.pidx);
-    std::swap(c->tile_count, b.tile_count);
-    std::swap(c->tile_start, b.tile_start);
-    std::swap(c->tile_cap, b.tile_cap);
-    std::swap(c->flags, b.flags);
-    std::swap(c->scan_tmp, b.scan_tmp);
-  }
-};
-
-int pmx_values_scatter(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
-                       const float* val, float vs, int nchan, float* mesh) {
-  const MeshGeom g = plain_geom(c);
-  const TileGeom& tg = c->tg;
-  const UseVbin use(c);
-  int rc;
-  if ((rc = pmx_bin_particles(c, pmid, disp, n))) return rc;
-  const size_t lds =
-      (size_t)(tg.tx + 1) * (tg.ty + 1) * (tg.tz + 1) * sizeof(double) * (size_t)nchan;
-#define CALL(NC)                                                                               \
-  deposit_vals_k<NC><<<(unsigned)c->ntiles, ValTpb<NC>::v, lds, c->stream>>>(                  \
-      c->rec, c->pidx, c->tile_start, c->tile_count, g, tg, val, vs, mesh)
-  pmx_tic(c, PMX_T_DEPOSIT);
-  VAL_SWITCH(nchan, CALL);
-  pmx_toc(c, PMX_T_DEPOSIT);
-#undef CALL
-  PMX_LAUNCH_CHECK();
-  return PMX_OK;
+// The binned scatter; false where the caller scatters without it.  It runs on
+// scratch of its own (c->vbin), so that a graph captured over any call of the
+// context neither loses what it addresses when that scratch grows nor meets
+// it while it replays; under capture, and where there is no room for the
+// scratch, it is not taken.  Threads that queue on one stream take turns.
+bool pmx_values_scatter(pmx_ctx* c, const int16_t* pmid, const float* disp, long long n,
+                        const float* val, float vs, int nchan, float* mesh, int* rc) {
+  if (!values_tiled(c, n, nchan) || n >= (1LL << 32) - 2048 || pmx_capturing(c)) return false;
+  const VbinTurn turn(c);
+  if (pmx_ensure_vbin(c, n) != PMX_OK) return false;
+  pmx_ctx v = with_vbin(c);
+  *rc = pmx_bin_particles(&v, pmid, disp, n);
+  c->vbin.caps_valid = v.caps_valid;
+  c->vbin.caps_n = v.caps_n;
+  if (*rc == PMX_OK) *rc = deposit_vals(&v, val, vs, nchan, mesh);
+  return true;
 }

@@ -103,3 +103,37 @@ def test_trim_gives_the_value_scratch_back(dev):
     for x in (b, c):
         np.testing.assert_allclose(x.cpu().numpy(), a.cpu().numpy(), rtol=1e-5, atol=1e-5)
     ctx.close()
+
+
+def test_threads_on_one_context(dev):
+    """Threads that scatter values on one context and stream at once, beside
+    one that takes densities there, each get their own numbers."""
+    import threading
+    import pmwd_amd as pa
+    from pmwd_amd import _lib
+    cases = [_state(dev, (20, 12, 35), k, 10 + k) for k in (1, 2, 3)]
+    conf = cases[0][0]
+    _lib.context(conf.mesh_shape, conf.cell_size, dev)   # the one that all share
+    works = [lambda p=p, v=v: pa.scatter(p, conf, val=v) for _, p, v in cases]
+    works.append(lambda: pa.scatter(cases[0][1], conf))
+    want = [w().clone() for w in works]
+    wrong = []
+
+    def loop(work, ref):
+        try:
+            torch.cuda.set_device(dev)
+            for _ in range(40):
+                got = work()
+                torch.cuda.synchronize()
+                if not torch.allclose(got, ref, rtol=1e-5, atol=1e-5):
+                    wrong.append(float((got - ref).abs().max()))
+        except Exception as e:   # reported by the assertion below
+            wrong.append(repr(e))
+
+    threads = [threading.Thread(target=loop, args=a) for a in zip(works, want)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[:5]
+    assert len(_lib._ctx_cache) == 1
