@@ -1,9 +1,9 @@
 // Cloud-in-cell scatter/gather, gravity and time stepping (gfx950).
 //
 // Hot scatter (pmx_scatter_mass): particles are binned by the mesh tile that
-// holds their lower CIC corner (wave-aggregated integer atomics over a
-// capacity layout, or count, scan and emit), then one workgroup per tile accumulates its
-// particles into an LDS copy of the tile plus a +1 halo shell and writes the
+// holds their lower CIC corner (counted per workgroup in LDS, one global
+// atomic a tile; over a capacity layout, or count, scan and emit), then one
+// workgroup per tile accumulates its particles into an LDS copy of the tile plus a +1 halo shell and writes the
 // tile interior with plain stores and the shell to a halo buffer; a fold
 // pass adds each tile's incoming shells.  No float atomics touch global
 // memory on this path.  The tile-staged gather and the forward KDK step
@@ -96,7 +96,7 @@ extern "C" int pmx_tile_keys(pmx_ctx* c, const int16_t* pmid, const float* disp,
 // (TileTable) and takes one per tile: consecutive particles share few tiles,
 // 8192 of them about 200 against eight per wave of 64.  Its records for a
 // tile are then one run of the tile, long enough to fill cache lines.  512^3
-// particles: count 0.55 ms, emit 1.5 ms; with atomics per wave 1.0 ms for the
+// particles: count 0.54 ms, emit 1.27 ms; with atomics per wave 1.0 ms for the
 // counts and ranks and 2.2 ms for a separate fill.
 enum { BIN_COUNT = 0, BIN_FIRST = 1, BIN_EMIT = 2, BIN_BOTH = 3 };
 
@@ -195,9 +195,8 @@ __device__ __forceinline__ int shell_index(int qx, int qy, int qz, int sx, int s
 
 // Fixed-point scale for tile accumulation: 2^k with |v| * 2^k < 2^30, so a
 // sum of up to 2^33 contributions fits a signed 64-bit integer; resolution
-// is 2^-30 of the largest |v|.  LDS float atomics serialise on gfx950 while
-// 64-bit integer LDS atomics run at full rate, and integer sums make the
-// accumulation order-independent (bitwise deterministic).
+// is 2^-30 of the largest |v|.  Integer sums make the accumulation
+// order-independent (bitwise deterministic).
 __device__ __forceinline__ double fixed_scale(float vmax) {
   int e = 0;
   if (vmax > 0.f) frexpf(vmax, &e);  // vmax < 2^e

@@ -450,7 +450,7 @@ int pmx_ensure_ptcl(pmx_ctx* c, long long n) {
   free_adj_state(c);
   c->ptcl_cap = c->rec_cap = c->vrec_cap = c->pl_cap = 0;
   c->caps_valid = 0;
-  // pkey/prank hold a tile and rank per particle
+  // pkey/prank hold a tile and rank per particle, for the pipelines' first fill
   int rc = dev_alloc(c, (void**)&c->rec, rcap * 16);
   rc |= dev_alloc(c, (void**)&c->pidx, rcap * 4);
   rc |= dev_alloc(c, (void**)&c->pkey, rcap * 4);

@@ -412,13 +412,6 @@ __device__ __forceinline__ void pmx_wgrad(const CicAxis* ax, int j, float g[3]) 
   g[2] = s2 * (f0 * f1);
 }
 
-__device__ __forceinline__ long long pmx_cell_index(const CicAxis* ax, int j, int n1, int rs) {
-  int i0 = (j & 1) ? ax[0].hi : ax[0].lo;
-  int i1 = (j & 2) ? ax[1].hi : ax[1].lo;
-  int i2 = (j & 4) ? ax[2].hi : ax[2].lo;
-  return ((long long)i0 * n1 + i1) * rs + i2;
-}
-
 // fixed tree order used for every 8-neighbour sum
 __device__ __forceinline__ float pmx_tree8(const float v[8]) {
   return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));

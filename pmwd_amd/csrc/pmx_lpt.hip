@@ -15,7 +15,7 @@
 // so a strain costs under five mesh reads or writes instead of ten and no particle
 // array is read back.  The passes are bound by memory (3.5 to 8 TB/s, the
 // larger where a mesh stays in cache).  White noise to 2LPT at 256^3: 2403 ->
-// 1236 us; with its gradient at 128^3 (before: tensor ops) 5000 -> 690 us.
+// 1190 us; with its gradient at 128^3 (before: tensor ops) 5000 -> 636 us.
 // Odd n2 (rows in pairs, no half-length transform) keeps separate z passes.
 #include "pmx_fft.h"
 

@@ -1,9 +1,9 @@
 // A default-argument CIC mass assignment that allocates nothing: the same
 // binning and LDS-tile deposit kernels as pmx_scatter_mass, with their
-// scratch (tile counts, starts and capacities, the overflow flag, the scan
-// partials, the +1 halo shells, and per record slot the record, index, tile
-// and rank words) carved from one file-scope device array instead of a
-// context's allocations.  For callers that cannot allocate device memory
+// scratch (tile counts, starts and capacities, the overflow flags, the scan
+// partials, the +1 halo shells, and per record slot the record, index and two
+// words that keep the limit below where callers know it) carved from one
+// file-scope device array instead of a context's allocations.  For callers that cannot allocate device memory
 // (code under graph capture, tight serving loops, hosts that forbid it).
 //
 // Each device holds its own copy of the array until the process ends; its
@@ -84,8 +84,7 @@ extern "C" int pmx_scatter_mass_noalloc(const int16_t* pmid, const float* disp, 
   sz.take<float>((size_t)nt * c.tg.shell);         // one channel of halo shells
   sz.take<float4>(rcap);                           // records
   sz.take<uint32_t>(rcap);                         // pidx
-  sz.take<uint32_t>(rcap);                         // pkey
-  sz.take<uint32_t>(rcap);                         // prank
+  sz.take<uint32_t>(2 * rcap);                     // not read (the limit)
   PMX_REQUIRE(sz.used <= PMX_NOALLOC_BYTES,
               "pmx_scatter_mass_noalloc: %lld particles on a %dx%dx%d mesh need %zu bytes of "
               "scratch, more than the %llu it holds (use pmx_scatter_mass)", n, n0, n1, n2,
@@ -103,8 +102,6 @@ extern "C" int pmx_scatter_mass_noalloc(const int16_t* pmid, const float* disp, 
   c.halo_nch = 1;
   c.rec = cv.take<float4>(rcap);
   c.pidx = cv.take<uint32_t>(rcap);
-  c.pkey = cv.take<uint32_t>(rcap);
-  c.prank = cv.take<uint32_t>(rcap);
   c.ptcl_cap = cap;
   c.rec_cap = rcap;
   c.caps_valid = 0;   // exact count, scan and fill: nothing read from the last call
